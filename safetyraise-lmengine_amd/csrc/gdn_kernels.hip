@@ -530,8 +530,8 @@ __global__ void __launch_bounds__(NTH) gdn_head_kernel(const GdnParams p, const 
 // element by element with the same operations gdn_head_kernel applies (a
 // product, then a multiply-add), so the rebuilt state is the one the forward
 // held after that row; the history is the last K-1 of (the history before
-// the call, x_0 .. x_{keep-1}).  Blocks 0..Hv-1 rebuild one value head's
-// state each, the others 256 conv channels each.
+// the call, x_0 .. x_{keep-1}).  The first Hv * kRbBlocks blocks rebuild
+// kRbRows state rows of one value head each, the others 256 conv channels each.
 // ---------------------------------------------------------------------------
 struct RollbackParams {
     const float *state_in;  // [Hv][Dv][Dk] before the call
@@ -542,56 +542,82 @@ struct RollbackParams {
     uint32_t rec_stride, keep, value_heads, channels, conv_k;
 };
 
+// What bounds it: at 32 heads 2 MB are read and 2 MB written, far below what a
+// launch costs, so the chain of loads.  A workgroup takes 16 state rows (8 per
+// value head: 256 workgroups at 32 heads, one per CU; one per head left 7/8 of
+// them idle), and requests the state and kRbBatch rows of records before it
+// uses any.  A lane holds dims [4 l16, +4) and [64 + 4 l16, +4), so the state
+// and the keys move as 16-byte accesses over 256 contiguous bytes: the keys
+// read as 8 dwords per lane cost 3.6 us of a 5.9 us launch.  kKeyVec: the
+// records' keys are 16-byte aligned (value_heads a multiple of 4; rec_stride
+// then is too).  K1T: the conv kernel's K - 1 where it is known (3), else 0.
+constexpr uint32_t kRbRows = 16;                   // state rows per workgroup
+constexpr uint32_t kRbBlocks = kHeadDv / kRbRows;  // workgroups per value head
+constexpr uint32_t kRbBatch = 4;                   // records in flight
+
+template <bool kKeyVec, uint32_t K1T>
 __global__ void __launch_bounds__(256) gdn_rollback_kernel(const RollbackParams p) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
     const uint32_t tid = threadIdx.x;
     const uint32_t hv_dv = p.value_heads * kHeadDv;
-    if (blockIdx.x < p.value_heads) {
-        const uint32_t h = blockIdx.x;
-        const uint32_t l16 = tid & 15, g = tid >> 4;  // rows g + 16 i, dims 8 l16 .. + 8
-        const float *src = p.state_in + (size_t)h * kHeadDv * kDk + 8 * l16;
-        float *dst = p.state_out + (size_t)h * kHeadDv * kDk + 8 * l16;
-        float S[8][8];
+    const uint32_t state_blocks = p.value_heads * kRbBlocks;
+    if (blockIdx.x < state_blocks) {
+        const uint32_t h = blockIdx.x / kRbBlocks;
+        const uint32_t v = (blockIdx.x % kRbBlocks) * kRbRows + (tid >> 4);
+        const uint32_t d0 = 4 * (tid & 15);
+        const size_t at = ((size_t)h * kHeadDv + v) * kDk + d0;
+        f4 S[2] = {*(const f4 *)(p.state_in + at), *(const f4 *)(p.state_in + at + kDk / 2)};
+        for (uint32_t r0 = 0; r0 < p.keep; r0 += kRbBatch) {
+            float alpha[kRbBatch], corr[kRbBatch];
+            f4 kh[kRbBatch][2];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float *s = src + (size_t)(g + 16 * i) * kDk;
-            const float4 x0 = *(const float4 *)s, x1 = *(const float4 *)(s + 4);
-            S[i][0] = x0.x; S[i][1] = x0.y; S[i][2] = x0.z; S[i][3] = x0.w;
-            S[i][4] = x1.x; S[i][5] = x1.y; S[i][6] = x1.z; S[i][7] = x1.w;
-        }
-        for (uint32_t r = 0; r < p.keep; ++r) {
-            const float *rec = p.records + (size_t)r * p.rec_stride;
-            const float alpha = rec[h];
-            float kh[8];
+            for (uint32_t u = 0; u < kRbBatch; ++u) {
+                // (rows past the last kept one read it again, unused)
+                const float *rec = p.records + (size_t)min(r0 + u, p.keep - 1) * p.rec_stride;
+                alpha[u] = rec[h];
+                corr[u] = rec[p.value_heads + h * kHeadDv + v];
+                const float *key = rec + p.value_heads + hv_dv + h * kDk + d0;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) kh[j] = rec[p.value_heads + hv_dv + h * kDk + 8 * l16 + j];
+                for (int i = 0; i < 2; ++i) {
+                    if constexpr (kKeyVec) {
+                        kh[u][i] = *(const f4 *)(key + i * (kDk / 2));
+                    } else {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float corr = rec[p.value_heads + h * kHeadDv + g + 16 * i];
+                        for (int j = 0; j < 4; ++j) kh[u][i][j] = key[i * (kDk / 2) + j];
+                    }
+                }
+            }
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    S[i][j] *= alpha;
-                    S[i][j] += corr * kh[j];
+            for (uint32_t u = 0; u < kRbBatch; ++u) {
+                if (r0 + u < p.keep) {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) S[i][j] = fmaf(corr[u], kh[u][i][j], S[i][j] * alpha[u]);
                 }
             }
         }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            float *d = dst + (size_t)(g + 16 * i) * kDk;
-            *(float4 *)d = make_float4(S[i][0], S[i][1], S[i][2], S[i][3]);
-            *(float4 *)(d + 4) = make_float4(S[i][4], S[i][5], S[i][6], S[i][7]);
-        }
+        *(f4 *)(p.state_out + at) = S[0];
+        *(f4 *)(p.state_out + at + kDk / 2) = S[1];
         return;
     }
-    const uint32_t c = (blockIdx.x - p.value_heads) * 256 + tid;
-    const uint32_t K1 = p.conv_k - 1;
+    const uint32_t c = (blockIdx.x - state_blocks) * 256 + tid;
+    const uint32_t K1 = K1T != 0 ? K1T : p.conv_k - 1;
     if (c >= p.channels || K1 == 0) return;
     // position t of (history before the call, x_0, x_1, ...): the last K-1
-    // positions up to row keep - 1 are t = keep .. keep + K1 - 1
-    for (uint32_t i = 0; i < K1; ++i) {
-        const uint32_t t = p.keep + i;
-        p.hist_out[(size_t)c * K1 + i] =
-            t < K1 ? p.hist_in[(size_t)c * K1 + t]
-                   : p.records[(size_t)(t - K1) * p.rec_stride + p.value_heads + 2 * hv_dv + c];
+    // positions up to row keep - 1 are t = keep .. keep + K1 - 1; all of them
+    // are requested before the first is stored
+    constexpr uint32_t kMost = K1T != 0 ? K1T : kMaxK - 1;
+    float x[kMost];
+#pragma unroll
+    for (uint32_t i = 0; i < kMost; ++i) {
+        const uint32_t t = p.keep + min(i, K1 - 1);
+        x[i] = *(t < K1 ? p.hist_in + (size_t)c * K1 + t
+                        : p.records + (size_t)(t - K1) * p.rec_stride + p.value_heads + 2 * hv_dv + c);
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kMost; ++i) {
+        if (i < K1) p.hist_out[(size_t)c * K1 + i] = x[i];
     }
 }
 
@@ -1852,13 +1878,24 @@ hipError_t launch_gdn_rollback(hipStream_t stream, const GdnRollback &r) {
     p.value_heads = r.value_heads;
     p.channels = r.channels;
     p.conv_k = r.conv_k;
-    const uint32_t blocks = r.value_heads + (r.channels + 255) / 256;
+    const uint32_t conv_blocks = (r.channels + 255) / 256;
     if (r.key_dim == kDk && r.value_dim == kHeadDv) {
-        SR_LAUNCH("gdn_rollback_kernel", gdn_rollback_kernel, dim3(blocks), dim3(256), 0, stream, p);
+        const dim3 grid(r.value_heads * kRbBlocks + conv_blocks);
+        const bool key_vec = r.value_heads % 4 == 0;
+        if (key_vec && r.conv_k == 4) {
+            SR_LAUNCH("gdn_rollback_kernel", (gdn_rollback_kernel<true, 3>), grid, dim3(256), 0,
+                      stream, p);
+        } else if (key_vec) {
+            SR_LAUNCH("gdn_rollback_kernel", (gdn_rollback_kernel<true, 0>), grid, dim3(256), 0,
+                      stream, p);
+        } else {
+            SR_LAUNCH("gdn_rollback_kernel", (gdn_rollback_kernel<false, 0>), grid, dim3(256), 0,
+                      stream, p);
+        }
     } else {
         const RollbackGenericParams q{p, r.key_dim, r.value_dim};
-        SR_LAUNCH("gdn_rollback_generic_kernel", gdn_rollback_generic_kernel, dim3(blocks),
-                  dim3(256), 0, stream, q);
+        SR_LAUNCH("gdn_rollback_generic_kernel", gdn_rollback_generic_kernel,
+                  dim3(r.value_heads + conv_blocks), dim3(256), 0, stream, q);
     }
     return hipGetLastError();
 }

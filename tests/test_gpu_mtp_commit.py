@@ -174,3 +174,29 @@ def test_hybrid_commit_attention_truncate_and_gdn_rollback(pkg, backend, rng):
     assert kv.len(seq) == ctx + j + 1
     kv.destroy()
     gdn.destroy()
+
+
+@pytest.mark.parametrize("hk,hv,conv,rows", [(2, 4, 4, 9), (1, 8, 3, 5), (3, 3, 4, 8), (1, 2, 8, 9),
+                                             (2, 2, 2, 4)])
+def test_gdn_rollback_head_counts_conv_kernels_and_record_batches(pkg, backend, rng, hk, hv, conv,
+                                                                  rows):
+    # head counts that are and are not a multiple of 4 (16-byte key records),
+    # conv kernels 2..8, and kept rows on both sides of a batch of 4 records
+    L = Layer(rng, hk, hv, 128, 128, conv)
+    pool = pkg.GdnState(backend, hk, hv, 128, 128, conv, 3, keep_rows=rows)
+    s = pool.open()
+    plugin_rows(pkg, backend, pool, L, [s], [2], L.inputs(rng, 2))
+    pre = pool.fork(s)
+    x = L.inputs(rng, rows)
+    gdn_rows_keep(pkg, backend, pool, L, [s], [rows], x)
+    for j in sorted({0, 1, 3, 4, 5, rows - 1, rows}):
+        pool.rollback(s, j)
+        m, h = pool.read(s)
+        f = pool.fork(pre)
+        for r in range(j):  # one row a call
+            plugin_rows(pkg, backend, pool, L, [f], [1], rows_of(x, r, r + 1))
+        fm, fh = pool.read(f)
+        assert np.array_equal(m, fm), f"state after rollback to row {j}"
+        assert np.array_equal(h, fh), f"history after rollback to row {j}"
+        pool.close(f)
+    pool.destroy()

@@ -189,7 +189,7 @@ def test_gdn_rollback_head_counts_conv_kernels_and_record_batches(pkg, backend, 
     pre = pool.fork(s)
     x = L.inputs(rng, rows)
     gdn_rows_keep(pkg, backend, pool, L, [s], [rows], x)
-    for j in sorted({0, 1, 3, 4, 5, rows - 1, rows}):
+    for j in sorted(k for k in {0, 1, 3, 4, 5, rows - 1, rows} if k <= rows):
         pool.rollback(s, j)
         m, h = pool.read(s)
         f = pool.fork(pre)

@@ -108,14 +108,14 @@ struct ConvChan {
         float acc = 0.0f;
 #pragma unroll
         for (int j = 0; j < kMaxK - 1; ++j) {
-            if (j + 1 < (int)K) acc += hist[j] * w[j];
+            if (j + 1 < (int)K) acc = fmaf(hist[j], w[j], acc);
         }
         float wl = 0.0f;
 #pragma unroll
         for (int j = 0; j < kMaxK; ++j) {
             if (j + 1 == (int)K) wl = w[j];
         }
-        const float value = acc + x * wl;
+        const float value = fmaf(x, wl, acc);
 #pragma unroll
         for (int j = 0; j < kMaxK - 1; ++j) {
             if (j + 2 < (int)K) hist[j] = hist[j + 1];
@@ -265,10 +265,9 @@ __global__ void __launch_bounds__(kThreads) gdn_delta_kernel(const GdnParams p) 
 // state row, 8 rows per 16-lane group, 8 dims per lane), so the q/k/v conv
 // channels of the head are computed once and the per-head RMSNorm * silu(z)
 // of Gdn::forward (native.rs:737-740) runs in the same kernel: no raw-output
-// round trip and no second launch.  Every global input of the first row -
-// state, history, conv weights, qkv, z, a, b - is requested before the
-// first barrier, and each later row's inputs are loaded while the current
-// row computes.  Used for decode-sized calls (few rows per sequence), where
+// round trip and no second launch.  Every global input of the first batch of
+// rows - state, history, conv weights, qkv, z, a, b - is requested before the
+// first barrier.  Used for decode-sized calls (few rows per sequence), where
 // the sequences x heads workgroups fill the GPU.
 // ---------------------------------------------------------------------------
 constexpr int kHeadDv = 128;
@@ -314,20 +313,32 @@ struct HeadArgs {
 };
 constexpr int kHeadCh = 2 * kDk + kHeadDv;  // q, k and v channels of one head
 constexpr int kHeadThreads = 512;
+constexpr int kHeadRows = 8;  // rows per batch of a multi-row call (one per wave)
+static_assert(kHeadThreads >= kHeadCh && kHeadThreads / 64 >= kHeadRows, "thread layout");
 
-template <int NTH, class Conv>
-__global__ void __launch_bounds__(NTH) gdn_head_kernel(const GdnParams p, const float *norm,
-                                                            const void *z, float *out,
-                                                            uint32_t *err_word, float eps) {
-    __shared__ float conv_s[kHeadCh];
-    __shared__ float out_s[kHeadDv];
-    __shared__ float red_s[2];
-    __shared__ float ab_s[2];
+// NR: rows per batch, 1 for calls with one row per sequence, else kHeadRows.
+// Only the delta rule is serial over the rows: the conv (registers of a
+// channel's thread), the q/k norms and the output norms of a batch's rows run
+// first and last, a row per wave, so a batch takes four barriers where each
+// row used to take three; between them the state rows of a 16-lane group
+// step through the batch without any.  The multiply-adds are written out, so
+// that both forms (and gdn_rollback_kernel) round alike.  4 sequences x 5 rows at 32 heads:
+// 16.8 to 12.3 us a call.
+template <class Conv, int NR>
+__global__ void __launch_bounds__(kHeadThreads) gdn_head_kernel(const GdnParams p,
+                                                                const float *norm, const void *z,
+                                                                float *out, uint32_t *err_word,
+                                                                float eps) {
+    constexpr int NTH = kHeadThreads;
+    __shared__ __align__(16) float conv_s[NR][kHeadCh];
+    __shared__ float out_s[NR][kHeadDv];
+    __shared__ float red_s[NR][2];
+    __shared__ float ab_s[NR][2];
 
     constexpr int RPG = kHeadDv / (NTH / 16);  // state rows per 16-lane group
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = wave_index();
     const int group = tid >> 4;
     const int l16 = tid & 15;
     // Every kernel argument used below is read here, in one batch of scalar
@@ -354,42 +365,39 @@ __global__ void __launch_bounds__(NTH) gdn_head_kernel(const GdnParams p, const 
         if (c < 2 * kDk) return key_width + kh * kDk + (c - kDk);
         return 2 * key_width + h * kHeadDv + (c - 2 * kDk);
     };
-    // this thread's conv channels: tid (if < 384), and tid + NTH when that is
-    // < 384 (only with fewer than 384 threads)
-    constexpr bool kTwo = NTH < kHeadCh;
+    // this thread's conv channel
     const bool one = tid < kHeadCh;
-    const bool two = kTwo && tid + NTH < kHeadCh;
     const uint32_t ch0 = one ? chan(tid) : 0;
-    const uint32_t ch1 = two ? chan(tid + NTH) : 0;
 
     const size_t hist_slot = ((size_t)m.parity * a.max_slots + m.slot) * a.channels;
     const size_t hist_next = ((size_t)(1 - m.parity) * a.max_slots + m.slot) * a.channels;
     // (all loads unconditional: a conditional load ends in a wait for every
     // load in flight; threads without a channel read channel 0 and ignore it)
-    Conv cv0, cv1;
+    Conv cv0;
     cv0.load(a.history + (hist_slot + ch0) * K1, a.conv_w + (size_t)ch0 * a.conv_k, a.conv_k);
-    if constexpr (kTwo) {
-        cv1.load(a.history + (hist_slot + ch1) * K1, a.conv_w + (size_t)ch1 * a.conv_k, a.conv_k);
-    }
-    // inputs of a row: qkv channels, z of this head (dims lane and lane + 64,
-    // used by wave 0), a and b
-    // a and b are the same for every lane; read through a per-lane offset the
-    // compiler cannot fold (zero), they stay in vector registers.  As
-    // wave-uniform values they were moved to scalar registers right after
-    // the next row's loads, and that move waited for every load in flight,
-    // the whole state included.
-    uint32_t vzero = 0;
-    asm volatile("" : "+v"(vzero));
-    float x0 = 0.0f, x1 = 0.0f, z0 = 0.0f, z1 = 0.0f, av = 0.0f, bv = 0.0f;
-    auto load_row = [&](size_t row) {
-        x0 = load_act_nb(a.qkv, row * a.channels + ch0, bf16_in);
-        if constexpr (kTwo) x1 = load_act_nb(a.qkv, row * a.channels + ch1, bf16_in);
-        z0 = load_act_nb(a.z, row * width + h * kHeadDv + lane, bf16_in);
-        z1 = load_act_nb(a.z, row * width + h * kHeadDv + lane + 64, bf16_in);
-        av = load_act_nb(a.a, row * a.value_heads + h + vzero, bf16_in);
-        bv = load_act_nb(a.b, row * a.value_heads + h + vzero, bf16_in);
+    // inputs of a batch of rows: this channel's qkv of every row, z of this
+    // head (dims lane and lane + 64) of the wave's row, a and b of the lane's
+    // row (lanes 0 .. NR - 1 of wave 0 use them; read through per-lane
+    // offsets they stay in vector registers.  As wave-uniform values they
+    // were moved to scalar registers, and that move waited for every load in
+    // flight, the whole state included.)  Rows past the last read it again.
+    float x[NR], z0 = 0.0f, z1 = 0.0f, av = 0.0f, bv = 0.0f;
+    uint32_t lrow = (uint32_t)lane & (NR - 1);
+    asm volatile("" : "+v"(lrow));
+    auto load_rows = [&](uint32_t r0) __attribute__((always_inline)) {
+        const uint32_t last = m.rows - 1;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            x[r] = load_act_nb(a.qkv, (size_t)(m.row0 + min(r0 + r, last)) * a.channels + ch0, bf16_in);
+        }
+        const size_t zrow = m.row0 + min(r0 + (NR == 1 ? 0u : (uint32_t)wave), last);
+        z0 = load_act_nb(a.z, zrow * width + h * kHeadDv + lane, bf16_in);
+        z1 = load_act_nb(a.z, zrow * width + h * kHeadDv + lane + 64, bf16_in);
+        const size_t abrow = m.row0 + min(r0 + lrow, last);
+        av = load_act_nb(a.a, abrow * a.value_heads + h, bf16_in);
+        bv = load_act_nb(a.b, abrow * a.value_heads + h, bf16_in);
     };
-    load_row(m.row0);
+    load_rows(0);
     // state rows v = (NTH/16) i + group, dims [4 l16, 4 l16 + 4) and
     // [64 + 4 l16, 64 + 4 l16 + 4): each 16-byte load or store instruction
     // then covers 256 contiguous bytes of a row; requested after
@@ -422,104 +430,110 @@ __global__ void __launch_bounds__(NTH) gdn_head_kernel(const GdnParams p, const 
     }
     const float a_log_e = expf(a_log_v);
     const float qscale = 1.0f / sqrtf((float)kDk);  // math.rs:213
-    __syncthreads();
 
-    for (uint32_t r = 0; r < m.rows; ++r) {
-        const size_t row = (size_t)m.row0 + r;
-        float *rec = keep ? a.records + ((size_t)m.slot * a.keep_rows + r) * a.rec_stride : nullptr;
+    for (uint32_t r0 = 0; r0 < m.rows; r0 += NR) {
+        const uint32_t nb = NR == 1 ? 1u : min(m.rows - r0, (uint32_t)NR);
+        // the batch's records, row r0 + r at rec0 + r * rec_stride
+        float *rec0 = keep ? a.records + ((size_t)m.slot * a.keep_rows + r0) * a.rec_stride : nullptr;
+        if (NR > 1 && r0 > 0) load_rows(r0);
         // A. causal conv + silu (math.rs:175-185), history in registers
-        if (one) conv_s[tid] = cv0.step(x0, a.conv_k);
-        if constexpr (kTwo) {
-            if (two) conv_s[tid + NTH] = cv1.step(x1, a.conv_k);
-        }
-        if (keep) {
-            // the row's raw conv inputs (q/k channels by the key group's first head)
-            float *rx = rec + a.value_heads + 2 * hv_dv;
-            if (one && (tid >= 2 * kDk || owns_qk)) rx[ch0] = x0;
-            if constexpr (kTwo) {
-                if (two && (tid + NTH >= 2 * kDk || owns_qk)) rx[ch1] = x1;
+        if (one) {
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                if (NR == 1 || (uint32_t)r < nb) conv_s[r][tid] = cv0.step(x[r], a.conv_k);
             }
         }
-        if (tid == 0) {
-            // math.rs:220-221
-            ab_s[0] = expf(-a_log_e * softplus_ref(av + dt));
-            ab_s[1] = ref_sigmoid(bv);
-            if (keep) rec[h] = ab_s[0];
+        if (keep && one && (tid >= 2 * kDk || owns_qk)) {
+            // the rows' raw conv inputs (q/k channels by the key group's first head)
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                if (NR == 1 || (uint32_t)r < nb) {
+                    rec0[(size_t)r * a.rec_stride + a.value_heads + 2 * hv_dv + ch0] = x[r];
+                }
+            }
         }
-        const float zc0 = z0, zc1 = z1;
-        load_row(m.row0 + min(r + 1, m.rows - 1));  // next row's inputs (unconditional)
+        if (tid < (int)nb) {
+            // math.rs:220-221
+            const float alpha = expf(-a_log_e * softplus_ref(av + dt));
+            ab_s[tid][0] = alpha;
+            ab_s[tid][1] = ref_sigmoid(bv);
+            if (keep) rec0[(size_t)tid * a.rec_stride + h] = alpha;
+        }
         __syncthreads();
-        // B. L2 norms of q and k (math.rs:218-219): wave 0 -> q, wave 1 -> k
-        if (wave < 2) {
-            const float y0 = conv_s[wave * kDk + lane];
-            const float y1 = conv_s[wave * kDk + lane + 64];
-            const float ss = sum64(y0 * y0 + y1 * y1);
-            if (lane == 0) red_s[wave] = 1.0f / sqrtf(ss + 1e-6f);
+        // B. L2 norms of q and k (math.rs:218-219), one vector per wave
+        for (uint32_t t = wave; t < 2 * nb; t += NTH / 64) {
+            const float *y = &conv_s[t >> 1][(t & 1) * kDk];
+            const float y0 = y[lane], y1 = y[lane + 64];
+            const float ss = sum64(fmaf(y1, y1, y0 * y0));
+            if (lane == 0) red_s[t >> 1][t & 1] = 1.0f / sqrtf(ss + 1e-6f);
         }
         __syncthreads();
         // C. delta rule on the 8 state rows of this group (math.rs:222-236)
-        const float qi = red_s[0];
-        const float ki = red_s[1];
-        const float alpha = ab_s[0];
-        const float beta = ab_s[1];
-        float kh8[8], qh8[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int dim = (j < 4) ? 4 * l16 + j : kDk / 2 + 4 * l16 + (j - 4);
-            kh8[j] = conv_s[kDk + dim] * ki;
-            qh8[j] = conv_s[dim] * qi;
-            if (keep && group == 0) rec[a.value_heads + hv_dv + h * kDk + dim] = kh8[j];
-        }
-#pragma unroll
-        for (int i = 0; i < RPG; ++i) {
-            const int v = (NTH / 16) * i + group;
-            float pred = 0.0f;
+#pragma unroll 1
+        for (uint32_t r = 0; r < nb; ++r) {
+            const float qi = red_s[r][0];
+            const float ki = red_s[r][1];
+            const float alpha = ab_s[r][0];
+            const float beta = ab_s[r][1];
+            float *rec = keep ? rec0 + (size_t)r * a.rec_stride : nullptr;
+            float kh8[8], qh8[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                S[i][j] *= alpha;
-                pred += S[i][j] * kh8[j];
+                const int dim = (j < 4) ? 4 * l16 + j : kDk / 2 + 4 * l16 + (j - 4);
+                kh8[j] = conv_s[r][kDk + dim] * ki;
+                qh8[j] = conv_s[r][dim] * qi;
+                if (keep && group == 0) rec[a.value_heads + hv_dv + h * kDk + dim] = kh8[j];
             }
-            pred = sum16(pred);
-            const float corr = beta * (conv_s[2 * kDk + v] - pred);
-            if (keep && l16 == 0) rec[a.value_heads + h * kHeadDv + v] = corr;
-            float rd = 0.0f;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                S[i][j] += corr * kh8[j];
-                rd += S[i][j] * qh8[j];
-            }
-            rd = sum16(rd);
-            if (l16 == 0) out_s[v] = rd * qscale;
-            if (r + 1 == m.rows) {
-                // final values of this slice: written now, so that the state
-                // writes stream out while later slices are still arriving
-                float *dst = obase + (size_t)v * kDk;
-                __builtin_nontemporal_store(nt_f32x4{S[i][0], S[i][1], S[i][2], S[i][3]},
-                                            (nt_f32x4 *)dst);
-                __builtin_nontemporal_store(nt_f32x4{S[i][4], S[i][5], S[i][6], S[i][7]},
-                                            (nt_f32x4 *)(dst + kDk / 2));
+            for (int i = 0; i < RPG; ++i) {
+                const int v = (NTH / 16) * i + group;
+                float pred = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    S[i][j] *= alpha;
+                    pred = fmaf(S[i][j], kh8[j], pred);
+                }
+                pred = sum16(pred);
+                const float corr = beta * (conv_s[r][2 * kDk + v] - pred);
+                if (keep && l16 == 0) rec[a.value_heads + h * kHeadDv + v] = corr;
+                float rd = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    S[i][j] = fmaf(corr, kh8[j], S[i][j]);
+                    rd = fmaf(S[i][j], qh8[j], rd);
+                }
+                rd = sum16(rd);
+                if (l16 == 0) out_s[r][v] = rd * qscale;
+                if (r0 + r + 1 == m.rows) {
+                    // final values of this slice: written now, so that the state
+                    // writes stream out while later slices are still arriving
+                    float *dst = obase + (size_t)v * kDk;
+                    __builtin_nontemporal_store(nt_f32x4{S[i][0], S[i][1], S[i][2], S[i][3]},
+                                                (nt_f32x4 *)dst);
+                    __builtin_nontemporal_store(nt_f32x4{S[i][4], S[i][5], S[i][6], S[i][7]},
+                                                (nt_f32x4 *)(dst + kDk / 2));
+                }
             }
         }
         __syncthreads();
-        // D. RMSNorm without offset (math.rs:28-50), then * silu(z)
-        if (wave == 0) {
-            const float o0 = out_s[lane], o1 = out_s[lane + 64];
-            const float ss = sum64(o0 * o0 + o1 * o1);
+        // D. RMSNorm without offset (math.rs:28-50), then * silu(z): a row per wave
+        if ((uint32_t)wave < nb) {
+            const float o0 = out_s[wave][lane], o1 = out_s[wave][lane + 64];
+            const float ss = sum64(fmaf(o1, o1, o0 * o0));
             const float variance = ss / (float)kHeadDv;
             if (!isfinite(variance) && lane == 0) atomicOr(a.err_word, kErrNonFiniteVariance);
             const float inv = 1.0f / sqrtf(variance + a.eps);
-            float *dst = a.out + row * width + h * kHeadDv;
-            dst[lane] = o0 * inv * nw0 * (zc0 * ref_sigmoid(zc0));
-            dst[lane + 64] = o1 * inv * nw1 * (zc1 * ref_sigmoid(zc1));
+            float *dst = a.out + (size_t)(m.row0 + r0 + wave) * width + h * kHeadDv;
+            dst[lane] = o0 * inv * nw0 * (z0 * ref_sigmoid(z0));
+            dst[lane + 64] = o1 * inv * nw1 * (z1 * ref_sigmoid(z1));
         }
+        // (the next batch writes conv_s and red_s, last read before the
+        // barrier above, and out_s only after its own barriers)
     }
 
     // next history: v channels here; q/k channels by the first value head of
     // the key group (the others compute the same values)
     if (one && (tid >= 2 * kDk || owns_qk)) cv0.store(a.history + (hist_next + ch0) * K1, a.conv_k);
-    if constexpr (kTwo) {
-        if (two && (tid + NTH >= 2 * kDk || owns_qk)) cv1.store(a.history + (hist_next + ch1) * K1, a.conv_k);
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -779,8 +793,8 @@ struct ConvK {
     __device__ __forceinline__ float pre(float x, uint32_t) {
         float acc = 0.0f;
 #pragma unroll
-        for (int j = 0; j < K - 1; ++j) acc += hist[j] * w[j];
-        const float value = acc + x * w[K - 1];
+        for (int j = 0; j < K - 1; ++j) acc = fmaf(hist[j], w[j], acc);
+        const float value = fmaf(x, w[K - 1], acc);
 #pragma unroll
         for (int j = 0; j + 1 < K - 1; ++j) hist[j] = hist[j + 1];
         if constexpr (K > 1) hist[K - 2] = x;
@@ -1457,6 +1471,22 @@ hipError_t launch_chunk(hipStream_t stream, const GdnParams &p, uint32_t max_chu
     return hipGetLastError();
 }
 
+// One workgroup per (value head, sequence); a launch with a sequence of more
+// than one row takes the batched form.
+template <class Conv>
+hipError_t launch_head(hipStream_t stream, const GdnParams &p, const GdnLaunch &g,
+                       uint32_t max_rows) {
+    const dim3 grid(p.value_heads, p.nseq);
+    if (max_rows == 1) {
+        SR_LAUNCH("gdn_head_kernel", (gdn_head_kernel<Conv, 1>), grid, dim3(kHeadThreads), 0, stream,
+                  p, g.norm, g.z, g.out, g.err_word, g.eps);
+    } else {
+        SR_LAUNCH("gdn_head_kernel", (gdn_head_kernel<Conv, kHeadRows>), grid, dim3(kHeadThreads), 0,
+                  stream, p, g.norm, g.z, g.out, g.err_word, g.eps);
+    }
+    return hipGetLastError();
+}
+
 struct NormParams {
     const float *raw;   // [rows][Hv*Dv]
     const void *z;      // [rows][Hv*Dv]
@@ -1812,23 +1842,19 @@ hipError_t launch_gdn(hipStream_t stream, const GdnLaunch &g, const GdnSeq *seqs
         p.bf16_in = g.bf16_in ? 1 : 0;
         p.nseq = (uint32_t)n;
         p.chunk_rec = g.chunk_rec;
-        uint32_t chunks = 0, max_chunks = 0;
+        uint32_t chunks = 0, max_chunks = 0, max_rows = 0;
         for (int i = 0; i < n; ++i) {
             const GdnSeq &q = seqs[base + i];
+            max_rows = q.rows > max_rows ? q.rows : max_rows;
             p.meta[i] = GdnMeta{q.slot, q.rows, q.row0, q.parity, q.state_in, q.state_out, chunks};
             const uint32_t nc = (q.rows + kCk - 1) / kCk;
             chunks += nc;
             max_chunks = nc > max_chunks ? nc : max_chunks;
         }
         if (head_kernel) {
-            const dim3 grid(pool->value_heads, (uint32_t)n);
-            if (p.conv_k == 4) {
-                SR_LAUNCH("gdn_head_kernel", (gdn_head_kernel<kHeadThreads, ConvK<4>>), grid,
-                          dim3(kHeadThreads), 0, stream, p, g.norm, g.z, g.out, g.err_word, g.eps);
-            } else {
-                SR_LAUNCH("gdn_head_kernel", (gdn_head_kernel<kHeadThreads, ConvChan>), grid,
-                          dim3(kHeadThreads), 0, stream, p, g.norm, g.z, g.out, g.err_word, g.eps);
-            }
+            const hipError_t e = p.conv_k == 4 ? launch_head<ConvK<4>>(stream, p, g, max_rows)
+                                               : launch_head<ConvChan>(stream, p, g, max_rows);
+            if (e != hipSuccess) return e;
         } else if (route == GdnRoute::kGeneric) {
             const uint32_t hch = 2 * pool->key_dim + pool->value_dim;
             const size_t lds = (size_t)hch * pool->conv_kernel * sizeof(float);

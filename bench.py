@@ -1010,10 +1010,10 @@ def bench_linear_prefill(args, torch, pkg, steps, warmup, rows=2048):
     ms = t0.elapsed_time(t1) / steps
     flops = [2 * rows * o * i for o, i in LINEAR_SHAPES]
     tflops = sum(flops) / (ms * 1e-3) / 1e12
-    # the tiled products: linear_gemm_wide_kernel for calls with many
-    # outputs, linear_gemm_kernel for the others; their mean launch over all
-    # calls, weighted by the share of calls each takes
-    tiled = [kernels[k] for k in ("linear_gemm_wide_kernel", "linear_gemm_kernel") if k in kernels]
+    # the products: linear_gemm_wide_kernel for calls with many output tiles,
+    # linear_rows_kernel for the others; their mean launch over all calls,
+    # weighted by the share of calls each takes
+    tiled = [kernels[k] for k in ("linear_gemm_wide_kernel", "linear_rows_kernel") if k in kernels]
     gemm_us = sum(k["per_call"] * k["us"] for k in tiled) / sum(k["per_call"] for k in tiled)
     # the roofline: the MFMA work of one call (3 passes) over the mean
     # tiled-kernel launch, the calls' FLOPs averaged the same way
@@ -1029,7 +1029,7 @@ def bench_linear_prefill(args, torch, pkg, steps, warmup, rows=2048):
             "bound": "mfma", "achieved": round(mfma_tf, 2), "peak": MFMA_BF16_PEAK_TFS,
             "unit": "TFLOP/s", "frac": round(mfma_tf / MFMA_BF16_PEAK_TFS, 4),
             "traffic": None,
-            "kernel": "linear_gemm_wide_kernel + linear_gemm_kernel (all seven calls; achieved = "
+            "kernel": "linear_gemm_wide_kernel + linear_rows_kernel (all seven calls; achieved = "
                       "3 bf16 MFMA passes per exact product, the calls' mean FLOPs over the mean "
                       "launch)",
             "launch_us_mean": round(float(gemm_us), 2),
@@ -1038,9 +1038,9 @@ def bench_linear_prefill(args, torch, pkg, steps, warmup, rows=2048):
             "fp32_matrix_peak": MFMA_F32_PEAK_TFS,
             "mfma_util": mfma_from_profiles(
                 "linear_prefill_qwen3_8b", [k for k in ("linear_gemm_wide_kernel",
-                                                        "linear_gemm_kernel") if k in kernels],
+                                                        "linear_rows_kernel") if k in kernels],
                 {k: float(kernels[k]["us"]) for k in ("linear_gemm_wide_kernel",
-                                                      "linear_gemm_kernel") if k in kernels}),
+                                                      "linear_rows_kernel") if k in kernels}),
         },
         "kernels": kernels,
     }

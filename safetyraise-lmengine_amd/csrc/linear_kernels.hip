@@ -19,8 +19,8 @@
 // contiguous memory instead of 64 bytes of 16 rows, and every call reads
 // aligned whole blocks whatever its shape.
 //
-// Work split.  A workgroup owns 16 rows x 16 T outputs (T tiles per wave)
-// and a contiguous range of K; its W waves take equal parts of that range
+// Work split of linear_kernel.  A workgroup owns 16 R rows (R = 1, or 2 in one
+// plan) x 16 T outputs (T tiles per wave) and a contiguous range of K; its W waves take equal parts of that range
 // and meet in LDS.  Decode-sized calls (M <= 16) stream every weight row
 // once, the HBM-bound regime the ABI's projections live in; each k block
 // loads 32 bytes of x per lane, used by T tiles, and 8 weight elements per
@@ -137,30 +137,33 @@ __device__ __forceinline__ void split3(const f32x8 &x, bf16x8 &hi, bf16x8 &mid, 
 
 // y: the output, or (grid z > 1) partial sums [grid z][M][N].  T: output tiles per wave (the workgroup owns 16 T
 // outputs; each x fragment a lane loads feeds T MFMAs, so x is read once
-// per 16 T outputs).  W: waves per workgroup, splitting its k range.  kGroup: k
+// per 16 T outputs).  R: row tiles per workgroup (each weight fragment feeds
+// R rows' MFMAs; with R = 2 the weight is read once per 32 rows).  W: waves per workgroup, splitting its k range.  kGroup: k
 // blocks per register set (4; 2 for calls with many workgroups per CU, which
 // then hold more waves per SIMD).  kExact: every wave's k range is a whole
 // number of pairs of groups of whole blocks (the host checks), so no load
 // reaches past it, nothing is masked and the last pair prefetches nothing.
-template <int DT, bool kVec, int T, int W, int kGroup, bool kExact>
+template <int DT, bool kVec, int T, int W, int kGroup, bool kExact, int R>
 __global__ __launch_bounds__(64 * W) void linear_kernel(const float *x, const void *w, float *y,
                                                         uint32_t M, uint32_t N, uint32_t K) {
     static_assert(!kExact || kVec, "exact ranges use the vector loads");
-    __shared__ f32x4 red[W - 1][T][64];
+    __shared__ f32x4 red[W - 1][R][T][64];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const uint32_t r = lane & 15, g = lane >> 4;
-    const uint32_t n0 = blockIdx.x * kLinTile * T, m0 = blockIdx.y * kLinTile;
+    const uint32_t n0 = blockIdx.x * kLinTile * T, m0 = blockIdx.y * kLinTile * R;
     // rows past M / N read the last row and their results are not stored
     if (K == 0) {  // empty sums (uniform): zeros
         if (wave == 0) {
 #pragma unroll
-            for (int u = 0; u < T; ++u)
+            for (int q = 0; q < R; ++q)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const uint32_t m = m0 + 4 * g + i, n = n0 + kLinTile * u + r;
-                    if (m < M && n < N) y[(size_t)m * N + n] = 0.0f;
-                }
+                for (int u = 0; u < T; ++u)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint32_t m = m0 + kLinTile * q + 4 * g + i, n = n0 + kLinTile * u + r;
+                        if (m < M && n < N) y[(size_t)m * N + n] = 0.0f;
+                    }
         }
         return;
     }
@@ -169,7 +172,9 @@ __global__ __launch_bounds__(64 * W) void linear_kernel(const float *x, const vo
     // tile instead of 8 v_mfma_f32_16x16x4f32
     constexpr bool kTiled = DT == SAFETYRAISE_KERNEL_DTYPE_BF16;
     const uint32_t nblk = (K + kLinBlock - 1) / kLinBlock;
-    const size_t xrow = (size_t)min(m0 + r, M - 1) * K;
+    size_t xrow[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) xrow[q] = (size_t)min(m0 + kLinTile * q + r, M - 1) * K;
     // row-major weights: the row of output r of each tile; tiled: this
     // lane's 16 bytes in block 0 of each tile (tiles past N read the last)
     size_t wrow[T];
@@ -195,17 +200,20 @@ __global__ __launch_bounds__(64 * W) void linear_kernel(const float *x, const vo
     // explicitly, so the compiler cannot merge them into one and wait for
     // loads it has just issued)
     using WV = std::conditional_t<kTiled, bf16x8, f32x8>;
-    f32x8 xa[kGroup], xb[kGroup];
+    f32x8 xa[kGroup][R], xb[kGroup][R];
     WV wa[kGroup][T], wb[kGroup][T];
-    auto load_group = [&](uint32_t b, f32x8 (&xv)[kGroup], WV (&wv)[kGroup][T])
+    auto load_group = [&](uint32_t b, f32x8 (&xv)[kGroup][R], WV (&wv)[kGroup][T])
                           __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < kGroup; ++j) {
             const uint32_t k = kLinBlock * (b + j) + 8 * g;
-            if constexpr (kExact) {
-                xv[j] = load8_at<SAFETYRAISE_KERNEL_DTYPE_F32>(x, xrow + k);
-            } else {
-                xv[j] = load8<SAFETYRAISE_KERNEL_DTYPE_F32, kVec>(x, xrow, k, K, kend);
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                if constexpr (kExact) {
+                    xv[j][q] = load8_at<SAFETYRAISE_KERNEL_DTYPE_F32>(x, xrow[q] + k);
+                } else {
+                    xv[j][q] = load8<SAFETYRAISE_KERNEL_DTYPE_F32, kVec>(x, xrow[q], k, K, kend);
+                }
             }
 #pragma unroll
             for (int u = 0; u < T; ++u) {
@@ -232,32 +240,39 @@ __global__ __launch_bounds__(64 * W) void linear_kernel(const float *x, const vo
     // t % kChains, or one chain per part of x), so consecutive MFMAs do not
     // wait for each other's results
     constexpr int kChains = kTiled ? 3 : (T == 1 ? 4 : 2);
-    f32x4 acc4[T][kChains];
+    f32x4 acc4[R][T][kChains];
 #pragma unroll
-    for (int u = 0; u < T; ++u)
+    for (int q = 0; q < R; ++q)
 #pragma unroll
-        for (int c = 0; c < kChains; ++c) acc4[u][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    auto mfma_group = [&](const f32x8 (&xv)[kGroup], const WV (&wv)[kGroup][T])
+        for (int u = 0; u < T; ++u)
+#pragma unroll
+            for (int c = 0; c < kChains; ++c) acc4[q][u][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto mfma_group = [&](const f32x8 (&xv)[kGroup][R], const WV (&wv)[kGroup][T])
                           __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < kGroup; ++j) {
             if constexpr (kTiled) {
-                bf16x8 part[3];
-                split3(xv[j], part[0], part[1], part[2]);
 #pragma unroll
-                for (int c = 0; c < 3; ++c)
+                for (int q = 0; q < R; ++q) {
+                    bf16x8 part[3];
+                    split3(xv[j][q], part[0], part[1], part[2]);
 #pragma unroll
-                    for (int u = 0; u < T; ++u)
-                        acc4[u][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part[c], wv[j][u],
-                                                                             acc4[u][c], 0, 0, 0);
+                    for (int c = 0; c < 3; ++c)
+#pragma unroll
+                        for (int u = 0; u < T; ++u)
+                            acc4[q][u][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                part[c], wv[j][u], acc4[q][u][c], 0, 0, 0);
+                }
             } else {
 #pragma unroll
                 for (int t = 0; t < 8; ++t) {
 #pragma unroll
-                    for (int u = 0; u < T; ++u) {
-                        f32x4 &a = acc4[u][t % kChains];
-                        a = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[j][t], wv[j][u][t], a, 0, 0, 0);
-                    }
+                    for (int u = 0; u < T; ++u)
+#pragma unroll
+                        for (int q = 0; q < R; ++q) {
+                            f32x4 &a = acc4[q][u][t % kChains];
+                            a = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[j][q][t], wv[j][u][t], a, 0, 0, 0);
+                        }
                 }
             }
         }
@@ -287,31 +302,37 @@ __global__ __launch_bounds__(64 * W) void linear_kernel(const float *x, const vo
         }
     }
     // the chains summed last to first (with split x: lo + mid, then hi)
-    f32x4 acc[T];
+    f32x4 acc[R][T];
 #pragma unroll
-    for (int u = 0; u < T; ++u) {
-        acc[u] = acc4[u][kChains - 1];
+    for (int q = 0; q < R; ++q)
 #pragma unroll
-        for (int c = kChains - 2; c >= 0; --c) acc[u] += acc4[u][c];
-    }
+        for (int u = 0; u < T; ++u) {
+            acc[q][u] = acc4[q][u][kChains - 1];
+#pragma unroll
+            for (int c = kChains - 2; c >= 0; --c) acc[q][u] += acc4[q][u][c];
+        }
     if (wave > 0) {
 #pragma unroll
-        for (int u = 0; u < T; ++u) red[wave - 1][u][lane] = acc[u];
+        for (int q = 0; q < R; ++q)
+#pragma unroll
+            for (int u = 0; u < T; ++u) red[wave - 1][q][u][lane] = acc[q][u];
     }
     __syncthreads();
     if (wave != 0) return;
 #pragma unroll
-    for (int u = 0; u < T; ++u) {
-        f32x4 sum = acc[u];
+    for (int q = 0; q < R; ++q)
 #pragma unroll
-        for (int j = 0; j < W - 1; ++j) sum += red[j][u][lane];
-        const uint32_t n = n0 + kLinTile * u + r;
+        for (int u = 0; u < T; ++u) {
+            f32x4 sum = acc[q][u];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t m = m0 + 4 * g + i;
-            if (m < M && n < N) y[(size_t)m * N + n] = sum[i];
+            for (int j = 0; j < W - 1; ++j) sum += red[j][q][u][lane];
+            const uint32_t n = n0 + kLinTile * u + r;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t m = m0 + kLinTile * q + 4 * g + i;
+                if (m < M && n < N) y[(size_t)m * N + n] = sum[i];
+            }
         }
-    }
 }
 
 // y[i] = sum over z < splits of part[z][i], added in z order (splits <=
@@ -330,35 +351,188 @@ __global__ __launch_bounds__(256) void linear_split_sum_kernel(const float *part
 }
 
 // ---------------------------------------------------------------------------
-// Calls with many rows (prefill chunks) on bf16 weights: a tiled product.
-// linear_split_x_kernel first writes x once as its three bf16 parts (split3)
-// in MFMA lane order: for row tile t (16 rows), k block b (32 columns) and
-// part c, the 1 KB at ((t * nblk + b) * 3 + c) KB holds, at lane 16 g + r,
-// x[16 t + r][32 b + 8 g .. + 8].  linear_gemm_kernel then owns 128 rows x
-// 128 outputs per workgroup; its 8 waves are 4 (rows) x 2 (outputs), each
-// computing 32 rows x 64 outputs (2 x 4 tiles of 16 x 16).  Per stage of 64 k
-// (two 32-k blocks) the workgroup copies its 48 KB of split x straight from
-// memory into LDS (global_load_lds: no registers, no VALU), double-buffered;
-// a wave reads its row tiles' parts with ds_read_b128 and its 4 weight tiles
-// straight from the tile layout (16 bytes per lane, prefetched one stage
-// ahead).  So x is read once per 128 outputs and the weight once per 128
-// rows, and the loop is loads and MFMAs only.  Two accumulation chains per
-// tile: the hi part's products, and the mid and lo parts' (three chains of 8
-// tiles would not fit the registers of two waves per SIMD).  Requires K % 64
-// == 0; rows past M and tiles past N read clamped copies whose results are
-// not stored.
+// linear_rows_kernel: bf16 weights with more than one row tile, up to the calls
+// whose 128 x 128 output tiles fill the chip on their own.  A workgroup owns
+// 16 RT rows (32 or 64) x 128 outputs, 8 waves x 16 outputs, and a range of K
+// (grid z, whole stages; linear_split_sum_kernel adds the partial sums).  Each
+// weight byte is read once per workgroup, straight from the tile layout into
+// registers one stage ahead, and feeds 3 RT MFMAs; per stage of 8 / RT k
+// blocks every thread splits one x fragment (16 RT rows x 8 / RT blocks = 512
+// fragments) into LDS, double-buffered, one barrier per stage, and the 8 waves
+// share it: x needs no pass of its own.  Two workgroups per CU (48 KB of LDS,
+// at most 128 registers) cover each other's barriers and loads.
+// What bounds it: up to 64 rows the weight stream (33.5 MB at 32 rows 12.8 us,
+// 100 MB at 64 rows 35 us, the partial sums' launch included), above that the
+// MFMAs and LDS reads (1024 rows x 4096 x 4096: 99 us, 1.04 PFLOP/s of bf16
+// passes).  linear_kernel, which reads the weight once per 16 rows, took 19.2
+// and 63 us, the tiled product below, with 256 workgroups there, 171 us.
+// Measured and dropped: two output tiles per wave (spills at two workgroups
+// per CU, 41 us at one), loads four stages ahead (36.6), the next block's LDS
+// reads issued ahead (29.7 against 28.2 us at 32 rows), stages started in
+// another order per workgroup (32.4).
+// Sums: the hi parts in one chain, mid and lo in another, moved to a total
+// every kLinFlush columns, so that no chain is longer than those of
+// linear_kernel.
+// Requires K % (32 * 8 / RT) == 0.  kVec: x is 16-byte aligned.
 // ---------------------------------------------------------------------------
-constexpr int kGemmWM = 4, kGemmWN = 2;  // waves over rows, over outputs
-constexpr int kGemmRT = 2, kGemmCT = 4;  // 16 x 16 tiles per wave: rows, outputs
-constexpr int kGemmBM = 16 * kGemmRT * kGemmWM;  // 128 rows per workgroup
-constexpr int kGemmBN = 16 * kGemmCT * kGemmWN;  // 128 outputs per workgroup
-constexpr int kGemmKB = 2;                       // 32-k blocks per stage
-constexpr uint32_t kGemmK = kGemmKB * kLinBlock;  // 64 k per stage
-constexpr uint32_t kGemmMinRows = 64;             // rows from which calls take this kernel
-// one stage of split x in LDS: [k block][part][row tile][lane] x 16 bytes
-constexpr int kGemmStageBytes = kGemmKB * 3 * (kGemmBM / 16) * 64 * 16;
-constexpr int kGemmStageBlocks = kGemmStageBytes / 1024;  // 1 KB blocks per stage (48)
+constexpr int kRowsWaves = 8;
+constexpr int kRowsBN = kLinTile * kRowsWaves;  // 128 outputs per workgroup
+constexpr uint32_t kLinFlush = 512;
 
+template <int RT, bool kVec>
+__global__ __launch_bounds__(64 * kRowsWaves, 4) void linear_rows_kernel(const float *x, const void *w,
+                                                                       float *y, uint32_t M,
+                                                                       uint32_t N, uint32_t K) {
+    constexpr int KB = 8 / RT;  // k blocks per stage
+    constexpr uint32_t kStageBytes = KB * 3 * RT * 1024;
+    constexpr uint32_t kFlushStages = kLinFlush / (KB * kLinBlock);
+    static_assert(kFlushStages % 2 == 0, "flushed after a pair of stages");
+    __shared__ __align__(16) unsigned char xs[2 * kStageBytes];
+    typedef uint32_t u32x4r __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) unsigned char lds_byte;
+    typedef __attribute__((address_space(3))) u32x4r lds_u32x4r;
+    lds_byte *lds = (lds_byte *)xs;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const uint32_t r = lane & 15, g = lane >> 4;
+    const uint32_t nblk = K / kLinBlock;
+    const uint32_t units = nblk / KB;
+    const uint32_t u0 = (uint32_t)((uint64_t)units * blockIdx.z / gridDim.z);
+    const uint32_t u1 = (uint32_t)((uint64_t)units * (blockIdx.z + 1) / gridDim.z);
+    const uint32_t m0 = blockIdx.y * kLinTile * RT;
+    const uint32_t tile = blockIdx.x * kRowsWaves + wave;  // the wave's output tile
+
+    // the x fragment this thread splits: row tile wave % RT, k block wave / RT
+    // of the stage, 8 columns of row r (rows past M read the last one)
+    const uint32_t xrt = (uint32_t)wave % RT, xkb = (uint32_t)wave / RT;
+    const float *xrow = x + (size_t)min(m0 + kLinTile * xrt + r, M - 1) * K;
+    const uint32_t xdst = ((xkb * 3) * RT + xrt) * 1024 + lane * 16;  // part 0; the others RT KB on
+    // this lane's 16 bytes of block 0 of its tile (tiles past N read the last)
+    const uint16_t *wt =
+        (const uint16_t *)w + (size_t)min(tile, (N - 1) / kLinTile) * nblk * 512 + (size_t)lane * 8;
+    // (stages past the range load its last one again, unused)
+    auto load_x = [&](uint32_t s) __attribute__((always_inline)) {
+        const float *src = xrow + kLinBlock * (KB * min(s, u1 - 1) + xkb) + 8 * g;
+        if constexpr (kVec) return load8_at<SAFETYRAISE_KERNEL_DTYPE_F32>(src, 0);
+        f32x8 v;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = src[j];
+        return v;
+    };
+    auto store_x = [&](uint32_t buf, const f32x8 &v) __attribute__((always_inline)) {
+        bf16x8 part[3];
+        split3(v, part[0], part[1], part[2]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            *(lds_u32x4r *)(lds + buf * kStageBytes + xdst + c * RT * 1024) =
+                __builtin_bit_cast(u32x4r, part[c]);
+        }
+    };
+    auto load_w = [&](uint32_t s, bf16x8 (&wv)[KB]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+            wv[kb] = *(const bf16x8 *)(wt + (size_t)(KB * min(s, u1 - 1) + kb) * 512);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    f32x4 acc[RT][2], tot[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) acc[i][0] = acc[i][1] = tot[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto compute = [&](uint32_t buf, const bf16x8 (&wv)[KB]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                bf16x8 a[RT];
+#pragma unroll
+                for (int i = 0; i < RT; ++i) {
+                    a[i] = __builtin_bit_cast(bf16x8, *(lds_u32x4r *)(lds + buf * kStageBytes +
+                                                                      ((kb * 3 + c) * RT + i) * 1024 +
+                                                                      lane * 16));
+                }
+#pragma unroll
+                for (int i = 0; i < RT; ++i) {
+                    f32x4 &ac = acc[i][c == 0 ? 0 : 1];
+                    ac = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], wv[kb], ac, 0, 0, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto flush = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+            tot[i] += acc[i][1] + acc[i][0];
+            acc[i][0] = acc[i][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    };
+
+    // stage u0 + i: x in buffer i & 1, its weights in wa (even i) or wb.  The
+    // next stage's x is stored into the other buffer, last read before the
+    // previous barrier, while this one is multiplied.
+    bf16x8 wa[KB], wb[KB];
+    f32x8 xa = load_x(u0);
+    load_w(u0, wa);
+    f32x8 xb = load_x(u0 + 1);
+    load_w(u0 + 1, wb);
+    store_x(0, xa);
+    xa = load_x(u0 + 2);
+    __syncthreads();
+    uint32_t since = 0;
+    for (uint32_t s = u0; s < u1; s += 2) {
+        store_x(1, xb);
+        xb = load_x(s + 3);
+        compute(0, wa);
+        load_w(s + 2, wa);
+        __syncthreads();
+        store_x(0, xa);
+        xa = load_x(s + 4);
+        if (s + 1 < u1) compute(1, wb);
+        load_w(s + 3, wb);
+        __syncthreads();
+        since += 2;
+        if (since == kFlushStages) {
+            flush();
+            since = 0;
+        }
+    }
+    flush();
+    // lane (r, g) holds y[row 4g + e][output r] of each tile in element e
+    y += (size_t)blockIdx.z * M * N;
+    const uint32_t n = tile * kLinTile + r;
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t m = m0 + kLinTile * i + 4 * g + e;
+            if (m < M && n < N) y[(size_t)m * N + n] = tot[i][e];
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Calls whose 128 x 128 output tiles exceed two per CU (large prefill chunks):
+// a tiled product.  linear_split_x_kernel first writes x once as its three
+// bf16 parts (split3) in MFMA lane order: for row tile t (16 rows), k block b
+// (32 columns) and part c, the 1 KB at ((t * nblk + b) * 3 + c) KB holds, at
+// lane 16 g + r, x[16 t + r][32 b + 8 g .. + 8].  linear_gemm_wide_kernel then
+// owns 128 rows x 128 outputs per workgroup: 4 waves, each 64 rows x 64
+// outputs (4 x 4 tiles of 16 x 16), two workgroups per CU.  Per stage of one
+// k block the workgroup copies its 24 KB of split x straight from memory into
+// LDS (global_load_lds: no registers, no VALU), double-buffered; a wave reads
+// 12 A fragments from LDS and 4 weight fragments from the tile layout (16
+// bytes per lane, prefetched one stage ahead) for 48 MFMAs, and each
+// workgroup's barriers are covered by the other's work.  One accumulation
+// chain per tile.  Requires K % 64 == 0; rows past M and tiles past N read
+// clamped copies whose results are not stored.
+// Measured at 2048 rows x 12288 x 4096: 409 us with the split (1.51 PFLOP/s of
+// bf16 passes), 501 us with linear_rows_kernel; 64 x 128 wave tiles (256
+// accumulators, one workgroup per CU) lost 23 %, the compiler moving
+// accumulators between register files.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kGemmK = 64;  // K granularity: stages in pairs
 // Thread c: lane c % 64 of (row tile, k block) c / 64, its 8 values split.
 template <bool kVec>
 __global__ __launch_bounds__(256) void linear_split_x_kernel(const float *x, uint16_t *xs,
@@ -388,147 +562,6 @@ __global__ __launch_bounds__(256) void linear_split_x_kernel(const float *x, uin
     }
 }
 
-__global__ __launch_bounds__(512) void linear_gemm_kernel(const uint16_t *xs, const void *w,
-                                                         float *y, uint32_t M, uint32_t N,
-                                                         uint32_t K) {
-    extern __shared__ __align__(16) unsigned char gemm_lds[];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int wm = wave % kGemmWM, wn = wave / kGemmWM;
-    const uint32_t m0 = blockIdx.y * kGemmBM, n0 = blockIdx.x * kGemmBN;
-    const uint32_t nblk = K / kLinBlock;
-    const uint32_t stages = K / kGemmK;
-    const uint32_t last_tile = (N - 1) / kLinTile;
-    const uint32_t last_row_tile = (M - 1) / kLinTile;
-
-    // the split-x blocks this wave copies per stage: blocks q = 6 wave .. +6
-    // of the stage's 48, block q = (k block, part, row tile) in LDS order
-    const uint16_t *xsrc[kGemmStageBlocks / 8];
-    uint32_t xdst[kGemmStageBlocks / 8];
-#pragma unroll
-    for (int i = 0; i < kGemmStageBlocks / 8; ++i) {
-        const uint32_t q = (uint32_t)wave * (kGemmStageBlocks / 8) + i;
-        const uint32_t rt = q % (kGemmBM / 16), part = (q / (kGemmBM / 16)) % 3,
-                       kb = q / (3 * (kGemmBM / 16));
-        const uint32_t t = min(m0 / kLinTile + rt, last_row_tile);
-        xsrc[i] = xs + (((size_t)t * nblk + kb) * 3 + part) * 512 + (size_t)lane * 8;
-        xdst[i] = q * 1024;
-    }
-    // this wave's weight tiles: 16 bytes of block 0 per lane (tiles past N
-    // read the last one)
-    const uint16_t *wt[kGemmCT];
-#pragma unroll
-    for (int j = 0; j < kGemmCT; ++j) {
-        const uint32_t tile = min(n0 / kLinTile + kGemmCT * wn + j, last_tile);
-        wt[j] = (const uint16_t *)w + (size_t)tile * nblk * 512 + (size_t)lane * 8;
-    }
-    typedef uint32_t u32x4g __attribute__((ext_vector_type(4)));
-    typedef __attribute__((address_space(3))) unsigned char lds_byte;
-    lds_byte *lds = (lds_byte *)gemm_lds;
-    auto copy_x = [&](uint32_t s, uint32_t buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < kGemmStageBlocks / 8; ++i) {
-            // a stage's two k blocks: block s of the call's stages is k
-            // blocks 2 s, 2 s + 1, i.e. (2 s) * 3 * 512 elements past block 0
-            __builtin_amdgcn_global_load_lds(xsrc[i] + (size_t)s * kGemmKB * 3 * 512,
-                                             lds + buf * kGemmStageBytes + xdst[i], 16, 0, 0);
-        }
-    };
-    auto load_w = [&](uint32_t s, bf16x8 (&wv)[kGemmKB][kGemmCT]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int kb = 0; kb < kGemmKB; ++kb)
-#pragma unroll
-            for (int j = 0; j < kGemmCT; ++j)
-                wv[kb][j] = *(const bf16x8 *)(wt[j] + (size_t)(kGemmKB * s + kb) * 512);
-    };
-
-    f32x4 acc[kGemmRT][kGemmCT][2];
-#pragma unroll
-    for (int i = 0; i < kGemmRT; ++i)
-#pragma unroll
-        for (int j = 0; j < kGemmCT; ++j)
-#pragma unroll
-            for (int c = 0; c < 2; ++c) acc[i][j][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    bf16x8 wa[kGemmKB][kGemmCT], wb[kGemmKB][kGemmCT];
-    copy_x(0, 0);
-    load_w(0, wa);
-    __syncthreads();
-    auto compute = [&](uint32_t buf, const bf16x8 (&wv)[kGemmKB][kGemmCT]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int kb = 0; kb < kGemmKB; ++kb) {
-            bf16x8 a[kGemmRT][3];
-#pragma unroll
-            for (int i = 0; i < kGemmRT; ++i)
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    const uint32_t chunk = ((kb * 3 + c) * (kGemmBM / 16) + kGemmRT * wm + i) * 64 + lane;
-                    a[i][c] = __builtin_bit_cast(
-                        bf16x8, *(const __attribute__((address_space(3))) u32x4g *)(
-                                    lds + buf * kGemmStageBytes + chunk * 16));
-                }
-#pragma unroll
-            for (int c = 0; c < 3; ++c)
-#pragma unroll
-                for (int i = 0; i < kGemmRT; ++i)
-#pragma unroll
-                    for (int j = 0; j < kGemmCT; ++j) {
-                        f32x4 &ac = acc[i][j][c == 0 ? 0 : 1];
-                        ac = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][c], wv[kb][j], ac, 0, 0, 0);
-                    }
-        }
-    };
-    // stages in pairs, so that the two weight register sets alternate by
-    // name; the copy of stage s + 1 into the other buffer is in flight while
-    // stage s computes, and the barrier after it waits for the copy
-    uint32_t s = 0;
-    for (; s + 2 <= stages; s += 2) {
-        const bool more1 = s + 1 < stages;
-        if (more1) {
-            copy_x(s + 1, (s + 1) & 1);
-            load_w(s + 1, wb);
-        }
-        compute(s & 1, wa);
-        __syncthreads();
-        const bool more2 = s + 2 < stages;
-        if (more2) {
-            copy_x(s + 2, s & 1);
-            load_w(s + 2, wa);
-        }
-        compute((s + 1) & 1, wb);
-        __syncthreads();
-    }
-    if (s < stages) compute(s & 1, wa);
-
-    // the mid + lo chain, then hi; lane (r, g) holds y[row 4g + e][output
-    // r] of each tile in element e
-    const uint32_t r = lane & 15, g = lane >> 4;
-#pragma unroll
-    for (int i = 0; i < kGemmRT; ++i)
-#pragma unroll
-        for (int j = 0; j < kGemmCT; ++j) {
-            const f32x4 sum = acc[i][j][1] + acc[i][j][0];
-            const uint32_t n = n0 + kLinTile * (kGemmCT * wn + j) + r;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t m = m0 + kLinTile * (kGemmRT * wm + i) + 4 * g + e;
-                if (m < M && n < N) y[(size_t)m * N + n] = sum[e];
-            }
-        }
-}
-
-// The form for calls with many outputs (at least kWideMinOutputs): 4 waves
-// per 128 x 128 tile, each owning 64 rows x 64 outputs (4 x 4 tiles), two
-// workgroups per CU.  Per 32-k block a wave reads 12 A fragments from LDS and
-// 4 weight fragments from memory for 48 MFMAs: half the weight bytes per
-// MFMA of linear_gemm_kernel's 32 x 64 wave tiles, and a 24 KB stage (one
-// k block), so that two workgroups fit a CU and each one's barriers are
-// covered by the other.  Measured on the Qwen3-8B layer at 2048 rows: 2.19
-// ms per layer against 2.61 with linear_gemm_kernel for every call; 64 x 128
-// wave tiles (256 accumulators, one workgroup per CU) measured 2.70 ms, the
-// compiler moving accumulators between register files, and this form for
-// the 1024-output k/v calls too 2.26 ms (half the CUs idle).
 constexpr int kWideWM = 2, kWideWN = 2;           // waves over rows, over outputs
 constexpr int kWideRT = 4, kWideCT = 4;           // 16 x 16 tiles per wave
 constexpr int kWideBM = 16 * kWideRT * kWideWM;   // 128 rows per workgroup
@@ -536,7 +569,6 @@ constexpr int kWideBN = 16 * kWideCT * kWideWN;   // 128 outputs per workgroup
 constexpr int kWideStageBytes = 3 * (kWideBM / 16) * 1024;  // [part][row tile] 1 KB blocks
 constexpr int kWideStageBlocks = kWideStageBytes / 1024;    // 24
 constexpr int kWideThreads = 64 * kWideWM * kWideWN;
-constexpr uint32_t kWideMinOutputs = 2048;
 
 __global__ __launch_bounds__(kWideThreads, 2) void linear_gemm_wide_kernel(const uint16_t *xs,
                                                                          const void *w, float *y,
@@ -727,14 +759,14 @@ void launch_dt(hipStream_t stream, const float *x, const void *w, float *y, uint
         const bool exact = K % kLinBlock == 0 &&
                            (K / kLinBlock) % (splits * (uint32_t)W * 2u * (uint32_t)kGroup) == 0;
         if (exact) {
-            SR_LAUNCH(name, (linear_kernel<DT, true, T, W, kGroup, true>), grid, dim3(64 * W), 0,
+            SR_LAUNCH(name, (linear_kernel<DT, true, T, W, kGroup, true, 1>), grid, dim3(64 * W), 0,
                       stream, x, w, y, M, N, K);
         } else {
-            SR_LAUNCH(name, (linear_kernel<DT, true, T, W, kGroup, false>), grid, dim3(64 * W), 0,
+            SR_LAUNCH(name, (linear_kernel<DT, true, T, W, kGroup, false, 1>), grid, dim3(64 * W), 0,
                       stream, x, w, y, M, N, K);
         }
     } else {
-        SR_LAUNCH(name, (linear_kernel<DT, false, T, W, kGroup, false>), grid, dim3(64 * W), 0,
+        SR_LAUNCH(name, (linear_kernel<DT, false, T, W, kGroup, false, 1>), grid, dim3(64 * W), 0,
                   stream, x, w, y, M, N, K);
     }
 }
@@ -797,28 +829,110 @@ hipError_t linear_pack_bf16(hipStream_t stream, const void *src, void *dst, uint
 namespace {
 constexpr uint32_t kMaxRows = 65535u * kLinTile;  // grid y limit of one row-tile launch
 
-// Whether a call takes the tiled product: bf16 weight, 64+ rows, K a multiple
-// of 64, and 128 x 128 tiles for at least half the CUs (fewer, and the
-// row-tile kernel's weight stream is faster).  Calls above kMaxRows rows run
-// as row blocks without scratch.
-bool gemm_applies(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus) {
-    if (dtype != SAFETYRAISE_KERNEL_DTYPE_BF16 || M < kGemmMinRows || M > kMaxRows || K == 0 ||
-        K % kGemmK != 0) {
-        return false;
-    }
-    const uint64_t tiles = (uint64_t)((M + kGemmBM - 1) / kGemmBM) * ((N + kGemmBN - 1) / kGemmBN);
-    return 2 * tiles >= (uint64_t)(num_cus > 0 ? num_cus : 1);
-}
-// split x of a tiled-product call: whole row tiles x K x 3 bf16 parts
-size_t gemm_split_bytes(uint32_t M, uint32_t K) {
+// Which kernels a call takes.  All of it rests on cold-weight timings of
+// 13 shapes (K, N of 256 .. 12288) at 17 .. 3000 rows; the figures are us.
+enum class LinRoute {
+    kTile,  // linear_kernel, 16 rows per workgroup (linear_plan)
+    kPair,  // linear_kernel, 32 rows per workgroup
+    kRows,  // linear_rows_kernel
+    kWide,  // split x + linear_gemm_wide_kernel
+};
+struct LinChoice {
+    LinRoute route;
+    uint32_t splits;  // of K over grid z (kRows)
+    size_t scratch;   // bytes the route uses
+};
+
+// Split x of a tiled-product call: whole row tiles x K x 3 bf16 parts.
+size_t split_x_bytes(uint32_t M, uint32_t K) {
     return (size_t)((M + kLinTile - 1) / kLinTile) * kLinTile * K * 3 * sizeof(uint16_t);
+}
+
+// K splits of linear_rows_kernel: the least of stages x time per stage (one
+// workgroup on a CU, two sharing it, or several rounds of two) plus, with a
+// split, the second launch and the partial sums' traffic.  Reproduces the best
+// measured split or one within 5 % of it, e.g. 512 rows of 3072 x 1024: 1
+// (17.6; 2: 25.7), 1024 of 1024 x 4096: 4 (35.1; 1: 55.4, 3: 40.3).
+uint32_t rows_splits(uint32_t M, uint32_t N, uint32_t units, uint32_t base, bool two_tiles,
+                     uint64_t cus, size_t scratch) {
+    const double one = two_tiles ? 1.1 : 0.86, two = two_tiles ? 1.9 : 1.5;  // us per stage
+    const uint64_t outputs = (uint64_t)M * N;
+    uint32_t best = 1;
+    double best_us = 0.0;
+    for (uint32_t s = 1; s <= kLinMaxSplits && s <= units; ++s) {
+        if (s > 1 && (outputs > UINT32_MAX || outputs * s > scratch / sizeof(float))) break;
+        const uint64_t wgs = (uint64_t)base * s;
+        const uint64_t rounds = wgs / (2 * cus), rest = wgs % (2 * cus);
+        double us = (double)((units + s - 1) / s) *
+                    ((double)rounds * two + (rest == 0 ? 0.0 : rest <= cus ? one : two));
+        if (s > 1) us += 3.0 + (double)(outputs * (2 * s + 1) * sizeof(float)) / 5e6;
+        if (s == 1 || us < best_us) {
+            best = s;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
+// scratch: the bytes that are there (SIZE_MAX: as many as the call likes).
+LinChoice linear_choice(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus,
+                        bool x_aligned, size_t scratch) {
+    const uint64_t cus = (uint64_t)(num_cus > 0 ? num_cus : 1);
+    const LinPlan plan = linear_plan(M, N, K, dtype, num_cus);
+    const LinChoice tile = {LinRoute::kTile, plan.splits,
+                            plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0};
+    if (dtype != SAFETYRAISE_KERNEL_DTYPE_BF16 || M <= (uint32_t)kLinTile || M > kMaxRows) return tile;
+    const uint64_t weight = (uint64_t)N * K, work = weight * M;
+    // nearly two 128 x 128 output tiles per CU or more: 2048 rows of 12288 x
+    // 4096 (1536 tiles) 476 against 540 with kRows, of 4096 x 4096 (512) 185 / 210;
+    // with fewer kRows, which can split K: 1500 rows of it (384) 173 / 160, 1024
+    // (256) 160 / 106
+    const uint64_t tiles = (uint64_t)((M + kWideBM - 1) / kWideBM) * ((N + kWideBN - 1) / kWideBN);
+    if (M > 64 && K % kGemmK == 0 && K > 0 && 4 * tiles >= 7 * cus && split_x_bytes(M, K) <= scratch) {
+        return {LinRoute::kWide, 1, split_x_bytes(M, K)};
+    }
+    const bool pair = M <= 2 * kLinTile;
+    // 32 rows, one workgroup of three output tiles on nearly every CU: 12288 x
+    // 4096 25.1 against 34.8 (kTile) and 28.2 (kRows, its best split)
+    if (pair && x_aligned && K % 8 == 0 && 8 * ((uint64_t)(N + 3 * kLinTile - 1) / (3 * kLinTile)) >= 7 * cus) {
+        return {LinRoute::kPair, 1, 0};
+    }
+    const uint32_t stage = pair ? 4 * kLinBlock : 2 * kLinBlock;
+    if (K == 0 || K % stage != 0) return tile;
+    // Where the stages and the second launch cost less than reading the
+    // weight once per 16 rows: 32 rows of 4096 x 4096 12.8 against 19.2, of
+    // 2048 x 6144 13.0 / 15.2, but 2048 x 2048 8.3 / 6.7 and, where kTile
+    // covers the CUs without a split, 6144 x 2048 13.0 / 10.0; 64 rows of
+    // 2048 x 6144 17.8 / 27.2, 1024 x 4096 13.2 / 10.8, 33 of 6144 x 2048 15.0 /
+    // 13.8; 100 of 2048 x 2048 12.5 / 15.7, 512 of 512 x 2048 13.6 / 15.3, but
+    // 333 of it 12.3 / 8.8 and 65 (two row blocks, one nearly empty) of 6144 x
+    // 2048 20.6 / 19.6; short K: 256 of 3072 x 1024 16.5 / 15.8, 300 of it 17.9 /
+    // 18.8.
+    bool pays;
+    if (pair) {
+        pays = weight >= (12u << 20) && (plan.T < 3 || plan.splits > 1 || weight >= (24u << 20));
+    } else if (M <= 64) {
+        pays = weight >= (K < 4096 ? 16u << 20 : 12u << 20);
+    } else if (M <= 80 && K < 4096) {
+        pays = work >= 1000000000u;
+    } else {
+        pays = work >= (K < 2048 ? 850000000u : N < 1024 ? 500000000u : 300000000u);
+    }
+    if (!pays) return tile;
+    const uint32_t rows = pair ? 2 * kLinTile : 4 * kLinTile;
+    const uint32_t base = ((N + kRowsBN - 1) / kRowsBN) * ((M + rows - 1) / rows);
+    const uint32_t s = rows_splits(M, N, K / stage, base, pair, cus, scratch);
+    return {LinRoute::kRows, s, s > 1 ? (size_t)s * M * N * sizeof(float) : 0};
 }
 }  // namespace
 
 size_t linear_scratch_bytes(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus) {
-    if (gemm_applies(M, N, K, dtype, num_cus)) return gemm_split_bytes(M, K);
-    const uint32_t s = linear_plan(M, N, K, dtype, num_cus).splits;
-    return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+    return linear_choice(M, N, K, dtype, num_cus, true, SIZE_MAX).scratch;
+}
+
+bool linear_scratch_required(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus) {
+    const LinChoice c = linear_choice(M, N, K, dtype, num_cus, true, SIZE_MAX);
+    return c.scratch > 0 && c.route != LinRoute::kRows;
 }
 
 // y = 0 for calls with no inputs per output (K = 0): the sum over an empty
@@ -831,7 +945,7 @@ __global__ __launch_bounds__(256) void linear_zero_kernel(float *y, uint64_t cou
 
 hipError_t launch_linear(hipStream_t stream, const float *x, const void *w, uint32_t dtype,
                          float *y, uint32_t M, uint32_t N, uint32_t K, float *scratch,
-                         int num_cus) {
+                         size_t scratch_bytes, int num_cus) {
     if (M == 0 || N == 0) return hipSuccess;
     if (K == 0) {
         const uint64_t count = (uint64_t)M * N;
@@ -848,60 +962,83 @@ hipError_t launch_linear(hipStream_t stream, const float *x, const void *w, uint
         for (uint32_t r0 = 0; r0 < M; r0 += per) {
             const uint32_t m = std::min(per, M - r0);
             const hipError_t e = launch_linear(stream, x + (size_t)r0 * K, w, dtype,
-                                               y + (size_t)r0 * N, m, N, K, nullptr, num_cus);
+                                               y + (size_t)r0 * N, m, N, K, nullptr, 0, num_cus);
             if (e != hipSuccess) return e;
         }
         return hipSuccess;
     }
-    if (scratch != nullptr && gemm_applies(M, N, K, dtype, num_cus)) {
-        // x split once into scratch, then the tiled product; its two x
-        // stages take 96 KB of LDS, above the default limit
-        static const hipError_t configured = hipFuncSetAttribute(
-            (const void *)linear_gemm_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-            2 * kGemmStageBytes);
-        if (configured != hipSuccess) return configured;
+    const bool x_aligned = ((uintptr_t)x & 15u) == 0;
+    const LinChoice choice = linear_choice(M, N, K, dtype, num_cus, x_aligned,
+                                           scratch != nullptr ? scratch_bytes : 0);
+    if (choice.scratch > 0 && (scratch == nullptr || choice.scratch > scratch_bytes)) {
+        return hipErrorInvalidValue;
+    }
+    if (choice.route == LinRoute::kWide) {
+        // x split once into scratch, then the tiled product
         uint16_t *xs = (uint16_t *)scratch;
         const uint64_t chunks = (uint64_t)((M + kLinTile - 1) / kLinTile) * (K / kLinBlock) * 64;
         const dim3 sgrid((uint32_t)((chunks + 255) / 256));
-        if (((uintptr_t)x & 15u) == 0) {
+        if (x_aligned) {
             SR_LAUNCH("linear_split_x_kernel", linear_split_x_kernel<true>, sgrid, dim3(256), 0,
                       stream, x, xs, M, K, chunks);
         } else {
             SR_LAUNCH("linear_split_x_kernel", linear_split_x_kernel<false>, sgrid, dim3(256), 0,
                       stream, x, xs, M, K, chunks);
         }
-        const uint64_t wide_tiles =
-            (uint64_t)((M + kWideBM - 1) / kWideBM) * ((N + kWideBN - 1) / kWideBN);
-        if (N >= kWideMinOutputs && 2 * wide_tiles >= (uint64_t)(num_cus > 0 ? num_cus : 1)) {
-            const dim3 grid((N + kWideBN - 1) / kWideBN, (M + kWideBM - 1) / kWideBM);
-            SR_LAUNCH("linear_gemm_wide_kernel", linear_gemm_wide_kernel, grid, dim3(kWideThreads),
-                      2 * kWideStageBytes, stream, xs, w, y, M, N, K);
-            return hipGetLastError();
-        }
-        const dim3 grid((N + kGemmBN - 1) / kGemmBN, (M + kGemmBM - 1) / kGemmBM);
-        SR_LAUNCH("linear_gemm_kernel", linear_gemm_kernel, grid, dim3(64 * kGemmWM * kGemmWN),
-                  2 * kGemmStageBytes, stream, xs, w, y, M, N, K);
+        const dim3 grid((N + kWideBN - 1) / kWideBN, (M + kWideBM - 1) / kWideBM);
+        SR_LAUNCH("linear_gemm_wide_kernel", linear_gemm_wide_kernel, grid, dim3(kWideThreads),
+                  2 * kWideStageBytes, stream, xs, w, y, M, N, K);
         return hipGetLastError();
     }
-    const LinPlan plan = linear_plan(M, N, K, dtype, num_cus);
-    const uint32_t splits = plan.splits;
-    if (splits > 1 && scratch == nullptr) return hipErrorInvalidValue;
+    const uint32_t splits = choice.splits;
     float *dst = splits > 1 ? scratch : y;
-    switch (dtype) {
-        case SAFETYRAISE_KERNEL_DTYPE_F32:
-            launch_dt_plan<SAFETYRAISE_KERNEL_DTYPE_F32>(stream, x, w, dst, M, N, K, plan, num_cus);
-            break;
-        case SAFETYRAISE_KERNEL_DTYPE_F16:
-            launch_dt_plan<SAFETYRAISE_KERNEL_DTYPE_F16>(stream, x, w, dst, M, N, K, plan, num_cus);
-            break;
-        case SAFETYRAISE_KERNEL_DTYPE_BF16:
-            launch_dt_plan<SAFETYRAISE_KERNEL_DTYPE_BF16>(stream, x, w, dst, M, N, K, plan, num_cus);
-            break;
-        default:
-            return hipErrorInvalidValue;
+    if (choice.route == LinRoute::kRows) {
+        const bool pair = M <= 2 * kLinTile;
+        const uint32_t rows = pair ? 2 * kLinTile : 4 * kLinTile;
+        const dim3 grid((N + kRowsBN - 1) / kRowsBN, (M + rows - 1) / rows, splits);
+        const dim3 block(64 * kRowsWaves);
+        if (pair && x_aligned) {
+            SR_LAUNCH("linear_rows_kernel", (linear_rows_kernel<2, true>), grid, block, 0, stream, x, w,
+                      dst, M, N, K);
+        } else if (pair) {
+            SR_LAUNCH("linear_rows_kernel", (linear_rows_kernel<2, false>), grid, block, 0, stream, x,
+                      w, dst, M, N, K);
+        } else if (x_aligned) {
+            SR_LAUNCH("linear_rows_kernel", (linear_rows_kernel<4, true>), grid, block, 0, stream, x, w,
+                      dst, M, N, K);
+        } else {
+            SR_LAUNCH("linear_rows_kernel", (linear_rows_kernel<4, false>), grid, block, 0, stream, x,
+                      w, dst, M, N, K);
+        }
+    } else if (choice.route == LinRoute::kPair) {
+        const dim3 grid((N + 3 * kLinTile - 1) / (3 * kLinTile), 1);
+        constexpr int DT = SAFETYRAISE_KERNEL_DTYPE_BF16;
+        if (K % (kLinBlock * 16) == 0) {  // eight waves' ranges in whole pairs of blocks
+            SR_LAUNCH("linear_kernel_t3", (linear_kernel<DT, true, 3, 8, 1, true, 2>), grid, dim3(512), 0,
+                      stream, x, w, y, M, N, K);
+        } else {
+            SR_LAUNCH("linear_kernel_t3", (linear_kernel<DT, true, 3, 8, 1, false, 2>), grid, dim3(512),
+                      0, stream, x, w, y, M, N, K);
+        }
+    } else {
+        const LinPlan plan = linear_plan(M, N, K, dtype, num_cus);
+        switch (dtype) {
+            case SAFETYRAISE_KERNEL_DTYPE_F32:
+                launch_dt_plan<SAFETYRAISE_KERNEL_DTYPE_F32>(stream, x, w, dst, M, N, K, plan, num_cus);
+                break;
+            case SAFETYRAISE_KERNEL_DTYPE_F16:
+                launch_dt_plan<SAFETYRAISE_KERNEL_DTYPE_F16>(stream, x, w, dst, M, N, K, plan, num_cus);
+                break;
+            case SAFETYRAISE_KERNEL_DTYPE_BF16:
+                launch_dt_plan<SAFETYRAISE_KERNEL_DTYPE_BF16>(stream, x, w, dst, M, N, K, plan, num_cus);
+                break;
+            default:
+                return hipErrorInvalidValue;
+        }
     }
     if (splits > 1) {
-        // splits > 1 only when the tiles do not cover the CUs, so M * N is small
+        // (M * N fits 32 bits: kTile splits only when its tiles do not cover
+        // the CUs, kRows checks it)
         const uint32_t count = M * N;
         SR_LAUNCH("linear_split_sum_kernel", linear_split_sum_kernel, dim3((count + 255) / 256),
                   dim3(256), 0, stream, scratch, y, count, splits);

@@ -369,16 +369,32 @@ static int32_t check_linear(Ctx *ctx, const safetyraise_kernel_weight *w, const 
     return kOk;
 }
 
-// The partial-sum buffer of a call that splits K (nullptr when it does not).
+// The context's linear scratch for a call (none: nullptr and 0 bytes).  A call
+// that can do without (linear_scratch_required) goes without when the buffer
+// cannot grow, and while the stream is captured: a graph would keep the
+// buffer's address, and a later, larger call replaces the buffer.
 static int32_t linear_scratch(Ctx *ctx, const safetyraise_kernel_weight *w, uint64_t rows,
-                              float **part) {
-    const size_t bytes = linear_scratch_bytes((uint32_t)rows, (uint32_t)w->rows,
-                                              (uint32_t)w->cols, w->dtype, ctx->num_cus);
+                              float **part, size_t *have) {
+    const uint32_t m = (uint32_t)rows, n = (uint32_t)w->rows, k = (uint32_t)w->cols;
+    const size_t bytes = linear_scratch_bytes(m, n, k, w->dtype, ctx->num_cus);
     *part = nullptr;
+    *have = 0;
     if (bytes == 0) return kOk;
+    const bool required = linear_scratch_required(m, n, k, w->dtype, ctx->num_cus);
+    if (!required) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess) (void)hipGetLastError();
+        if (capture != hipStreamCaptureStatusNone) return kOk;
+    }
     const int32_t e = ensure_buffer(ctx, ctx->linear_part, bytes, false);
+    if (e == kNoMemory && !required) {
+        (void)hipGetLastError();
+        ctx->error.clear();
+        return kOk;
+    }
     if (e != kOk) return e;
     *part = (float *)ctx->linear_part.ptr;
+    *have = bytes;
     return kOk;
 }
 }  // namespace sr
@@ -408,7 +424,8 @@ SAFETYRAISE_KERNEL_EXPORT int32_t safetyraise_kernel_linear(
     e = ensure_buffer(context, context->linear_out, (size_t)out_count * 4, false);
     if (e != kOk) return e;
     float *part = nullptr;
-    e = linear_scratch(context, weight, input_rows, &part);
+    size_t part_bytes = 0;
+    e = linear_scratch(context, weight, input_rows, &part, &part_bytes);
     if (e != kOk) return e;
     float *d_in = (float *)context->linear_in.ptr;
     float *d_out = (float *)context->linear_out.ptr;
@@ -418,7 +435,8 @@ SAFETYRAISE_KERNEL_EXPORT int32_t safetyraise_kernel_linear(
     }
     SR_HIP(context, launch_linear(context->stream, d_in, weight->d_data, weight->dtype, d_out,
                                   (uint32_t)input_rows, (uint32_t)weight->rows,
-                                  (uint32_t)weight->cols, part, context->num_cus));
+                                  (uint32_t)weight->cols, part, part_bytes,
+                                  context->num_cus));
     SR_HIP(context, hipMemcpyAsync(output, d_out, out_count * 4, hipMemcpyDeviceToHost,
                                    context->stream));
     SR_HIP(context, hipStreamSynchronize(context->stream));
@@ -439,11 +457,13 @@ SAFETYRAISE_KERNEL_EXPORT int32_t safetyraise_kernel_linear_device(
     if (st != kOk) return st;
     if (out_count == 0) return kOk;
     float *part = nullptr;
-    const int32_t e = linear_scratch(context, weight, input_rows, &part);
+    size_t part_bytes = 0;
+    const int32_t e = linear_scratch(context, weight, input_rows, &part, &part_bytes);
     if (e != kOk) return e;
     SR_HIP(context, launch_linear(context->stream, input, weight->d_data, weight->dtype, output,
                                   (uint32_t)input_rows, (uint32_t)weight->rows,
-                                  (uint32_t)weight->cols, part, context->num_cus));
+                                  (uint32_t)weight->cols, part, part_bytes,
+                                  context->num_cus));
     return kOk;
 }
 

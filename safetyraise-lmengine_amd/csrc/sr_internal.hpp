@@ -362,9 +362,11 @@ struct GdnRollback {
 hipError_t launch_gdn_rollback(hipStream_t stream, const GdnRollback &r);
 
 // y[M][N] = x[M][K] . W[N][K]^T with f32 products, W of dtype F32/F16/BF16
-// (linear_kernels.hip).  scratch holds linear_scratch_bytes(...) bytes of
-// partial sums (none when that is 0) for calls that split K.
+// (linear_kernels.hip).  linear_scratch_bytes: the scratch a call likes (split
+// x, or partial sums of calls that split K); unless linear_scratch_required(),
+// a call without it takes a route that needs none.
 size_t linear_scratch_bytes(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus);
+bool linear_scratch_required(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus);
 // Device bytes of a [rows][cols] weight as the kernels read it: row-major for
 // F32 and F16, whole 1 KB tiles for BF16 (SIZE_MAX when that overflows).
 size_t linear_weight_bytes(uint64_t rows, uint64_t cols, uint32_t dtype);
@@ -373,7 +375,7 @@ hipError_t linear_pack_bf16(hipStream_t stream, const void *src, void *dst, uint
                             uint64_t cols);
 hipError_t launch_linear(hipStream_t stream, const float *x, const void *w, uint32_t dtype,
                          float *y, uint32_t M, uint32_t N, uint32_t K, float *scratch,
-                         int num_cus);
+                         size_t scratch_bytes, int num_cus);
 
 // Conv + delta rule over every row of every sequence, then RMSNorm * silu(z).
 // Calls that take the chunked form need g.chunk_rec with

@@ -317,3 +317,86 @@ def test_inputs_above_the_bf16_range(backend, rng, torch_mod, rows, cols, out):
             assert not bad.any(), (rows, np.abs(got - ref).max())
     finally:
         prepared.destroy()
+
+
+# bf16 calls of more than 16 rows: (rows, cols, out) at the edges of each route
+# (linear_choice in linear_kernels.hip): 32 rows per workgroup with whole and
+# ragged k ranges; 32- and 64-row workgroups with and without a K split, row
+# and output counts on and off the tiles; the tiled product
+ROUTES = [(17, 512, 10800), (32, 520, 10753), (17, 12288, 1027), (32, 4096, 4099), (33, 4096, 4099),
+          (64, 12352, 1030), (65, 4160, 1111), (100, 2112, 1500), (129, 2048, 1140),
+          (300, 960, 3000), (1000, 64, 7100), (130, 128, 28700)]
+
+
+def device_call(backend, prepared, x, dy, rows, cols, out):
+    backend.check(backend.lib.safetyraise_kernel_linear_device(
+        backend.context, prepared.handle, C.c_void_p(x.data_ptr()), rows, cols,
+        C.c_void_p(dy.data_ptr()), rows, out), "linear_device")
+
+
+@pytest.mark.parametrize("rows,cols,out", ROUTES)
+def test_routes_of_many_rows(backend, rng, torch_mod, rows, cols, out):
+    # random inputs at the reordered-sum bound, from a 16-byte aligned and an
+    # unaligned x, and integer inputs bit for bit
+    torch = torch_mod
+    for integers in (False, True):
+        if integers:
+            x = rng.integers(-8, 9, size=(rows, cols)).astype(np.float32)
+            w = rng.integers(-8, 9, size=(out, cols)).astype(np.float32)
+        else:
+            x = (2 * rng.standard_normal((rows, cols))).astype(np.float32)
+            w = rng.standard_normal((out, cols)).astype(np.float32)
+        bits = weight_bits(w, BF16)
+        wide = torch.from_numpy(widened(bits, BF16)).cuda()
+        x64 = torch.from_numpy(x).cuda().double()
+        ref = x64 @ wide.T
+        bound = 1e-5 * (x64.abs() @ wide.abs().T) + 1e-4 * ref.abs()
+        prepared = backend.create_weight(bits, BF16)
+        try:
+            for shift in (0, 1):
+                buf = torch.zeros(rows * cols + 1, device="cuda")
+                buf[shift:shift + rows * cols] = torch.from_numpy(x).cuda().flatten()
+                dy = torch.full((rows, out), float("nan"), device="cuda")
+                torch.cuda.synchronize()
+                device_call(backend, prepared, buf[shift:], dy, rows, cols, out)
+                backend.synchronize()
+                if integers:
+                    assert torch.equal(dy.double(), ref), (rows, cols, out, shift)
+                else:
+                    assert bool(((dy.double() - ref).abs() <= bound).all()), (rows, cols, out, shift)
+        finally:
+            prepared.destroy()
+
+
+def test_captured_call_keeps_no_scratch(backend, rng, torch_mod):
+    # a call whose K split is optional is captured without it: its replays
+    # stay right after a larger call has replaced the context's scratch
+    torch = torch_mod
+    rows, cols, out = 64, 4096, 4096
+    bits = weight_bits(rng.integers(-8, 9, size=(out, cols)).astype(np.float32), BF16)
+    prepared = backend.create_weight(bits, BF16)
+    x = torch.zeros((rows, cols), device="cuda")
+    dy = torch.zeros((rows, out), device="cuda")
+    big = torch.zeros((4096, cols), device="cuda")
+    by = torch.zeros((4096, out), device="cuda")
+    wide = torch.from_numpy(widened(bits, BF16)).cuda()
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    backend.set_stream(stream.cuda_stream)
+    try:
+        device_call(backend, prepared, x, dy, rows, cols, out)
+        backend.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            device_call(backend, prepared, x, dy, rows, cols, out)
+        for _ in range(3):
+            x.copy_(torch.from_numpy(rng.integers(-8, 9, size=(rows, cols)).astype(np.float32)))
+            dy.fill_(float("nan"))
+            device_call(backend, prepared, big, by, 4096, cols, out)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(dy.double(), x.double() @ wide.T)
+    finally:
+        backend.set_stream(None)
+        prepared.destroy()

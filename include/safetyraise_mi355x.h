@@ -185,7 +185,8 @@ SAFETYRAISE_KERNEL_EXPORT int32_t safetyraise_kernel_kv_read(
  * verify drafts) to the multi-row split-K verify kernel (every cached K/V
  * tile read once for up to 128 query vectors, rows * heads/kv_heads, at
  * head_dim <= 128 and 64 at head_dim 256; more rows run as row slices, each
- * reading the cache once); 16 or more rows to the MFMA prefill kernels.
+ * reading the cache once); 16 or more rows to the MFMA prefill kernels, or to
+ * the split-K ones where the row blocks alone would leave most CUs idle.
  * Query-head groups other than 1..8 heads per KV head and RoPE widths not a
  * multiple of 32 go row by row to the decode kernel.  Head widths other than
  * 64, 128 and 256 (up to 512) take plain f32 kernels for every row: all rows

@@ -49,6 +49,9 @@ void *grow_rope(void *user, size_t bytes) {
     return ctx->rope_scratch.ptr;
 }
 
+// most scratch that prefill rows take for the split-K form's records
+constexpr uint64_t kSplitRecordBytes = 256ull << 20;
+
 // One launch of the decode kernels over up to kMetaPerLaunch sequences, each
 // contributing the row `row0` at cache length `ctx`.
 int32_t run_decode_pack(Ctx *ctx, const AttnLaunch &a, const std::vector<SeqMeta> &pack,
@@ -65,14 +68,13 @@ int32_t run_decode_pack(Ctx *ctx, const AttnLaunch &a, const std::vector<SeqMeta
 // The first pack launched carries the call's inline page-table entries
 // (AttnLaunch::tbl_*); they are cleared once a launch has taken them.
 int32_t run_verify_pack(Ctx *ctx, AttnLaunch &a, const std::vector<SeqMeta> &pack,
-                        const AttnScratch &scratch, void *rope) {
+                        const AttnScratch &scratch, void *rope, uint64_t record_limit) {
     DecodePlanInput plan{ctx->num_cus, scratch.partials, scratch.user};
     const hipError_t e =
-        launch_attn_verify(ctx->stream, a, pack.data(), (int)pack.size(), rope, plan);
+        launch_attn_verify(ctx->stream, a, pack.data(), (int)pack.size(), rope, plan, record_limit);
+    if (e == hipErrorOutOfMemory) return kNoMemory;  // (nothing was launched)
     a.tbl_n = 0;
-    if (e != hipSuccess) {
-        return e == hipErrorOutOfMemory ? kNoMemory : hip_fail(ctx, e, "verify attention launch");
-    }
+    if (e != hipSuccess) return hip_fail(ctx, e, "verify attention launch");
     return kOk;
 }
 
@@ -338,57 +340,72 @@ int32_t attention_forward_impl(Ctx *ctx, const safetyraise_kernel_attention_args
         rope = scratch.rope(scratch.user, prefill_rope_bytes(L, total_rows));
         if (rope == nullptr) return kNoMemory;
     }
+    auto meta = [&](uint32_t i) {
+        SeqMeta m{};
+        m.slot = A.seq_ids[i];
+        m.ctx = (uint32_t)old_len[i];
+        m.rows = A.seq_rows[i];
+        m.row0 = (uint32_t)row0[i];
+        return m;
+    };
+    // every sequence that `which` selects, in packs of one launch each
+    auto run_packs = [&](auto which, auto run) -> int32_t {
+        std::vector<SeqMeta> pack;
+        for (uint32_t i = 0; i < A.num_seqs; ++i) {
+            if (!which(i)) continue;
+            serial[i] = 0;
+            any_prefill = true;
+            pack.push_back(meta(i));
+            if (pack.size() == (size_t)kMetaPerLaunch) {
+                const int32_t st = run(pack);
+                if (st != kOk) return st;
+                pack.clear();
+            }
+        }
+        return pack.empty() ? kOk : run(pack);
+    };
     // Sequences with 2..15 rows (MTP verify drafts) take the multi-row
     // split-K kernel: every cached K/V tile is read once for all rows.
-    {
-        std::vector<SeqMeta> pack;
-        for (uint32_t i = 0; i < A.num_seqs; ++i) {
-            if (A.seq_rows[i] >= kPrefillMinRows || !verify_supported(L, A.seq_rows[i])) continue;
-            serial[i] = 0;
-            any_prefill = true;
-            SeqMeta m{};
-            m.slot = A.seq_ids[i];
-            m.ctx = (uint32_t)old_len[i];
-            m.rows = A.seq_rows[i];
-            m.row0 = (uint32_t)row0[i];
-            pack.push_back(m);
-            if (pack.size() == (size_t)kMetaPerLaunch) {
-                int32_t st = run_verify_pack(ctx, L, pack, scratch, rope);
-                if (st != kOk) return st;
-                pack.clear();
-            }
+    int32_t pst = run_packs(
+        [&](uint32_t i) {
+            return A.seq_rows[i] < kPrefillMinRows && verify_supported(L, A.seq_rows[i]);
+        },
+        [&](const std::vector<SeqMeta> &pack) {
+            return run_verify_pack(ctx, L, pack, scratch, rope, UINT64_MAX);
+        });
+    if (pst != kOk) return pst;
+    // Prefill rows whose row blocks would leave most of the CUs idle take it
+    // too, or the prefill kernels if there is no memory for its records or
+    // they are many (rows by the thousand over pages of a few tokens).
+    std::vector<SeqMeta> candidates;
+    std::vector<uint8_t> split(A.num_seqs, 0);
+    for (uint32_t i = 0; prefill_ok && i < A.num_seqs; ++i) {
+        if (A.seq_rows[i] < kPrefillMinRows || !split_candidate(L, (uint32_t)old_len[i], A.seq_rows[i])) {
+            continue;
         }
-        if (!pack.empty()) {
-            int32_t st = run_verify_pack(ctx, L, pack, scratch, rope);
-            if (st != kOk) return st;
-        }
+        split[i] = 1;
+        candidates.push_back(meta(i));
     }
-    {
-        std::vector<SeqMeta> pack;
-        for (uint32_t i = 0; i < A.num_seqs; ++i) {
-            if (!serial[i]) continue;
-            if (!prefill_ok || A.seq_rows[i] < kPrefillMinRows) {
-                serial_rows = std::max(serial_rows, A.seq_rows[i]);
-                continue;
-            }
-            serial[i] = 0;
-            any_prefill = true;
-            SeqMeta m{};
-            m.slot = A.seq_ids[i];
-            m.ctx = (uint32_t)old_len[i];
-            m.rows = A.seq_rows[i];
-            m.row0 = (uint32_t)row0[i];
-            pack.push_back(m);
-            if (pack.size() == (size_t)kMetaPerLaunch) {
-                int32_t st = run_prefill_pack(ctx, L, pack, rope);
-                if (st != kOk) return st;
-                pack.clear();
-            }
-        }
-        if (!pack.empty()) {
-            int32_t st = run_prefill_pack(ctx, L, pack, rope);
-            if (st != kOk) return st;
-        }
+    const bool preferred =
+        split_preferred(L, candidates.data(), (int)candidates.size(), ctx->num_cus);
+    pst = run_packs([&](uint32_t i) { return preferred && split[i]; },
+                    [&](const std::vector<SeqMeta> &pack) {
+                        const int32_t st =
+                            run_verify_pack(ctx, L, pack, scratch, rope, kSplitRecordBytes);
+                        if (st != kNoMemory) return st;
+                        (void)hipGetLastError();
+                        ctx->error.clear();
+                        return run_prefill_pack(ctx, L, pack, rope);
+                    });
+    if (pst != kOk) return pst;
+    pst = run_packs(
+        [&](uint32_t i) {
+            return prefill_ok && A.seq_rows[i] >= kPrefillMinRows && !(preferred && split[i]);
+        },
+        [&](const std::vector<SeqMeta> &pack) { return run_prefill_pack(ctx, L, pack, rope); });
+    if (pst != kOk) return pst;
+    for (uint32_t i = 0; i < A.num_seqs; ++i) {
+        if (serial[i]) serial_rows = std::max(serial_rows, A.seq_rows[i]);
     }
 
     // Row r of every selected sequence with more than r rows: one decode step

@@ -38,6 +38,7 @@
 // non-finite; the row is then flagged (kErrPrefillRange) for the host, which
 // recomputes the call on the f32 split-K path.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "sr_device.hpp"
@@ -1330,36 +1331,51 @@ __device__ __forceinline__ void softmax_tile_ref(f32x16 (&sacc)[2], uint32_t key
     l_run += lt;
 }
 
-// o / l, Qwen3.5 gate (math.rs sigmoid), f32 store; flags non-finite rows.
-template <int D>
-__device__ __forceinline__ void store_rows(const PrefillParams &p, uint32_t call_row, uint32_t head,
-                                           size_t qbase, int h, float l_run,
-                                           const f32x16 (&oacc)[D / 32]) {
-    constexpr int NT = D / 32;
+// Four consecutive activations from element i on (i a multiple of 4, the
+// tensor 16-byte aligned), widened to f32.
+__device__ __forceinline__ f32x4 load_act4(const void *p, size_t i, bool bf16) {
+    if (bf16) {
+        const uint2 w = *(const uint2 *)((const uint16_t *)p + i);
+        return f32x4{bf16lo(w.x), bf16hi(w.x), bf16lo(w.y), bf16hi(w.y)};
+    }
+    return *(const f32x4 *)((const float *)p + i);
+}
+
+// o / l, Qwen3.5 gate (math.rs sigmoid), f32 store of dims dim0 .. of a head of
+// `dims`; flags non-finite rows.  The gates of a 32-dim tile are requested
+// together, 16 bytes per load.
+template <int NT>
+__device__ __forceinline__ void store_dims(const PrefillParams &p, uint32_t call_row, uint32_t head,
+                                           size_t qbase, uint32_t dims, uint32_t dim0, int h,
+                                           float l_run, const f32x16 (&oacc)[NT]) {
     const bool bf16_in = (p.flags & SAFETYRAISE_MI355X_INPUT_BF16) != 0;
     const bool gated = (p.flags & SAFETYRAISE_MI355X_GATED) != 0;
     const float inv_l = 1.0f / l_run;
-    float *dst = p.out + (size_t)call_row * p.heads * D + (size_t)head * D;
+    float *dst = p.out + (size_t)call_row * p.heads * dims + (size_t)head * dims;
     bool finite = true;
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt) {
+        f32x4 o[4];
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
-            const uint32_t d0 = 32 * tt + 8 * a + 4 * h;
-            float o[4];
 #pragma unroll
             for (int bb = 0; bb < 4; ++bb) {
-                o[bb] = oacc[tt][4 * a + bb] * inv_l;
-                finite = finite && isfinite(o[bb]);
+                o[a][bb] = oacc[tt][4 * a + bb] * inv_l;
+                finite = finite && isfinite(o[a][bb]);
             }
-            if (gated) {
-#pragma unroll
-                for (int bb = 0; bb < 4; ++bb) {
-                    o[bb] *= ref_sigmoid(load_act(p.q, qbase + D + d0 + bb, bf16_in));
-                }
-            }
-            __builtin_nontemporal_store(f32x4{o[0], o[1], o[2], o[3]}, (f32x4 *)(dst + d0));
         }
+        const uint32_t d0 = dim0 + 32 * tt + 4 * h;
+        if (gated) {
+            f32x4 gate[4];
+#pragma unroll
+            for (int a = 0; a < 4; ++a) gate[a] = load_act4(p.q, qbase + dims + d0 + 8 * a, bf16_in);
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+#pragma unroll
+                for (int bb = 0; bb < 4; ++bb) o[a][bb] *= ref_sigmoid(gate[a][bb]);
+        }
+#pragma unroll
+        for (int a = 0; a < 4; ++a) __builtin_nontemporal_store(o[a], (f32x4 *)(dst + d0 + 8 * a));
     }
     if (!finite) atomicOr(p.err_word, kErrPrefillRange);
 }
@@ -1409,9 +1425,10 @@ __device__ __forceinline__ void store_rows_lds(const PrefillParams &p, uint32_t 
             if (r < valid) {
                 const size_t row = (size_t)(call_row0 + r);
                 if (gated) {
-                    const size_t gbase = row * p.heads * hs + (size_t)head * hs + D + d0;
+                    const f32x4 gate =
+                        load_act4(p.q, row * p.heads * hs + (size_t)head * hs + D + d0, bf16_in);
 #pragma unroll
-                    for (int bb = 0; bb < 4; ++bb) o[bb] *= ref_sigmoid(load_act(p.q, gbase + bb, bf16_in));
+                    for (int bb = 0; bb < 4; ++bb) o[bb] *= ref_sigmoid(gate[bb]);
                 }
                 __builtin_nontemporal_store(o, (f32x4 *)(p.out + row * p.heads * D + (size_t)head * D + d0));
             }
@@ -1502,7 +1519,7 @@ __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1))) void attn_prefill_kernel(
     }
     const uint32_t row = wrow0 + col;
     const float l = xhalf_sum(l_run);
-    if (row < b.m.rows) store_rows<D>(p, b.m.row0 + row, head, qbase, h, l, oacc);
+    if (row < b.m.rows) store_dims<NT>(p, b.m.row0 + row, head, qbase, D, 0, h, l, oacc);
 }
 
 // ---------------------------------------------------------------------------
@@ -2318,21 +2335,28 @@ hipError_t launch_d(hipStream_t stream, PrefillParams &p, uint32_t g, const SeqM
 // workgroup per (partition, KV head) runs the online softmax over its keys
 // and leaves a (max, sum, o[D]) record per query vector, which
 // attn_verify_combine_kernel merges (math.rs:133-152 split over the keys).
-// A workgroup holds at most 64 query vectors (two consumer waves of 32):
-// with more (e.g. 1 + 8 drafts at G = 8), the rows are cut into slices of
-// floor(64 / G) rows, one workgroup per (partition, KV head, slice); the
-// slices of a partition are dispatched to one XCD at about the same time,
-// so the second reads the partition's pages largely from its L2 and the
-// Infinity Cache.  Each (row, head) record is written by one slice.
+// A workgroup holds at most 64 query vectors (two consumer waves of 32), 128
+// in the all-tiles form: with more (e.g. 1 + 8 drafts at G = 8), the rows are
+// cut into slices, one workgroup per (partition, KV head, slice) over the keys
+// that the slice's rows see; the slices of a partition are dispatched to one
+// XCD at about the same time, so the second reads the partition's pages
+// largely from its L2 and the Infinity Cache.  Each (row, head) record is
+// written by one slice.
+//
+// Every block of the grid has work.  A workgroup fills its CU, and workgroups
+// go to the shader engines of an XCD in turn and in order: blocks of a regular
+// (unit, slice) grid that leave at once still take their turn, and every other
+// one being empty (the second slice of sequences that have one) left half of
+// the engines idle while the next block waited for a full one.  4 sequences of
+// 40 K to 131 K keys with 2 to 9 rows (16 / 2 x 256): 214 to 134 us.
 // ---------------------------------------------------------------------------
 struct VerifyParams {
     PrefillParams p;       // meta[s].nblk = records per (row, head) of sequence s
     float *partials;       // records of kRecordStride floats
     uint32_t part_keys;
-    uint32_t units;           // (partition, KV head) pairs of the launch
-    uint32_t slices;          // row slices per unit (each <= 64 query vectors)
-    uint32_t rows_per_slice;  // floor(64 / G)
-    uint32_t blk0[kMetaPerLaunch];  // first partition of each sequence (prefix)
+    uint32_t rows_per_slice;  // floor(64 / G), all-tiles form floor(128 / G)
+    uint32_t direct;          // every (row, head) has one record: no combine pass
+    uint32_t blk0[kMetaPerLaunch];  // first workgroup of each sequence (prefix)
     uint32_t rec0[kMetaPerLaunch];  // first record of each sequence
 };
 static_assert(sizeof(VerifyParams) <= 4096, "kernel arguments stay within 4 KiB");
@@ -2380,7 +2404,7 @@ struct VerifyIo {
                                          uint32_t gt) const {
         const uint32_t ch = gt % KCH, k0 = gt / KCH;
         const uint32_t key0 = t * kKeyTile;
-        // keys past the sequence's last are masked: they read its last row.
+        // keys past the range's last are masked: they read its last row.
         // A 4-key V group never straddles a page, and neither does its clamp.
         uint32_t tk[KL], tv[VL], pk[KL], pv[VL];
 #pragma unroll
@@ -2420,7 +2444,7 @@ struct VerifyIo {
                 }
         }
     }
-    // Keys past the sequence's last were loaded as copies of its last row
+    // Keys past the range's last were loaded as copies of its last row
     // (load clamps them), so their V rows are finite and need no zeroing: the
     // consumers mask their scores, and P = 0 times a finite value adds 0.
     __device__ __forceinline__ void store(const u32x4 (&kr)[KL], const u32x4 (&vr)[4 * VL],
@@ -2492,7 +2516,7 @@ constexpr size_t kVerifyTileLds = 2 * kVerifyTilesPerStep<D> * 2 * kTileBytes<D>
 // kAllTiles (D <= 128 only): each of the four consumer waves takes 32 query
 // vectors and both tiles of every step (up to 128 vectors per workgroup, one
 // record per partition), for calls with more than 64 vectors per KV head.
-template <int D, bool kAllTiles, bool kShared>
+template <int D, bool kAllTiles>
 __global__ __launch_bounds__(kVerifyThreads) __attribute__((amdgpu_waves_per_eu(2))) void
 attn_verify_kernel(const VerifyParams vp) {
     static_assert(!kAllTiles || D <= 128, "D = 256 splits the output dims instead");
@@ -2507,25 +2531,40 @@ attn_verify_kernel(const VerifyParams vp) {
     const int tid = threadIdx.x;
     const int wave = wave_index();
     const int lane = tid & 63;
-    // block -> (unit, slice): the slices of a unit are 8 blocks apart, so
-    // they land on the same XCD (block i runs on XCD i % 8) at about the
-    // same time; blocks past the last unit leave at once (whole workgroup)
-    const uint32_t grp8 = blockIdx.x / (8 * vp.slices);
-    const uint32_t slice = (blockIdx.x / 8) % vp.slices;
-    const uint32_t unit = grp8 * 8 + blockIdx.x % 8;
-    if (unit >= vp.units) return;
-    const uint32_t kvh = unit % p.kv_heads;
-    const uint32_t j = unit / p.kv_heads;
+    // block -> (sequence, unit, slice), a unit being a (partition, KV head):
+    // groups of 8 units, each group's slices 8 blocks apart, so that they land
+    // on the same XCD (block i runs on XCD i % 8) at about the same time, the
+    // slices with the most visible keys first.  A sequence's last group may be
+    // narrower.
     uint32_t s = 0;
-    while (s + 1 < p.nseq && vp.blk0[s + 1] <= j) ++s;
+    while (s + 1 < p.nseq && vp.blk0[s + 1] <= blockIdx.x) ++s;
     const PrefillMeta m = p.meta[s];
+    const uint32_t slices = (m.rows + vp.rows_per_slice - 1) / vp.rows_per_slice;
+    const uint32_t units = m.nblk / kRecPerPart * p.kv_heads;
+    const uint32_t at = blockIdx.x - vp.blk0[s];
+    const uint32_t unit0 = at / (8 * slices) * 8;
+    const uint32_t width = min(8u, units - unit0);
+    const uint32_t unit = unit0 + (at - unit0 * slices) % width;
+    const uint32_t slice = slices - 1 - (at - unit0 * slices) / width;
+    const uint32_t kvh = unit % p.kv_heads;
     const uint32_t row_begin = slice * vp.rows_per_slice;
-    if (row_begin >= m.rows) return;  // this sequence has fewer slices (whole workgroup)
     const QArgs qa = q_args(p);
-    const uint32_t part = j - vp.blk0[s];
-    const uint32_t total = m.ctx + m.rows;
+    const uint32_t part = unit / p.kv_heads;
+    const uint32_t slice_rows = min(vp.rows_per_slice, m.rows - row_begin);
+    // the partition's keys that the slice's last row sees (none: the slice
+    // leaves empty records)
     const uint32_t key_begin = part * vp.part_keys;
-    const uint32_t key_end = min(key_begin + vp.part_keys, total);
+    const uint32_t key_end = min(key_begin + vp.part_keys, m.ctx + row_begin + slice_rows);
+    const uint32_t G = p.heads / p.kv_heads;
+    if (key_begin >= key_end) {
+        for (uint32_t v = tid; v < slice_rows * G * kRecPerPart; v += kVerifyThreads) {
+            const uint32_t q = v % kRecPerPart, vec = v / kRecPerPart;
+            const size_t at = vp.rec0[s] + ((size_t)(row_begin + vec / G) * p.heads + kvh * G + vec % G) * m.nblk;
+            *(float2 *)(vp.partials + (at + kRecPerPart * part + q) * kRecordStride<D>) =
+                make_float2(-INFINITY, 0.0f);
+        }
+        return;
+    }
     const uint32_t t0 = key_begin / kKeyTile;
     const uint32_t t1 = (key_end + kKeyTile - 1) / kKeyTile;
     // both roles run the same padded number of steps (one barrier each)
@@ -2536,8 +2575,9 @@ attn_verify_kernel(const VerifyParams vp) {
         return lds + ((k & 1) * TPS + q) * 2 * kTileBytes<D>;
     };
 
-    if (wave >= 4) {
-        // ---- producers ----
+    // ---- producers ----
+    auto produce = [&](auto shared) __attribute__((always_inline)) {
+        constexpr bool kShared = decltype(shared)::value;
         const uint32_t pt = tid - 256;                 // 0..255
         const uint32_t q = TPS == 2 ? pt >> 7 : 0u;    // which tile of the step
         const uint32_t gt0 = TPS == 2 ? pt & 127 : pt;
@@ -2548,7 +2588,9 @@ attn_verify_kernel(const VerifyParams vp) {
         const size_t head_bytes = (size_t)(kvh / p.kv_rep) * p.num_pages * io.page_bytes;
         io.k_head = (const unsigned char *)p.k_pages + head_bytes;
         io.v_head = (const unsigned char *)p.v_pages + head_bytes;
-        io.last_tok = total - 1;
+        // (keys of the last tile past the slice's range may be on pages whose ids
+        // are not in LDS: the loads stop at the range's last key)
+        io.last_tok = key_end - 1;
         // the page ids of the partition's keys go to LDS once, so that no
         // tile load waits on a page-table read
         int32_t *pids = (int32_t *)(lds + kVerifyTileLds<D>);
@@ -2593,6 +2635,12 @@ attn_verify_kernel(const VerifyParams vp) {
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+    };
+    if (wave >= 4) {
+        // a sequence of more rows than a slice holds has sibling slices that
+        // read the same tiles
+        if (m.rows > vp.rows_per_slice) produce(std::true_type{});
+        else produce(std::false_type{});
         return;
     }
 
@@ -2603,8 +2651,7 @@ attn_verify_kernel(const VerifyParams vp) {
     const int cw = kAllTiles ? wave : (wave & 1);
     const int h = lane >> 5;
     const int col = lane & 31;
-    const uint32_t G = p.heads / p.kv_heads;
-    const uint32_t nvec = min(vp.rows_per_slice, m.rows - row_begin) * G;
+    const uint32_t nvec = slice_rows * G;
     const bool computes = 32u * cw < nvec;               // wave-uniform
     const uint32_t vec = min(32u * cw + col, nvec - 1);  // this lane's query vector
     const uint32_t r = row_begin + vec / G;
@@ -2634,7 +2681,7 @@ attn_verify_kernel(const VerifyParams vp) {
         s_tile<D>(kt, qop, h, col, sacc);
         // keys past the partition end (the last tile of the sequence) and
         // past a row's own position are masked
-        const bool edge = key0 + kKeyTile > min(key_end, m.ctx + 1);
+        const bool edge = key0 + kKeyTile > min(key_end, m.ctx + row_begin + 1);
         if (edge) {
 #pragma unroll
             for (int u = 0; u < 2; ++u)
@@ -2666,6 +2713,11 @@ attn_verify_kernel(const VerifyParams vp) {
     }
     const float l = xhalf_sum(l_run);
     if (32u * cw + col >= nvec) return;
+    if (vp.direct) {
+        // one record per (row, head): it is the output
+        store_dims<NTW>(p, m.row0 + r, head, qbase, D, 128 * half, h, l, oacc);
+        return;
+    }
     // record (sequence s, row r, head, partition, pair): o unnormalised
     const uint32_t nrec = m.nblk;  // records per (row, head): kRecPerPart per partition
     float *rec = vp.partials + ((size_t)vp.rec0[s] + ((size_t)r * p.heads + head) * nrec +
@@ -2685,56 +2737,63 @@ attn_verify_kernel(const VerifyParams vp) {
         }
 }
 
-// One workgroup of four waves per (sequence, row, head): merges the
-// partition records in the log2 domain, divides by the sum, applies the
-// Qwen3.5 gate and stores.  Wave w takes records w, w + 4, ...; every record
-// load of a batch is in flight at once, and the four partial sums meet in LDS.
+// Merges the partition records of a (sequence, row, head) in the log2 domain,
+// divides by the sum, applies the Qwen3.5 gate and stores.  kEach = false: one
+// workgroup of four waves per (row, head); wave w takes records w, w + 4, ...,
+// every record load of a batch in flight at once, and the four partial sums
+// meet in LDS.  kEach = true (calls of many rows, with at most kCombineBatch
+// records each): one wave per (row, head), all its loads in flight, no LDS;
+// 512 rows x 32 heads 24 to 8.5 us.
 constexpr int kCombineWaves = 4;
+constexpr int kCombineBatch = 8;  // records per batch of loads
 
-template <int D>
+template <int D, bool kEach>
 __global__ __launch_bounds__(64 * kCombineWaves) void attn_verify_combine_kernel(const VerifyParams vp) {
     constexpr int EPL = D / 64;
-    constexpr int kUnroll = 8;  // records per batch of loads
+    constexpr int kUnroll = kCombineBatch;
+    constexpr uint32_t kStep = kEach ? 1 : kCombineWaves;  // records between a wave's own
     __shared__ float part_s[kCombineWaves][D + 1];
     __shared__ float max_s[kCombineWaves];
     const PrefillParams &p = vp.p;
-    const uint32_t w = blockIdx.x;
-    const int wave = threadIdx.x >> 6;
+    const int wave = wave_index();
     const int lane = threadIdx.x & 63;
+    const uint32_t w = kEach ? blockIdx.x * kCombineWaves + wave : blockIdx.x;
     uint32_t s = 0, base = 0;
     for (; s < p.nseq; ++s) {
         const uint32_t n = p.meta[s].rows * p.heads;
         if (w < base + n) break;
         base += n;
     }
-    if (s >= p.nseq) return;  // whole workgroup: no barrier is skipped by part of it
+    if (s >= p.nseq) return;  // (kEach has no barrier; else the whole workgroup)
     const PrefillMeta m = p.meta[s];
     const uint32_t r = (w - base) / p.heads;
     const uint32_t head = (w - base) % p.heads;
     const uint32_t nparts = m.nblk;
     const float *rec = vp.partials +
                        ((size_t)vp.rec0[s] + ((size_t)r * p.heads + head) * nparts) * kRecordStride<D>;
-    // maximum over the partition maxima, all threads of the workgroup
+    // maximum over the partition maxima, all threads of the workgroup (or wave)
     float mx = -INFINITY;
-    for (uint32_t q = threadIdx.x; q < nparts; q += 64 * kCombineWaves) {
+    for (uint32_t q = kEach ? lane : threadIdx.x; q < nparts; q += 64 * kStep) {
         mx = fmaxf(mx, rec[(size_t)q * kRecordStride<D>]);
     }
     mx = max64(mx);
-    if (lane == 0) max_s[wave] = mx;
-    __syncthreads();
+    if constexpr (!kEach) {
+        if (lane == 0) max_s[wave] = mx;
+        __syncthreads();
 #pragma unroll
-    for (int i = 0; i < kCombineWaves; ++i) mx = fmaxf(mx, max_s[i]);
+        for (int i = 0; i < kCombineWaves; ++i) mx = fmaxf(mx, max_s[i]);
+    }
     // this wave's records: weight 2^(m - max) (0 for a record with no
     // visible key, m = -inf, whose o is never used), sum and output
     float l = 0.0f;
     float o[EPL] = {};
-    for (uint32_t q0 = wave; q0 < nparts; q0 += kCombineWaves * kUnroll) {
+    for (uint32_t q0 = kEach ? 0 : wave; q0 < nparts; q0 += kStep * kUnroll) {
         float2 ml[kUnroll];
         float x[kUnroll][EPL];
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
             // past the last record: the last one again, with weight 0
-            const uint32_t q = min(q0 + (uint32_t)(kCombineWaves * u), nparts - 1);
+            const uint32_t q = min(q0 + kStep * u, nparts - 1);
             const float *rq = rec + (size_t)q * kRecordStride<D>;
             ml[u] = *(const float2 *)rq;
 #pragma unroll
@@ -2742,26 +2801,28 @@ __global__ __launch_bounds__(64 * kCombineWaves) void attn_verify_combine_kernel
         }
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
-            const bool live = q0 + (uint32_t)(kCombineWaves * u) < nparts && ml[u].x != -INFINITY;
+            const bool live = q0 + kStep * u < nparts && ml[u].x != -INFINITY;
             const float sc = live ? fast_exp2(ml[u].x - mx) : 0.0f;
             l += live ? ml[u].y * sc : 0.0f;
 #pragma unroll
             for (int i = 0; i < EPL; ++i) o[i] += live ? x[u][i] * sc : 0.0f;
         }
     }
+    if constexpr (!kEach) {
 #pragma unroll
-    for (int i = 0; i < EPL; ++i) part_s[wave][lane + 64 * i] = o[i];
-    if (lane == 0) part_s[wave][D] = l;
-    __syncthreads();
-    if (wave != 0) return;
-    l = 0.0f;
+        for (int i = 0; i < EPL; ++i) part_s[wave][lane + 64 * i] = o[i];
+        if (lane == 0) part_s[wave][D] = l;
+        __syncthreads();
+        if (wave != 0) return;
+        l = 0.0f;
 #pragma unroll
-    for (int k = 0; k < kCombineWaves; ++k) l += part_s[k][D];
+        for (int k = 0; k < kCombineWaves; ++k) l += part_s[k][D];
 #pragma unroll
-    for (int i = 0; i < EPL; ++i) {
-        o[i] = 0.0f;
+        for (int i = 0; i < EPL; ++i) {
+            o[i] = 0.0f;
 #pragma unroll
-        for (int k = 0; k < kCombineWaves; ++k) o[i] += part_s[k][lane + 64 * i];
+            for (int k = 0; k < kCombineWaves; ++k) o[i] += part_s[k][lane + 64 * i];
+        }
     }
     const bool bf16_in = (p.flags & SAFETYRAISE_MI355X_INPUT_BF16) != 0;
     const bool gated = (p.flags & SAFETYRAISE_MI355X_GATED) != 0;
@@ -2780,22 +2841,30 @@ __global__ __launch_bounds__(64 * kCombineWaves) void attn_verify_combine_kernel
     if (!finite) atomicOr(p.err_word, kErrPrefillRange);
 }
 
-template <int D, bool kAllTiles, bool kShared = false>
+template <int D, bool kAllTiles>
 hipError_t launch_verify_d(hipStream_t stream, const VerifyParams &vp, uint32_t blocks,
                            uint32_t combine_rows) {
     const size_t lds = kVerifyTileLds<D> + kVerifyPageSlots * sizeof(int32_t);
     static_assert(kVerifyTileLds<D> + kVerifyPageSlots * sizeof(int32_t) <= 160 * 1024,
                   "verify LDS");
     static const hipError_t configured =
-        hipFuncSetAttribute((const void *)attn_verify_kernel<D, kAllTiles, kShared>,
+        hipFuncSetAttribute((const void *)attn_verify_kernel<D, kAllTiles>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (configured != hipSuccess) return configured;
-    SR_LAUNCH("attn_verify_kernel", (attn_verify_kernel<D, kAllTiles, kShared>), dim3(blocks),
+    SR_LAUNCH("attn_verify_kernel", (attn_verify_kernel<D, kAllTiles>), dim3(blocks),
               dim3(kVerifyThreads), lds, stream, vp);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    SR_LAUNCH("attn_verify_combine_kernel", attn_verify_combine_kernel<D>, dim3(combine_rows),
-              dim3(64 * kCombineWaves), 0, stream, vp);
+    if (e != hipSuccess || vp.direct) return e;
+    uint32_t records = 0;  // per (row, head), at most
+    for (uint32_t i = 0; i < vp.p.nseq; ++i) records = std::max(records, vp.p.meta[i].nblk);
+    if (records <= kCombineBatch && combine_rows >= 1024) {
+        SR_LAUNCH("attn_verify_combine_kernel", (attn_verify_combine_kernel<D, true>),
+                  dim3((combine_rows + kCombineWaves - 1) / kCombineWaves), dim3(64 * kCombineWaves), 0,
+                  stream, vp);
+    } else {
+        SR_LAUNCH("attn_verify_combine_kernel", (attn_verify_combine_kernel<D, false>),
+                  dim3(combine_rows), dim3(64 * kCombineWaves), 0, stream, vp);
+    }
     return hipGetLastError();
 }
 
@@ -2866,27 +2935,125 @@ hipError_t launch_attn_prefill(hipStream_t stream, const AttnLaunch &a, const Se
     }
 }
 
+// Sequences of 16 or more rows that may take the split-K kernel.  The prefill
+// kernels run one workgroup per row block and KV head down the whole context,
+// so a chunk of few rows leaves most CUs idle: 32 rows of 32 / 8 x 128 at 4096
+// keys 90 us, split 25; at 16 K keys 323 / 38.  Below these lengths the second
+// launch and the records cost what the split gives (32 rows at 320 keys 18 / 17
+// us, 256 rows at 640 keys 31 / 24 but four such sequences 32 / 58).  Head_dim
+// 256 has no kernel but the lock-step one, 10 us per 64 keys (32 rows of 16 / 2
+// at 1 K keys 206 us, split 28; 1024 rows 364 / 88, four such 668 / 292).
+bool split_candidate(const AttnLaunch &a, uint32_t ctx, uint32_t rows) {
+    if (!prefill_supported(a)) return false;
+    const uint32_t g = a.heads / (a.kv_heads * a.kv_rep);
+    const uint64_t keys = (uint64_t)ctx + rows;
+    if (a.head_dim > 128) return keys > 256;
+    return keys > (rows * g <= 128 && rows <= 64 ? 320u : 1024u);
+}
+
+// Whether the candidates of a call (all its sequences in seqs) run faster
+// split, by a margin of a tenth.  Times in us, fitted to calls of one and four
+// sequences of 16 to 1024 rows at 128 to 16 K keys: the prefill kernels take
+// a start and a time per 64-key tile of the longest workgroup (more with every
+// CU busy), the split form a start, a time per tile of an equal share per CU,
+// and the merge of the records.  32 / 8 x 128, estimated (measured): 512 rows
+// at 4096 keys 125 (105) / 78 (65), 1024 rows at 16 K 534 (373) / 400 (346),
+// four sequences of 512 rows at 4096 keys 150 (144) / 233 (243).
+bool split_preferred(const AttnLaunch &a, const SeqMeta *seqs, int nseq, int num_cus) {
+    if (nseq <= 0) return false;
+    if (a.head_dim > 128) return true;
+    struct Times {
+        double start, tile, tile_busy, split_start, split_tile;
+    };
+    const Times t = a.head_dim == 64 ? Times{6, 1.43, 0.05, 11, 0.95} : Times{12, 1.22, 0.7, 17, 1.4};
+    const uint32_t kvv = a.kv_heads * a.kv_rep, g = a.heads / kvv;
+    const double cus = num_cus > 0 ? num_cus : 1;
+    double wgs = 0, total = 0, longest = 0, split = 0, records = 0;
+    for (int i = 0; i < nseq; ++i) {
+        const double vectors = (double)seqs[i].rows * g;
+        const double tiles = ((double)seqs[i].ctx + seqs[i].rows) / kKeyTile;
+        const double blocks = ceil(vectors / 256) * kvv;
+        wgs += blocks;
+        total += blocks * tiles;
+        longest = std::max(longest, tiles);
+        split += ceil(vectors / 128) * kvv * (tiles - 0.5 * seqs[i].rows / kKeyTile);
+        records += vectors * kvv;
+    }
+    const double whole = t.start + (t.tile + t.tile_busy * std::min(1.0, wgs / cus)) *
+                                       std::max(longest, total / cus);
+    const double parts = t.split_start + t.split_tile * std::max(split / cus, 2.0) + 0.0004 * records;
+    return parts * 1.1 < whole;
+}
+
 bool verify_supported(const AttnLaunch &a, uint32_t rows) {
     // any rows (the router sends 2..15): more than 64 query vectors per KV
     // head run as row slices
     return prefill_supported(a) && rows >= 2;
 }
 
+// Keys per partition, a multiple of the 64-key tile, of sequences in descending
+// order of their keys.  A workgroup has a CU to itself and costs its keys plus
+// a start and end worth about 5 tiles, so the candidates are one to four
+// workgroups per CU, each with the smallest partition of at least 256 keys that
+// keeps to that number, and, with one record per partition, no split and no
+// merge pass: the first sequence's workgroups in whole rounds, those of shorter
+// ones after what is before them.
+uint32_t verify_partition(const AttnLaunch &a, const SeqMeta *seqs, int nseq, uint32_t rows_per_slice,
+                          uint32_t records_per_part, int num_cus) {
+    const uint64_t kvv = (uint64_t)a.kv_heads * a.kv_rep;
+    const uint64_t cus = std::max(num_cus, 1);
+    constexpr uint64_t kEnds = 5 * kKeyTile;
+    constexpr uint64_t kMerge = 3 * kKeyTile;
+    auto up = [](uint64_t x, uint64_t unit) { return (x + unit - 1) / unit; };
+    auto slices = [&](int i) { return up(seqs[i].rows, rows_per_slice); };
+    auto total = [&](int i) { return (uint64_t)seqs[i].ctx + seqs[i].rows; };
+    // a partition starting mid-page touches at most part/page_tokens + 2 pages
+    const uint64_t max_part = std::min<uint64_t>(
+        ((uint64_t)(kVerifyPageSlots - 2) * a.pool->page_tokens) / kKeyTile * kKeyTile, 1u << 30);
+    const uint64_t longest = up(total(0), kKeyTile) * kKeyTile;
+    uint64_t keys = 0, unsplit = 0, before = 0;
+    for (int i = 0; i < nseq; ++i) {
+        const uint64_t n = slices(i) * kvv;
+        // (a slice sees the context and the rows up to its own last)
+        keys += n * seqs[i].ctx + kvv * (seqs[i].rows + rows_per_slice * (slices(i) - 1)) * slices(i) / 2;
+        unsplit = std::max(unsplit, i == 0 ? up(n, cus) * (total(i) + kEnds)
+                                           : (before + n * (total(i) + kEnds)) / cus + total(i));
+        before += n * (total(i) + kEnds);
+    }
+    uint64_t best = std::min(longest, max_part);
+    uint64_t best_time = longest > max_part ? ~0ull : unsplit + (records_per_part > 1 ? kMerge : 0);
+    for (uint64_t per = 1; per <= 4; ++per) {
+        uint64_t part = std::max<uint64_t>(256, up(keys, per * cus * kKeyTile) * kKeyTile);
+        // (each sequence's last partition is short: a few steps up until they fit)
+        for (int step = 0; step < 32 && part < longest; ++step) {
+            uint64_t n = 0;
+            for (int i = 0; i < nseq; ++i) n += up(total(i), part) * kvv * slices(i);
+            if (n <= per * cus) break;
+            part += up(part, 32 * kKeyTile) * kKeyTile;
+        }
+        part = std::min(part, max_part);
+        if (part >= longest) continue;
+        const uint64_t time = per * (part + kEnds) + kMerge;
+        if (time < best_time) {
+            best_time = time;
+            best = part;
+        }
+    }
+    return (uint32_t)best;
+}
+
 hipError_t launch_attn_verify(hipStream_t stream, const AttnLaunch &a, const SeqMeta *seqs,
-                              int nseq, void *rope_scratch, const DecodePlanInput &in) {
+                              int nseq, void *rope_scratch, const DecodePlanInput &in,
+                              uint64_t record_limit) {
     if (nseq <= 0 || nseq > kMetaPerLaunch || rope_scratch == nullptr) return hipErrorInvalidValue;
     const uint32_t kvv = a.kv_heads * a.kv_rep;  // KV heads of the grid
     const uint32_t g = a.heads / kvv;
     VerifyParams vp{};
     vp.p = fill_params(a, nseq, rope_scratch);
     PrefillParams &p = vp.p;
-    // partition size: one workgroup per CU over the whole call, at least
-    // 256 keys, a multiple of the 64-key tile
-    uint64_t keys = 0;
     uint32_t max_rows = 0;
     for (int i = 0; i < nseq; ++i) {
         if (!verify_supported(a, seqs[i].rows)) return hipErrorInvalidValue;
-        keys += (uint64_t)seqs[i].ctx + seqs[i].rows;
         max_rows = std::max(max_rows, seqs[i].rows);
     }
     // query vectors per workgroup: 64 in the pair mode; at D <= 128 a call
@@ -2894,57 +3061,57 @@ hipError_t launch_attn_verify(hipStream_t stream, const AttnLaunch &a, const Seq
     // rows beyond run as further slices of the rows
     const bool all_tiles = a.head_dim <= 128 && max_rows * g > 64;
     vp.rows_per_slice = (all_tiles ? 128 : 64) / g;
-    vp.slices = (max_rows + vp.rows_per_slice - 1) / vp.rows_per_slice;
-    const uint64_t target = (uint64_t)std::max(in.num_cus, 1);
-    uint64_t part = (keys * kvv * vp.slices + target - 1) / target;
-    part = std::max<uint64_t>(256, (part + kKeyTile - 1) / kKeyTile * kKeyTile);
-    // a partition starting mid-page touches at most part/page_tokens + 2 pages
-    const uint64_t max_part =
-        ((uint64_t)(kVerifyPageSlots - 2) * a.pool->page_tokens) / kKeyTile * kKeyTile;
-    vp.part_keys = (uint32_t)std::min<uint64_t>(std::min(part, max_part), 1u << 30);
     const uint32_t tps = (a.head_dim <= 128 && !all_tiles) ? 2 : 1;  // records per partition
-    uint32_t blocks = 0, records = 0, waves = 0;
+    // the longest workgroups first: sequences in order of their keys
+    SeqMeta sorted[kMetaPerLaunch];
+    std::copy(seqs, seqs + nseq, sorted);
+    std::stable_sort(sorted, sorted + nseq, [](const SeqMeta &x, const SeqMeta &y) {
+        return (uint64_t)x.ctx + x.rows > (uint64_t)y.ctx + y.rows;
+    });
+    vp.part_keys = verify_partition(a, sorted, nseq, vp.rows_per_slice, tps, in.num_cus);
+    uint32_t blocks = 0, waves = 0;
+    uint64_t records = 0;
     for (int i = 0; i < nseq; ++i) {
         PrefillMeta &m = p.meta[i];
-        m.slot = seqs[i].slot;
-        m.ctx = seqs[i].ctx;
-        m.rows = seqs[i].rows;
-        m.row0 = seqs[i].row0;
+        const SeqMeta &q = sorted[i];
+        m.slot = q.slot;
+        m.ctx = q.ctx;
+        m.rows = q.rows;
+        m.row0 = q.row0;
         const uint32_t parts = (m.ctx + m.rows + vp.part_keys - 1) / vp.part_keys;
         m.nblk = tps * parts;  // records per (row, head): one per tile of a step
         vp.blk0[i] = blocks;
-        vp.rec0[i] = records;
-        blocks += parts;
-        records += m.nblk * m.rows * a.heads;
+        vp.rec0[i] = (uint32_t)records;
+        blocks += parts * kvv * ((m.rows + vp.rows_per_slice - 1) / vp.rows_per_slice);
+        records += (uint64_t)m.nblk * m.rows * a.heads;
         waves += m.rows * a.heads;
     }
     p.max_blk = 0;
     const size_t stride = a.head_dim == 64    ? kRecordStride<64>
                           : a.head_dim == 128 ? kRecordStride<128>
                                               : kRecordStride<256>;
-    vp.partials = in.reserve_partials((size_t)records * stride * sizeof(float));
-    if (vp.partials == nullptr) return hipErrorOutOfMemory;
+    vp.direct = tps == 1;
+    for (int i = 0; i < nseq; ++i) vp.direct = vp.direct && p.meta[i].nblk == 1;
+    if (!vp.direct) {
+        const uint64_t bytes = records * stride * sizeof(float);
+        vp.partials = bytes <= record_limit ? in.reserve_partials(bytes) : nullptr;
+        if (vp.partials == nullptr) return hipErrorOutOfMemory;
+    }
     // K/V of the new rows and their RoPE cos/sin first (append kernel)
     if (a.head_dim == 64) launch_append<64>(stream, p, max_rows);
     else if (a.head_dim == 128) launch_append<128>(stream, p, max_rows);
     else launch_append<256>(stream, p, max_rows);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    vp.units = blocks * kvv;
-    // (unit, slice) blocks: groups of 8 units, each group's slices 8 apart
-    const uint32_t grid = (vp.units + 7) / 8 * 8 * vp.slices;
     if (a.head_dim == 64) {
-        return all_tiles ? launch_verify_d<64, true>(stream, vp, grid, waves)
-                         : launch_verify_d<64, false>(stream, vp, grid, waves);
+        return all_tiles ? launch_verify_d<64, true>(stream, vp, blocks, waves)
+                         : launch_verify_d<64, false>(stream, vp, blocks, waves);
     }
     if (a.head_dim == 128) {
-        return all_tiles ? launch_verify_d<128, true>(stream, vp, grid, waves)
-                         : launch_verify_d<128, false>(stream, vp, grid, waves);
+        return all_tiles ? launch_verify_d<128, true>(stream, vp, blocks, waves)
+                         : launch_verify_d<128, false>(stream, vp, blocks, waves);
     }
-    // several row slices read each partition's tiles: ordinary loads keep
-    // them in L2 for the sibling slices (D <= 128 calls fit one slice)
-    return vp.slices > 1 ? launch_verify_d<256, false, true>(stream, vp, grid, waves)
-                         : launch_verify_d<256, false>(stream, vp, grid, waves);
+    return launch_verify_d<256, false>(stream, vp, blocks, waves);
 }
 
 }  // namespace sr

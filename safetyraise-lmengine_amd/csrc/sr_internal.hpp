@@ -312,17 +312,23 @@ bool prefill_supported(const AttnLaunch &a);
 size_t prefill_rope_bytes(const AttnLaunch &a, uint64_t total_rows);
 hipError_t launch_attn_prefill(hipStream_t s, const AttnLaunch &a, const SeqMeta *seqs, int nseq,
                                void *rope_scratch);
-// Multi-row verify (2..15 rows per sequence, rows x heads/kv_heads <= 64,
-// head_dim <= 128): split-K over key partitions with MFMA inner products,
-// then a combine pass; partial records come from in.reserve_partials.
+// Multi-row split-K attention (MTP verify rows, and prefill rows that would
+// leave most of the chip idle): key partitions with MFMA inner products, then
+// a combine pass; partial records come from in.reserve_partials, which is
+// asked before anything is launched (hipErrorOutOfMemory when it has none, or
+// when the records take more than record_limit bytes).
 bool verify_supported(const AttnLaunch &a, uint32_t rows);
+// Whether a sequence of prefill rows may take it, and whether a call's such
+// sequences should.
+bool split_candidate(const AttnLaunch &a, uint32_t ctx, uint32_t rows);
+bool split_preferred(const AttnLaunch &a, const SeqMeta *seqs, int nseq, int num_cus);
 // Head widths other than 64, 128 and 256 (up to kGenericMaxHeadDim): every
 // row of the call through the plain f32 kernels of attn_generic.hip (append,
 // then attention); a.rope_denom must hold the rotary pairs' denominators.
 bool generic_head_dim(uint32_t head_dim);
 hipError_t launch_attn_generic(hipStream_t s, const AttnLaunch &a, const SeqMeta *seqs, int nseq);
 hipError_t launch_attn_verify(hipStream_t s, const AttnLaunch &a, const SeqMeta *seqs, int nseq,
-                              void *rope_scratch, const DecodePlanInput &in);
+                              void *rope_scratch, const DecodePlanInput &in, uint64_t record_limit);
 
 struct GdnLaunch {
     const safetyraise_kernel_gdn_pool *pool;

@@ -269,3 +269,50 @@ def test_prefill_values_beyond_fp16_range_are_recomputed(pkg, backend, rng, torc
         backend.synchronize()
     assert "fp16 range" in str(err.value)
     pool.destroy()
+
+
+# (heads, kv_heads, head_dim, page tokens, [(context, rows)], attention kernels)
+SPLIT = "attn_verify_kernel"
+MERGE = "attn_verify_combine_kernel"
+SPLIT_CASES = [
+    # 128 and 132 query vectors (one slice, and one with a single row over),
+    # key counts one below, at and one above a multiple of the partition
+    (32, 8, 128, 64, [(1247, 33)], (SPLIT, MERGE)),
+    (32, 8, 128, 64, [(1248, 32)], (SPLIT, MERGE)),
+    (32, 8, 128, 16, [(1249, 32), (1300, 64)], (SPLIT, MERGE)),
+    # one slice of 64 vectors or fewer (a record per tile of a step)
+    (32, 8, 128, 16, [(1100, 16)], (SPLIT, MERGE)),
+    # slices whose rows end before the last partition begins
+    (8, 2, 256, 16, [(0, 600)], (SPLIT, MERGE)),
+    # a group of fewer than 8 (partition, KV head) units, ragged slices
+    (10, 2, 128, 16, [(2000, 90), (1500, 201), (2300, 17)], (SPLIT, MERGE)),
+    (14, 2, 64, 32, [(1500, 130), (1111, 19)], (SPLIT, MERGE)),
+    # row slices enough for every CU: no partitions, no merge
+    (16, 2, 256, 64, [(250, 700), (40, 500)], (SPLIT,)),
+    # with a short chunk (prefill kernels), drafts and a decode row beside it
+    (32, 8, 128, 64, [(2100, 40), (0, 50), (700, 3), (333, 1)],
+     (SPLIT, MERGE, "attn_prefill_pipe_kernel", "attn_decode_kernel")),
+]
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,page,seqs,kernels", SPLIT_CASES)
+def test_prefill_rows_split_over_the_keys(pkg, backend, rng, heads, kv_heads, dim, page, seqs,
+                                          kernels):
+    pool = new_pool(pkg, backend, kv_heads, dim, page_tokens=page, max_tokens=4096, seqs=4)
+    qk_norm, gated = dim != 64, dim == 256
+    gq, gk = gammas(rng, dim) if qk_norm else (None, None)
+    args = dict(rotary=dim)
+    if gated:
+        gq, gk = gq - 1, gk - 1
+        args = dict(rotary=64, theta=1e7, gated=True, offset=True, mrope=(11, 11, 10))
+    cases = [Case(rng, pool, heads, kv_heads, dim, ctx=c, rows=r, gated=gated, qk_norm=qk_norm,
+                  pos_axes=(0, 3, 7) if gated else None)
+             for c, r in seqs]
+    backend.timing(True)
+    try:
+        run_case(pkg, backend, pool, cases, gq=gq, gk=gk, **args)
+        ran = {name for name in backend.kernel_times() if name.startswith("attn_")}
+    finally:
+        backend.timing(False)
+    assert set(kernels) <= ran and (MERGE in kernels) == (MERGE in ran), ran
+    pool.destroy()

@@ -943,6 +943,20 @@ __global__ __launch_bounds__(256) void linear_zero_kernel(float *y, uint64_t cou
     if (i < count) y[i] = 0.0f;
 }
 
+// The input of a host call from pinned host memory: one 16-byte load a lane,
+// all in flight at once, so a call costs about one round trip over the host link.
+__global__ __launch_bounds__(256) void linear_input_kernel(const float4 *src, float4 *dst, uint32_t n) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
+hipError_t launch_linear_input(hipStream_t stream, const float *src, float *dst, uint64_t count) {
+    const uint32_t n = (uint32_t)((count + 3) / 4);
+    SR_LAUNCH("linear_input_kernel", linear_input_kernel, dim3((n + 255) / 256), dim3(256), 0, stream,
+              (const float4 *)src, (float4 *)dst, n);
+    return hipGetLastError();
+}
+
 hipError_t launch_linear(hipStream_t stream, const float *x, const void *w, uint32_t dtype,
                          float *y, uint32_t M, uint32_t N, uint32_t K, float *scratch,
                          size_t scratch_bytes, int num_cus) {

@@ -250,6 +250,7 @@ SAFETYRAISE_KERNEL_EXPORT int32_t safetyraise_kernel_destroy_context(
                             &context->linear_part}) {
         if (b->ptr != nullptr) (void)hipFree(b->ptr);
     }
+    if (context->linear_host != nullptr) (void)hipHostFree(context->linear_host);
     destroy_timer_events(context->timer);
     if (context->d_error_word != nullptr) (void)hipFree(context->d_error_word);
     if (context->own_stream != nullptr) (void)hipStreamDestroy(context->own_stream);
@@ -397,6 +398,25 @@ static int32_t linear_scratch(Ctx *ctx, const safetyraise_kernel_weight *w, uint
     *have = bytes;
     return kOk;
 }
+
+// The context's pinned staging for small host calls, allocated once.  Without
+// memory for it (or where it cannot be mapped) calls use pageable copies.
+static bool linear_host(Ctx *ctx) {
+    if (ctx->linear_host != nullptr) return true;
+    void *host = nullptr, *dev = nullptr;
+    if (hipHostMalloc(&host, 2 * kLinearHostBytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (hipHostGetDevicePointer(&dev, host, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipHostFree(host);
+        return false;
+    }
+    ctx->linear_host = host;
+    ctx->linear_host_dev = (float *)dev;
+    return true;
+}
 }  // namespace sr
 
 SAFETYRAISE_KERNEL_EXPORT int32_t safetyraise_kernel_linear(
@@ -411,25 +431,40 @@ SAFETYRAISE_KERNEL_EXPORT int32_t safetyraise_kernel_linear(
     const int32_t st = check_linear(context, weight, input, input_rows, input_cols, output,
                                     output_rows, output_cols, &in_count, &out_count);
     if (st != kOk) return st;
-    // native/cpu/safetyraise_cpu.c:221-226: every input must be finite
-    for (uint64_t i = 0; i < in_count; ++i) {
-        if (!std::isfinite(input[i])) {
-            return fail(context, kInvalid, "linear input contains non-finite values");
-        }
+    // Small calls stage through pinned memory (sr_internal.hpp: linear_host)
+    float *host_in = nullptr, *host_out = nullptr;
+    if (std::max(in_count, out_count) * 4 <= kLinearHostBytes && linear_host(context)) {
+        host_in = (float *)context->linear_host;
+        host_out = host_in + kLinearHostBytes / 4;
     }
+    // native/cpu/safetyraise_cpu.c:221-226: every input must be finite.  The
+    // exponent bits alone, without a branch per value: the loop is vectorised.
+    uint32_t infinite = 0;
+    for (uint64_t i = 0; i < in_count; ++i) {
+        uint32_t bits;
+        memcpy(&bits, input + i, sizeof bits);
+        infinite |= (bits & 0x7F800000u) == 0x7F800000u ? 1u : 0u;
+    }
+    if (infinite != 0) return fail(context, kInvalid, "linear input contains non-finite values");
     if (out_count == 0) return kOk;
     int32_t e = ensure_buffer(context, context->linear_in, (size_t)(in_count ? in_count : 1) * 4,
                               false);
     if (e != kOk) return e;
-    e = ensure_buffer(context, context->linear_out, (size_t)out_count * 4, false);
-    if (e != kOk) return e;
+    if (host_out == nullptr) {
+        e = ensure_buffer(context, context->linear_out, (size_t)out_count * 4, false);
+        if (e != kOk) return e;
+    }
     float *part = nullptr;
     size_t part_bytes = 0;
     e = linear_scratch(context, weight, input_rows, &part, &part_bytes);
     if (e != kOk) return e;
     float *d_in = (float *)context->linear_in.ptr;
-    float *d_out = (float *)context->linear_out.ptr;
-    if (in_count != 0) {
+    float *d_out = host_out != nullptr ? context->linear_host_dev + kLinearHostBytes / 4
+                                       : (float *)context->linear_out.ptr;
+    if (in_count != 0 && host_in != nullptr) {
+        memcpy(host_in, input, in_count * 4);
+        SR_HIP(context, launch_linear_input(context->stream, context->linear_host_dev, d_in, in_count));
+    } else if (in_count != 0) {
         SR_HIP(context, hipMemcpyAsync(d_in, input, in_count * 4, hipMemcpyHostToDevice,
                                        context->stream));
     }
@@ -437,9 +472,12 @@ SAFETYRAISE_KERNEL_EXPORT int32_t safetyraise_kernel_linear(
                                   (uint32_t)input_rows, (uint32_t)weight->rows,
                                   (uint32_t)weight->cols, part, part_bytes,
                                   context->num_cus));
-    SR_HIP(context, hipMemcpyAsync(output, d_out, out_count * 4, hipMemcpyDeviceToHost,
-                                   context->stream));
+    if (host_out == nullptr) {
+        SR_HIP(context, hipMemcpyAsync(output, d_out, out_count * 4, hipMemcpyDeviceToHost,
+                                       context->stream));
+    }
     SR_HIP(context, hipStreamSynchronize(context->stream));
+    if (host_out != nullptr) memcpy(output, host_out, out_count * 4);
     return kOk;
 }
 

@@ -90,6 +90,16 @@ struct RopeTable {
 
 }  // namespace sr
 
+namespace sr {
+// Host-pointer linear calls with at most this much input and output stage
+// through pinned memory: a kernel fetches the input and the outputs are written
+// straight to the host.  The seven projections of a 4096-wide layer (k/v 1024,
+// MLP 12288), pageable copies / pinned: 1 row 269 / 197 us, 6 rows 296 / 258,
+// 32 rows 745 / 667, 64 rows (3 MB of output) 1305 / 1245, where the copies
+// themselves outweigh the fixed costs.
+constexpr uint64_t kLinearHostBytes = 2 << 20;
+}  // namespace sr
+
 struct safetyraise_kernel_context {
     int device = 0;
     int num_cus = 256;
@@ -104,6 +114,10 @@ struct safetyraise_kernel_context {
     sr::DeviceBuffer linear_in;        // linear: the host input's device copy
     sr::DeviceBuffer linear_out;       // linear: the output before it goes back
     sr::DeviceBuffer linear_part;      // linear: partial sums of calls that split K
+    // linear: pinned host staging, kLinearHostBytes of input, then of output,
+    // and its device address
+    void *linear_host = nullptr;
+    float *linear_host_dev = nullptr;
     float rope_theta = 0.0f;
     uint32_t rope_dim = 0;
     sr::RopeTable rope{};
@@ -379,6 +393,9 @@ size_t linear_weight_bytes(uint64_t rows, uint64_t cols, uint32_t dtype);
 // The BF16 tile layout in dst from a row-major bf16 weight in device memory.
 hipError_t linear_pack_bf16(hipStream_t stream, const void *src, void *dst, uint64_t rows,
                             uint64_t cols);
+// count floats of mapped host memory to device memory (both 16-byte aligned,
+// with room up to a multiple of four floats)
+hipError_t launch_linear_input(hipStream_t stream, const float *src, float *dst, uint64_t count);
 hipError_t launch_linear(hipStream_t stream, const float *x, const void *w, uint32_t dtype,
                          float *y, uint32_t M, uint32_t N, uint32_t K, float *scratch,
                          size_t scratch_bytes, int num_cus);

@@ -400,3 +400,30 @@ def test_captured_call_keeps_no_scratch(backend, rng, torch_mod):
     finally:
         backend.set_stream(None)
         prepared.destroy()
+
+
+# host calls whose input or output is just within and just past the 2 MB that
+# stage through pinned memory, and counts that are no multiple of four floats
+@pytest.mark.parametrize("rows,cols,out", [(512, 1024, 33), (512, 1025, 33), (1024, 40, 512),
+                                           (1023, 40, 513), (3, 1001, 7), (1, 1, 1)])
+def test_host_calls_equal_device_calls(backend, rng, torch_mod, rows, cols, out):
+    torch = torch_mod
+    w = rng.standard_normal((out, cols)).astype(np.float32)
+    prepared = backend.create_weight(weight_bits(w, BF16), BF16)
+    try:
+        for _ in range(2):
+            x = rng.standard_normal((rows, cols)).astype(np.float32)
+            dx = torch.from_numpy(x).cuda()
+            dy = torch.full((rows, out), float("nan"), device="cuda")
+            torch.cuda.synchronize()
+            device_call(backend, prepared, dx, dy, rows, cols, out)
+            backend.synchronize()
+            assert np.array_equal(backend.linear(prepared, x), dy.cpu().numpy())
+        for bad in (np.nan, np.inf, -np.inf):
+            x[-1, -1] = bad
+            with pytest.raises(Exception, match="non-finite"):
+                backend.linear(prepared, x)
+        x[-1, -1] = np.finfo(np.float32).max
+        assert np.isfinite(backend.linear(prepared, 1e-6 * x)).all()
+    finally:
+        prepared.destroy()

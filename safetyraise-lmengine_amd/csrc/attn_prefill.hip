@@ -2659,11 +2659,15 @@ attn_verify_kernel(const VerifyParams vp) {
     const uint32_t key_limit = m.ctx + r;
     const uint32_t hs = (p.flags & SAFETYRAISE_MI355X_GATED) ? 2 * D : D;
     const size_t qbase = (size_t)(m.row0 + r) * p.heads * hs + (size_t)head * hs;
+    // (A) is for the producers: the consumers reach it at once and read their
+    // queries while the first tiles are on their way (a prompt of 1500 rows by
+    // 32, 32 / 8 x 128: 1089 to 1070 us with (A) before the queries).  Ending
+    // the loop below at the last step, not at a multiple of kVerifyDepth, took
+    // that to 1060 us but long contexts lost 2 % (4 sequences of 40 K to 131 K
+    // keys at 16 / 2 x 256: 145 to 148 us).
+    __builtin_amdgcn_s_barrier();
     f16x8 qop[NS];
     if (computes) q_operands<D>(qa, qbase, m.row0 + r, h, lane, qop);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_s_barrier();  // (A)
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 
     f32x16 oacc[NTW];
 #pragma unroll

@@ -20,8 +20,8 @@
 // aligned whole blocks whatever its shape.
 //
 // Work split of linear_kernel.  A workgroup owns 16 R rows (R = 1, or 2 in one
-// plan) x 16 T outputs (T tiles per wave) and a contiguous range of K; its W waves take equal parts of that range
-// and meet in LDS.  Decode-sized calls (M <= 16) stream every weight row
+// plan) x 16 T outputs (T tiles per wave) and a contiguous range of K; its W
+// waves take equal parts of that range and meet in LDS.  Decode-sized calls (M <= 16) stream every weight row
 // once, the HBM-bound regime the ABI's projections live in; each k block
 // loads 32 bytes of x per lane, used by T tiles, and 8 weight elements per
 // tile.  x is the larger share of the bytes a lane loads, so T > 1 keeps the
@@ -135,11 +135,11 @@ __device__ __forceinline__ void split3(const f32x8 &x, bf16x8 &hi, bf16x8 &mid, 
     lo = __builtin_convertvector(r2, bf16x8);
 }
 
-// y: the output, or (grid z > 1) partial sums [grid z][M][N].  T: output tiles per wave (the workgroup owns 16 T
-// outputs; each x fragment a lane loads feeds T MFMAs, so x is read once
+// y: the output, or (grid z > 1) partial sums [grid z][M][N].  T: output tiles
+// per wave (the workgroup owns 16 T outputs; each x fragment a lane loads feeds T MFMAs, so x is read once
 // per 16 T outputs).  R: row tiles per workgroup (each weight fragment feeds
-// R rows' MFMAs; with R = 2 the weight is read once per 32 rows).  W: waves per workgroup, splitting its k range.  kGroup: k
-// blocks per register set (4; 2 for calls with many workgroups per CU, which
+// R rows' MFMAs; with R = 2 the weight is read once per 32 rows).  W: waves per
+// workgroup, splitting its k range.  kGroup: k blocks per register set (4; 2 for calls with many workgroups per CU, which
 // then hold more waves per SIMD).  kExact: every wave's k range is a whole
 // number of pairs of groups of whole blocks (the host checks), so no load
 // reaches past it, nothing is masked and the last pair prefetches nothing.

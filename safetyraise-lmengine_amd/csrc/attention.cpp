@@ -68,10 +68,11 @@ int32_t run_decode_pack(Ctx *ctx, const AttnLaunch &a, const std::vector<SeqMeta
 // The first pack launched carries the call's inline page-table entries
 // (AttnLaunch::tbl_*); they are cleared once a launch has taken them.
 int32_t run_verify_pack(Ctx *ctx, AttnLaunch &a, const std::vector<SeqMeta> &pack,
-                        const AttnScratch &scratch, void *rope, uint64_t record_limit) {
+                        const AttnScratch &scratch, void *rope, uint64_t record_limit,
+                        bool strict) {
     DecodePlanInput plan{ctx->num_cus, scratch.partials, scratch.user};
-    const hipError_t e =
-        launch_attn_verify(ctx->stream, a, pack.data(), (int)pack.size(), rope, plan, record_limit);
+    const hipError_t e = launch_attn_verify(ctx->stream, a, pack.data(), (int)pack.size(), rope, plan,
+                                            record_limit, strict);
     if (e == hipErrorOutOfMemory) return kNoMemory;  // (nothing was launched)
     a.tbl_n = 0;
     if (e != hipSuccess) return hip_fail(ctx, e, "verify attention launch");
@@ -336,9 +337,13 @@ int32_t attention_forward_impl(Ctx *ctx, const safetyraise_kernel_attention_args
     bool any_prefill = false;
     // the per-row RoPE table of the verify and prefill kernels
     void *rope = nullptr;
+    uint64_t record_limit = 0;
     if (prefill_ok && any_fast_route) {
-        rope = scratch.rope(scratch.user, prefill_rope_bytes(L, total_rows));
+        const size_t bytes = prefill_rope_bytes(L, total_rows);
+        rope = scratch.rope(scratch.user, bytes);
         if (rope == nullptr) return kNoMemory;
+        const uint64_t held = (bytes + kAttnScratchAlign - 1) / kAttnScratchAlign * kAttnScratchAlign;
+        record_limit = held < kAttnScratchBytes ? kAttnScratchBytes - held : 0;
     }
     auto meta = [&](uint32_t i) {
         SeqMeta m{};
@@ -371,7 +376,7 @@ int32_t attention_forward_impl(Ctx *ctx, const safetyraise_kernel_attention_args
             return A.seq_rows[i] < kPrefillMinRows && verify_supported(L, A.seq_rows[i]);
         },
         [&](const std::vector<SeqMeta> &pack) {
-            return run_verify_pack(ctx, L, pack, scratch, rope, UINT64_MAX);
+            return run_verify_pack(ctx, L, pack, scratch, rope, record_limit, false);
         });
     if (pst != kOk) return pst;
     // Prefill rows whose row blocks would leave most of the CUs idle take it
@@ -391,7 +396,7 @@ int32_t attention_forward_impl(Ctx *ctx, const safetyraise_kernel_attention_args
     pst = run_packs([&](uint32_t i) { return preferred && split[i]; },
                     [&](const std::vector<SeqMeta> &pack) {
                         const int32_t st =
-                            run_verify_pack(ctx, L, pack, scratch, rope, kSplitRecordBytes);
+                            run_verify_pack(ctx, L, pack, scratch, rope, kSplitRecordBytes, true);
                         if (st != kNoMemory) return st;
                         (void)hipGetLastError();
                         ctx->error.clear();

@@ -1,0 +1,123 @@
+// How a split-K attention launch (attn_verify_kernel in attn_prefill.hip) is
+// cut.  Host code only, so that it is tested without a GPU.
+#pragma once
+
+#include <algorithm>
+#include <cstdint>
+
+#include "sr_internal.hpp"
+
+namespace sr {
+
+constexpr int kKeyTile = 64;  // keys per LDS stage of the prefill and split-K kernels
+
+// LDS entries for the page ids of one partition (a partition never spans more
+// pages)
+constexpr uint32_t kVerifyPageSlots = 2048;
+
+// Floats of a partition record: m, l, 2 unused, o[head_dim] (16-byte aligned).
+constexpr uint32_t record_stride(uint32_t head_dim) { return head_dim + 4; }
+
+struct SplitShape {
+    uint32_t heads, kv_heads;  // of the grid: at most 8 query heads per KV head
+    uint32_t head_dim, page_tokens;
+    int num_cus;
+};
+
+struct SplitPlan {
+    bool all_tiles;             // each consumer wave takes both tiles of a step
+    bool direct;                // every (row, head) has one record: the output itself
+    uint32_t rows_per_slice;    // query rows per workgroup
+    uint32_t records_per_part;  // per (row, head): one per tile of a step
+    uint32_t part_keys;
+    uint64_t record_bytes;
+};
+
+// Keys per partition, a multiple of the 64-key tile, of sequences in descending
+// order of their keys.  A workgroup has a CU to itself and costs its keys plus
+// a start and end worth about 5 tiles, so the candidates are one to four
+// workgroups per CU, each with the smallest partition of at least 256 keys that
+// keeps to that number, and, with one record per partition, no split and no
+// merge pass: the first sequence's workgroups in whole rounds, those of shorter
+// ones after what is before them.
+//
+// A candidate whose records take more than record_limit bytes has its
+// partitions enlarged until they fit; with a partition for every KV head's
+// whole context there is nothing larger, and if that takes too much as well the
+// plan is the first candidate (one workgroup per CU) as it was, with
+// record_bytes above the limit.  64 sequences of 16 K keys and 8 rows each (64 /
+// 8 x 128): four workgroups per CU took 69 MB of records, one takes 35.
+inline SplitPlan split_plan(const SplitShape &a, const SeqMeta *seqs, int nseq,
+                            uint64_t record_limit) {
+    const uint64_t kvv = a.kv_heads, group = a.heads / a.kv_heads;
+    const uint64_t cus = std::max(a.num_cus, 1);
+    constexpr uint64_t kEnds = 5 * kKeyTile;
+    constexpr uint64_t kMerge = 3 * kKeyTile;
+    auto up = [](uint64_t x, uint64_t unit) { return (x + unit - 1) / unit; };
+    auto total = [&](int i) { return (uint64_t)seqs[i].ctx + seqs[i].rows; };
+    SplitPlan plan{};
+    uint64_t max_rows = 0;
+    for (int i = 0; i < nseq; ++i) max_rows = std::max<uint64_t>(max_rows, seqs[i].rows);
+    // query vectors per workgroup: 64 in the pair mode; at D <= 128 a call
+    // with more takes the all-tiles form (128 vectors over its four consumer
+    // waves), rows beyond run as further slices of the rows
+    plan.all_tiles = a.head_dim <= 128 && max_rows * group > 64;
+    plan.rows_per_slice = (uint32_t)((plan.all_tiles ? 128 : 64) / group);
+    plan.records_per_part = (a.head_dim <= 128 && !plan.all_tiles) ? 2 : 1;
+    auto slices = [&](int i) { return up(seqs[i].rows, plan.rows_per_slice); };
+    auto direct = [&](uint64_t part) { return plan.records_per_part == 1 && total(0) <= part; };
+    auto bytes = [&](uint64_t part) -> uint64_t {
+        if (direct(part)) return 0;
+        uint64_t n = 0;
+        for (int i = 0; i < nseq; ++i) n += up(total(i), part) * seqs[i].rows;
+        return n * plan.records_per_part * a.heads * record_stride(a.head_dim) * sizeof(float);
+    };
+    // a partition starting mid-page touches at most part/page_tokens + 2 pages
+    const uint64_t max_part = std::min<uint64_t>(
+        ((uint64_t)(kVerifyPageSlots - 2) * a.page_tokens) / kKeyTile * kKeyTile, 1u << 30);
+    const uint64_t longest = up(total(0), kKeyTile) * kKeyTile;
+    const uint64_t most = std::min(longest, max_part);
+    uint64_t keys = 0, unsplit = 0, before = 0;
+    for (int i = 0; i < nseq; ++i) {
+        const uint64_t n = slices(i) * kvv;
+        // (a slice sees the context and the rows up to its own last)
+        keys += n * seqs[i].ctx +
+                kvv * (seqs[i].rows + plan.rows_per_slice * (slices(i) - 1)) * slices(i) / 2;
+        unsplit = std::max(unsplit, i == 0 ? up(n, cus) * (total(i) + kEnds)
+                                           : (before + n * (total(i) + kEnds)) / cus + total(i));
+        before += n * (total(i) + kEnds);
+    }
+    uint64_t best = 0, best_time = ~0ull, first = 0;
+    if (longest <= max_part && bytes(longest) <= record_limit) {
+        best = longest;
+        best_time = unsplit + (plan.records_per_part > 1 ? kMerge : 0);
+    }
+    for (uint64_t per = 1; per <= 4; ++per) {
+        uint64_t part = std::max<uint64_t>(256, up(keys, per * cus * kKeyTile) * kKeyTile);
+        // (each sequence's last partition is short: a few steps up until they fit)
+        for (int step = 0; step < 32 && part < longest; ++step) {
+            uint64_t n = 0;
+            for (int i = 0; i < nseq; ++i) n += up(total(i), part) * kvv * slices(i);
+            if (n <= per * cus) break;
+            part += up(part, 32 * kKeyTile) * kKeyTile;
+        }
+        part = std::min(part, most);
+        if (per == 1) first = part;
+        while (part < most && bytes(part) > record_limit) {
+            part = std::min(most, part + up(part, 8 * kKeyTile) * kKeyTile);
+        }
+        if (part >= longest || bytes(part) > record_limit) continue;
+        const uint64_t time = per * (part + kEnds) + kMerge;
+        if (time < best_time) {
+            best_time = time;
+            best = part;
+        }
+    }
+    if (best == 0) best = first;
+    plan.part_keys = (uint32_t)best;
+    plan.direct = direct(best);
+    plan.record_bytes = bytes(best);
+    return plan;
+}
+
+}  // namespace sr

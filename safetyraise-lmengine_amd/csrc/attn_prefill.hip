@@ -41,6 +41,7 @@
 #include <cmath>
 #include <type_traits>
 
+#include "attn_plan.hpp"
 #include "sr_device.hpp"
 
 namespace sr {
@@ -56,7 +57,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kRowTile = 32;   // query rows per wave (the MFMA N dimension)
-constexpr int kKeyTile = 64;   // keys per LDS stage
 constexpr float kLazyRescale = 8.0f;
 
 struct PrefillMeta {
@@ -2363,11 +2363,7 @@ static_assert(sizeof(VerifyParams) <= 4096, "kernel arguments stay within 4 KiB"
 
 
 template <int D>
-constexpr int kRecordStride = D + 4;  // m, l, 2 unused, o[D] (16-byte aligned)
-
-// LDS entries for the page ids of one partition (the host caps part_keys so
-// that a partition never spans more pages)
-constexpr uint32_t kVerifyPageSlots = 2048;
+constexpr int kRecordStride = record_stride(D);
 
 // Tile staging of the verify producers (NL lanes per tile, lane gt: 128 at
 // D <= 128, where a step stages two tiles, 256 at D = 256, one tile per
@@ -2995,63 +2991,11 @@ bool verify_supported(const AttnLaunch &a, uint32_t rows) {
     return prefill_supported(a) && rows >= 2;
 }
 
-// Keys per partition, a multiple of the 64-key tile, of sequences in descending
-// order of their keys.  A workgroup has a CU to itself and costs its keys plus
-// a start and end worth about 5 tiles, so the candidates are one to four
-// workgroups per CU, each with the smallest partition of at least 256 keys that
-// keeps to that number, and, with one record per partition, no split and no
-// merge pass: the first sequence's workgroups in whole rounds, those of shorter
-// ones after what is before them.
-uint32_t verify_partition(const AttnLaunch &a, const SeqMeta *seqs, int nseq, uint32_t rows_per_slice,
-                          uint32_t records_per_part, int num_cus) {
-    const uint64_t kvv = (uint64_t)a.kv_heads * a.kv_rep;
-    const uint64_t cus = std::max(num_cus, 1);
-    constexpr uint64_t kEnds = 5 * kKeyTile;
-    constexpr uint64_t kMerge = 3 * kKeyTile;
-    auto up = [](uint64_t x, uint64_t unit) { return (x + unit - 1) / unit; };
-    auto slices = [&](int i) { return up(seqs[i].rows, rows_per_slice); };
-    auto total = [&](int i) { return (uint64_t)seqs[i].ctx + seqs[i].rows; };
-    // a partition starting mid-page touches at most part/page_tokens + 2 pages
-    const uint64_t max_part = std::min<uint64_t>(
-        ((uint64_t)(kVerifyPageSlots - 2) * a.pool->page_tokens) / kKeyTile * kKeyTile, 1u << 30);
-    const uint64_t longest = up(total(0), kKeyTile) * kKeyTile;
-    uint64_t keys = 0, unsplit = 0, before = 0;
-    for (int i = 0; i < nseq; ++i) {
-        const uint64_t n = slices(i) * kvv;
-        // (a slice sees the context and the rows up to its own last)
-        keys += n * seqs[i].ctx + kvv * (seqs[i].rows + rows_per_slice * (slices(i) - 1)) * slices(i) / 2;
-        unsplit = std::max(unsplit, i == 0 ? up(n, cus) * (total(i) + kEnds)
-                                           : (before + n * (total(i) + kEnds)) / cus + total(i));
-        before += n * (total(i) + kEnds);
-    }
-    uint64_t best = std::min(longest, max_part);
-    uint64_t best_time = longest > max_part ? ~0ull : unsplit + (records_per_part > 1 ? kMerge : 0);
-    for (uint64_t per = 1; per <= 4; ++per) {
-        uint64_t part = std::max<uint64_t>(256, up(keys, per * cus * kKeyTile) * kKeyTile);
-        // (each sequence's last partition is short: a few steps up until they fit)
-        for (int step = 0; step < 32 && part < longest; ++step) {
-            uint64_t n = 0;
-            for (int i = 0; i < nseq; ++i) n += up(total(i), part) * kvv * slices(i);
-            if (n <= per * cus) break;
-            part += up(part, 32 * kKeyTile) * kKeyTile;
-        }
-        part = std::min(part, max_part);
-        if (part >= longest) continue;
-        const uint64_t time = per * (part + kEnds) + kMerge;
-        if (time < best_time) {
-            best_time = time;
-            best = part;
-        }
-    }
-    return (uint32_t)best;
-}
-
 hipError_t launch_attn_verify(hipStream_t stream, const AttnLaunch &a, const SeqMeta *seqs,
                               int nseq, void *rope_scratch, const DecodePlanInput &in,
-                              uint64_t record_limit) {
+                              uint64_t record_limit, bool strict) {
     if (nseq <= 0 || nseq > kMetaPerLaunch || rope_scratch == nullptr) return hipErrorInvalidValue;
     const uint32_t kvv = a.kv_heads * a.kv_rep;  // KV heads of the grid
-    const uint32_t g = a.heads / kvv;
     VerifyParams vp{};
     vp.p = fill_params(a, nseq, rope_scratch);
     PrefillParams &p = vp.p;
@@ -3060,19 +3004,25 @@ hipError_t launch_attn_verify(hipStream_t stream, const AttnLaunch &a, const Seq
         if (!verify_supported(a, seqs[i].rows)) return hipErrorInvalidValue;
         max_rows = std::max(max_rows, seqs[i].rows);
     }
-    // query vectors per workgroup: 64 in the pair mode; at D <= 128 a call
-    // with more runs every consumer wave over both tiles of a step (128);
-    // rows beyond run as further slices of the rows
-    const bool all_tiles = a.head_dim <= 128 && max_rows * g > 64;
-    vp.rows_per_slice = (all_tiles ? 128 : 64) / g;
-    const uint32_t tps = (a.head_dim <= 128 && !all_tiles) ? 2 : 1;  // records per partition
     // the longest workgroups first: sequences in order of their keys
     SeqMeta sorted[kMetaPerLaunch];
     std::copy(seqs, seqs + nseq, sorted);
     std::stable_sort(sorted, sorted + nseq, [](const SeqMeta &x, const SeqMeta &y) {
         return (uint64_t)x.ctx + x.rows > (uint64_t)y.ctx + y.rows;
     });
-    vp.part_keys = verify_partition(a, sorted, nseq, vp.rows_per_slice, tps, in.num_cus);
+    const SplitPlan plan = split_plan({a.heads, kvv, a.head_dim, a.pool->page_tokens, in.num_cus},
+                                      sorted, nseq, record_limit);
+    const bool all_tiles = plan.all_tiles;
+    vp.rows_per_slice = plan.rows_per_slice;
+    vp.part_keys = plan.part_keys;
+    vp.direct = plan.direct;
+    if (!plan.direct) {
+        // (draft rows have no other kernel but the row-serial one)
+        vp.partials = plan.record_bytes <= record_limit || !strict
+                          ? in.reserve_partials(plan.record_bytes)
+                          : nullptr;
+        if (vp.partials == nullptr) return hipErrorOutOfMemory;
+    }
     uint32_t blocks = 0, waves = 0;
     uint64_t records = 0;
     for (int i = 0; i < nseq; ++i) {
@@ -3083,7 +3033,7 @@ hipError_t launch_attn_verify(hipStream_t stream, const AttnLaunch &a, const Seq
         m.rows = q.rows;
         m.row0 = q.row0;
         const uint32_t parts = (m.ctx + m.rows + vp.part_keys - 1) / vp.part_keys;
-        m.nblk = tps * parts;  // records per (row, head): one per tile of a step
+        m.nblk = plan.records_per_part * parts;  // records per (row, head)
         vp.blk0[i] = blocks;
         vp.rec0[i] = (uint32_t)records;
         blocks += parts * kvv * ((m.rows + vp.rows_per_slice - 1) / vp.rows_per_slice);
@@ -3091,16 +3041,6 @@ hipError_t launch_attn_verify(hipStream_t stream, const AttnLaunch &a, const Seq
         waves += m.rows * a.heads;
     }
     p.max_blk = 0;
-    const size_t stride = a.head_dim == 64    ? kRecordStride<64>
-                          : a.head_dim == 128 ? kRecordStride<128>
-                                              : kRecordStride<256>;
-    vp.direct = tps == 1;
-    for (int i = 0; i < nseq; ++i) vp.direct = vp.direct && p.meta[i].nblk == 1;
-    if (!vp.direct) {
-        const uint64_t bytes = records * stride * sizeof(float);
-        vp.partials = bytes <= record_limit ? in.reserve_partials(bytes) : nullptr;
-        if (vp.partials == nullptr) return hipErrorOutOfMemory;
-    }
     // K/V of the new rows and their RoPE cos/sin first (append kernel)
     if (a.head_dim == 64) launch_append<64>(stream, p, max_rows);
     else if (a.head_dim == 128) launch_append<128>(stream, p, max_rows);

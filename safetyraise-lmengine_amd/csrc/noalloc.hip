@@ -28,9 +28,9 @@
 namespace sr {
 namespace {
 
-constexpr size_t kNoAllocScratchBytes = (size_t)64 << 20;
+constexpr size_t kNoAllocScratchBytes = kAttnScratchBytes;
 constexpr int kMaxDevices = 64;
-constexpr size_t kScratchAlign = 256;
+constexpr size_t kScratchAlign = kAttnScratchAlign;
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 

@@ -287,6 +287,12 @@ struct AttnLaunch {
 };
 constexpr uint32_t kInlineTable = 64;
 
+// Bytes of the no-allocation entry point's scratch, which a call's RoPE table and
+// its split-K records share.  The plans of draft rows keep to what the table
+// leaves of it, in both entry points.
+constexpr size_t kAttnScratchBytes = (size_t)64 << 20;
+constexpr size_t kAttnScratchAlign = 256;
+
 // Device scratch of one attention call: the split-K partial records (decode
 // and verify) and the prefill RoPE table.  Each function returns nullptr,
 // with the context's error text set, when it cannot provide `bytes`.  The
@@ -328,9 +334,9 @@ hipError_t launch_attn_prefill(hipStream_t s, const AttnLaunch &a, const SeqMeta
                                void *rope_scratch);
 // Multi-row split-K attention (MTP verify rows, and prefill rows that would
 // leave most of the chip idle): key partitions with MFMA inner products, then
-// a combine pass; partial records come from in.reserve_partials, which is
-// asked before anything is launched (hipErrorOutOfMemory when it has none, or
-// when the records take more than record_limit bytes).
+// a combine pass.  The plan keeps its partial records to record_limit bytes
+// where it can (attn_plan.hpp); a strict call that cannot, and one whose records
+// in.reserve_partials does not provide, launches nothing (hipErrorOutOfMemory).
 bool verify_supported(const AttnLaunch &a, uint32_t rows);
 // Whether a sequence of prefill rows may take it, and whether a call's such
 // sequences should.
@@ -342,7 +348,8 @@ bool split_preferred(const AttnLaunch &a, const SeqMeta *seqs, int nseq, int num
 bool generic_head_dim(uint32_t head_dim);
 hipError_t launch_attn_generic(hipStream_t s, const AttnLaunch &a, const SeqMeta *seqs, int nseq);
 hipError_t launch_attn_verify(hipStream_t s, const AttnLaunch &a, const SeqMeta *seqs, int nseq,
-                              void *rope_scratch, const DecodePlanInput &in, uint64_t record_limit);
+                              void *rope_scratch, const DecodePlanInput &in, uint64_t record_limit,
+                              bool strict);
 
 struct GdnLaunch {
     const safetyraise_kernel_gdn_pool *pool;

@@ -1,0 +1,117 @@
+"""How a split-K attention launch is cut (csrc/attn_plan.hpp), without a GPU.
+
+split_plan is host code: a small program compiled from the header answers for
+calls written to its standard input.
+"""
+import random
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+CUS = 256
+REGION = 64 << 20  # the no-allocation entry point's scratch
+
+PROGRAM = r"""
+#include <cstdio>
+#include "attn_plan.hpp"
+int main() {
+    unsigned heads, kv, dim, page, n;
+    unsigned long long limit;
+    while (scanf("%u %u %u %u %llu %u", &heads, &kv, &dim, &page, &limit, &n) == 6) {
+        sr::SeqMeta m[64] = {};
+        for (unsigned i = 0; i < n; ++i) {
+            if (scanf("%u %u", &m[i].ctx, &m[i].rows) != 2) return 1;
+        }
+        const sr::SplitPlan p = sr::split_plan({heads, kv, dim, page, 256}, m, (int)n, limit);
+        printf("%u %llu %u %u %d\n", p.part_keys, (unsigned long long)p.record_bytes,
+               p.rows_per_slice, p.records_per_part, (int)p.direct);
+    }
+}
+"""
+
+
+@pytest.fixture(scope="session")
+def plans(tmp_path_factory):
+    where = tmp_path_factory.mktemp("plan")
+    (where / "plan.cpp").write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", f"-I{ROOT / 'include'}",
+                    f"-I{ROOT / 'safetyraise-lmengine_amd' / 'csrc'}", str(where / "plan.cpp"),
+                    "-o", str(where / "plan")], check=True)
+
+    def ask(calls):
+        """calls: (heads, kv_heads, head_dim, page_tokens, limit, [(ctx, rows), ...]), the
+        sequences in descending order of their keys."""
+        text = "".join(f"{h} {kv} {d} {p} {lim} {len(seqs)} "
+                       + " ".join(f"{c} {r}" for c, r in seqs) + "\n"
+                       for h, kv, d, p, lim, seqs in calls)
+        out = subprocess.run([str(where / "plan")], input=text, capture_output=True, text=True,
+                             check=True).stdout
+        return [dict(zip(("part", "bytes", "rows_per_slice", "per_part", "direct"),
+                         map(int, line.split()))) for line in out.splitlines()]
+
+    return ask
+
+
+def up(x, unit):
+    return -(-x // unit)
+
+
+def rope_bytes(dim, seqs):
+    return up(sum(r for _, r in seqs) * (dim // 2) * 8, 256) * 256
+
+
+def one_workgroup_per_cu(heads, kv, dim, page, seqs):
+    """Record bytes of the plan with one workgroup per CU over the whole call: partitions of
+    an equal share of every slice's keys, at least 256."""
+    group, most = heads // kv, max(r for _, r in seqs)
+    wide = dim <= 128 and most * group > 64
+    slices = up(most, (128 if wide else 64) // group)
+    part = up(sum(c + r for c, r in seqs) * kv * slices, CUS)
+    part = min(max(256, up(part, 64) * 64), 2046 * page // 64 * 64)
+    per_part = 2 if dim <= 128 and not wide else 1
+    return sum(up(c + r, part) * r for c, r in seqs) * per_part * heads * (dim + 4) * 4
+
+
+def batch(rng):
+    heads, kv, dim = rng.choice([(64, 8, 128), (32, 8, 128), (16, 2, 256), (14, 2, 64), (8, 8, 128)])
+    seqs = [(int(2 ** rng.uniform(0, 17)), rng.randint(2, 15)) for _ in range(rng.randint(1, 64))]
+    if rng.random() < 0.3:
+        seqs = [seqs[0]] * len(seqs)
+    return heads, kv, dim, rng.choice([16, 64, 256]), sorted(seqs, key=sum, reverse=True)
+
+
+def test_draft_rows_fit_the_fixed_scratch_wherever_one_workgroup_per_cu_does(plans):
+    rng = random.Random(5)
+    calls = [(64, 8, 128, 16, [(16384, 8)] * 64), (64, 8, 128, 16, [(25669, 8)] * 18),
+             (16, 2, 256, 16, [(68790, 8)] * 46)] + [batch(rng) for _ in range(3000)]
+    limits = [max(0, REGION - rope_bytes(d, s)) for _, _, d, _, s in calls]
+    got = plans([(*c[:4], lim, c[4]) for c, lim in zip(calls, limits)])
+    assert len(got) == len(calls)
+    fitted = 0
+    for c, lim, p in zip(calls, limits, got):
+        if one_workgroup_per_cu(*c) <= lim:
+            fitted += 1
+            assert p["bytes"] <= lim, (c, lim, p)
+    assert fitted > 2000
+
+
+def test_plans_are_whole_and_a_limit_only_enlarges_partitions(plans):
+    rng = random.Random(6)
+    calls = [batch(rng) for _ in range(1000)]
+    free = plans([(*c[:4], 2 ** 63, c[4]) for c in calls])
+    tight = plans([(*c[:4], p["bytes"] // 2, c[4]) for c, p in zip(calls, free)])
+    for (heads, kv, dim, page, seqs), p, q in zip(calls, free, tight):
+        for plan in (p, q):
+            part = plan["part"]
+            assert part % 64 == 0 and part >= 64
+            # a partition starting mid-page touches at most 2048 pages
+            assert up(part, page) + 1 <= 2048
+            longest = sum(seqs[0])
+            assert plan["direct"] == (plan["per_part"] == 1 and longest <= part)
+            records = sum(up(c + r, part) * r for c, r in seqs) * plan["per_part"]
+            assert plan["bytes"] == (0 if plan["direct"] else records * heads * (dim + 4) * 4)
+        if q["bytes"] <= p["bytes"] // 2:
+            assert q["part"] >= p["part"]

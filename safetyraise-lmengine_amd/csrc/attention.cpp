@@ -49,9 +49,6 @@ void *grow_rope(void *user, size_t bytes) {
     return ctx->rope_scratch.ptr;
 }
 
-// most scratch that prefill rows take for the split-K form's records
-constexpr uint64_t kSplitRecordBytes = 256ull << 20;
-
 // One launch of the decode kernels over up to kMetaPerLaunch sequences, each
 // contributing the row `row0` at cache length `ctx`.
 int32_t run_decode_pack(Ctx *ctx, const AttnLaunch &a, const std::vector<SeqMeta> &pack,
@@ -68,11 +65,10 @@ int32_t run_decode_pack(Ctx *ctx, const AttnLaunch &a, const std::vector<SeqMeta
 // The first pack launched carries the call's inline page-table entries
 // (AttnLaunch::tbl_*); they are cleared once a launch has taken them.
 int32_t run_verify_pack(Ctx *ctx, AttnLaunch &a, const std::vector<SeqMeta> &pack,
-                        const AttnScratch &scratch, void *rope, uint64_t record_limit,
-                        bool strict) {
+                        const AttnScratch &scratch, void *rope, uint64_t record_limit) {
     DecodePlanInput plan{ctx->num_cus, scratch.partials, scratch.user};
-    const hipError_t e = launch_attn_verify(ctx->stream, a, pack.data(), (int)pack.size(), rope, plan,
-                                            record_limit, strict);
+    const hipError_t e =
+        launch_attn_verify(ctx->stream, a, pack.data(), (int)pack.size(), rope, plan, record_limit);
     if (e == hipErrorOutOfMemory) return kNoMemory;  // (nothing was launched)
     a.tbl_n = 0;
     if (e != hipSuccess) return hip_fail(ctx, e, "verify attention launch");
@@ -104,6 +100,41 @@ int32_t run_prefill_pack(Ctx *ctx, AttnLaunch &a, const std::vector<SeqMeta> &pa
     a.tbl_n = 0;
     if (e != hipSuccess) return hip_fail(ctx, e, "prefill attention launch");
     return kOk;
+}
+
+// Prefill rows through the split-K kernel.  A pack whose records would not keep
+// to the limit (rows by the hundred at contexts of several partitions, which a
+// small page holds short) is cut: into two packs, or one sequence's rows into
+// two launches, the second of which attends to the first's rows.  Where there
+// is no memory for the records, and for a few rows that do not fit on their
+// own, the prefill kernels run instead.
+int32_t run_split_pack(Ctx *ctx, AttnLaunch &a, const std::vector<SeqMeta> &pack,
+                       const AttnScratch &scratch, void *rope, uint64_t record_limit) {
+    if (!split_fits(a, pack.data(), (int)pack.size(), ctx->num_cus, record_limit)) {
+        const SeqMeta &m = pack[0];
+        std::vector<SeqMeta> first, second;
+        if (pack.size() > 1) {
+            const auto middle = pack.begin() + (ptrdiff_t)(pack.size() / 2);
+            first.assign(pack.begin(), middle);
+            second.assign(middle, pack.end());
+        } else if (m.rows >= 2 * kPrefillMinRows) {
+            const uint32_t half = m.rows / 2;
+            first = second = pack;
+            first[0].rows = half;
+            second[0].ctx += half;
+            second[0].row0 += half;
+            second[0].rows -= half;
+        } else {
+            return run_prefill_pack(ctx, a, pack, rope);
+        }
+        const int32_t st = run_split_pack(ctx, a, first, scratch, rope, record_limit);
+        return st != kOk ? st : run_split_pack(ctx, a, second, scratch, rope, record_limit);
+    }
+    const int32_t st = run_verify_pack(ctx, a, pack, scratch, rope, record_limit);
+    if (st != kNoMemory) return st;
+    (void)hipGetLastError();
+    ctx->error.clear();
+    return run_prefill_pack(ctx, a, pack, rope);
 }
 
 // A call at a head width the tuned kernels are not built for: every row of
@@ -376,12 +407,10 @@ int32_t attention_forward_impl(Ctx *ctx, const safetyraise_kernel_attention_args
             return A.seq_rows[i] < kPrefillMinRows && verify_supported(L, A.seq_rows[i]);
         },
         [&](const std::vector<SeqMeta> &pack) {
-            return run_verify_pack(ctx, L, pack, scratch, rope, record_limit, false);
+            return run_verify_pack(ctx, L, pack, scratch, rope, record_limit);
         });
     if (pst != kOk) return pst;
-    // Prefill rows whose row blocks would leave most of the CUs idle take it
-    // too, or the prefill kernels if there is no memory for its records or
-    // they are many (rows by the thousand over pages of a few tokens).
+    // Prefill rows whose row blocks would leave most of the CUs idle take it too.
     std::vector<SeqMeta> candidates;
     std::vector<uint8_t> split(A.num_seqs, 0);
     for (uint32_t i = 0; prefill_ok && i < A.num_seqs; ++i) {
@@ -395,12 +424,7 @@ int32_t attention_forward_impl(Ctx *ctx, const safetyraise_kernel_attention_args
         split_preferred(L, candidates.data(), (int)candidates.size(), ctx->num_cus);
     pst = run_packs([&](uint32_t i) { return preferred && split[i]; },
                     [&](const std::vector<SeqMeta> &pack) {
-                        const int32_t st =
-                            run_verify_pack(ctx, L, pack, scratch, rope, kSplitRecordBytes, true);
-                        if (st != kNoMemory) return st;
-                        (void)hipGetLastError();
-                        ctx->error.clear();
-                        return run_prefill_pack(ctx, L, pack, rope);
+                        return run_split_pack(ctx, L, pack, scratch, rope, record_limit);
                     });
     if (pst != kOk) return pst;
     pst = run_packs(

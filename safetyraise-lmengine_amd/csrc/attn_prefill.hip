@@ -2991,9 +2991,29 @@ bool verify_supported(const AttnLaunch &a, uint32_t rows) {
     return prefill_supported(a) && rows >= 2;
 }
 
+namespace {
+// The plan of a launch, and its sequences in order of their keys: the longest
+// workgroups first.
+SplitPlan sorted_plan(const AttnLaunch &a, const SeqMeta *seqs, int nseq, int num_cus,
+                      uint64_t record_limit, SeqMeta (&sorted)[kMetaPerLaunch]) {
+    std::copy(seqs, seqs + nseq, sorted);
+    std::stable_sort(sorted, sorted + nseq, [](const SeqMeta &x, const SeqMeta &y) {
+        return (uint64_t)x.ctx + x.rows > (uint64_t)y.ctx + y.rows;
+    });
+    return split_plan({a.heads, a.kv_heads * a.kv_rep, a.head_dim, a.pool->page_tokens, num_cus},
+                      sorted, nseq, record_limit);
+}
+}  // namespace
+
+bool split_fits(const AttnLaunch &a, const SeqMeta *seqs, int nseq, int num_cus,
+                uint64_t record_limit) {
+    SeqMeta sorted[kMetaPerLaunch];
+    return sorted_plan(a, seqs, nseq, num_cus, record_limit, sorted).record_bytes <= record_limit;
+}
+
 hipError_t launch_attn_verify(hipStream_t stream, const AttnLaunch &a, const SeqMeta *seqs,
                               int nseq, void *rope_scratch, const DecodePlanInput &in,
-                              uint64_t record_limit, bool strict) {
+                              uint64_t record_limit) {
     if (nseq <= 0 || nseq > kMetaPerLaunch || rope_scratch == nullptr) return hipErrorInvalidValue;
     const uint32_t kvv = a.kv_heads * a.kv_rep;  // KV heads of the grid
     VerifyParams vp{};
@@ -3004,23 +3024,14 @@ hipError_t launch_attn_verify(hipStream_t stream, const AttnLaunch &a, const Seq
         if (!verify_supported(a, seqs[i].rows)) return hipErrorInvalidValue;
         max_rows = std::max(max_rows, seqs[i].rows);
     }
-    // the longest workgroups first: sequences in order of their keys
     SeqMeta sorted[kMetaPerLaunch];
-    std::copy(seqs, seqs + nseq, sorted);
-    std::stable_sort(sorted, sorted + nseq, [](const SeqMeta &x, const SeqMeta &y) {
-        return (uint64_t)x.ctx + x.rows > (uint64_t)y.ctx + y.rows;
-    });
-    const SplitPlan plan = split_plan({a.heads, kvv, a.head_dim, a.pool->page_tokens, in.num_cus},
-                                      sorted, nseq, record_limit);
+    const SplitPlan plan = sorted_plan(a, seqs, nseq, in.num_cus, record_limit, sorted);
     const bool all_tiles = plan.all_tiles;
     vp.rows_per_slice = plan.rows_per_slice;
     vp.part_keys = plan.part_keys;
     vp.direct = plan.direct;
     if (!plan.direct) {
-        // (draft rows have no other kernel but the row-serial one)
-        vp.partials = plan.record_bytes <= record_limit || !strict
-                          ? in.reserve_partials(plan.record_bytes)
-                          : nullptr;
+        vp.partials = in.reserve_partials(plan.record_bytes);
         if (vp.partials == nullptr) return hipErrorOutOfMemory;
     }
     uint32_t blocks = 0, waves = 0;

@@ -288,8 +288,8 @@ struct AttnLaunch {
 constexpr uint32_t kInlineTable = 64;
 
 // Bytes of the no-allocation entry point's scratch, which a call's RoPE table and
-// its split-K records share.  The plans of draft rows keep to what the table
-// leaves of it, in both entry points.
+// its split-K records share.  The records' plans keep to what the table leaves of
+// it in both entry points, so that both run the same kernels.
 constexpr size_t kAttnScratchBytes = (size_t)64 << 20;
 constexpr size_t kAttnScratchAlign = 256;
 
@@ -335,21 +335,22 @@ hipError_t launch_attn_prefill(hipStream_t s, const AttnLaunch &a, const SeqMeta
 // Multi-row split-K attention (MTP verify rows, and prefill rows that would
 // leave most of the chip idle): key partitions with MFMA inner products, then
 // a combine pass.  The plan keeps its partial records to record_limit bytes
-// where it can (attn_plan.hpp); a strict call that cannot, and one whose records
-// in.reserve_partials does not provide, launches nothing (hipErrorOutOfMemory).
+// where it can (split_fits, attn_plan.hpp); a call whose records
+// in.reserve_partials does not provide launches nothing (hipErrorOutOfMemory).
 bool verify_supported(const AttnLaunch &a, uint32_t rows);
 // Whether a sequence of prefill rows may take it, and whether a call's such
 // sequences should.
 bool split_candidate(const AttnLaunch &a, uint32_t ctx, uint32_t rows);
 bool split_preferred(const AttnLaunch &a, const SeqMeta *seqs, int nseq, int num_cus);
+bool split_fits(const AttnLaunch &a, const SeqMeta *seqs, int nseq, int num_cus,
+                uint64_t record_limit);
 // Head widths other than 64, 128 and 256 (up to kGenericMaxHeadDim): every
 // row of the call through the plain f32 kernels of attn_generic.hip (append,
 // then attention); a.rope_denom must hold the rotary pairs' denominators.
 bool generic_head_dim(uint32_t head_dim);
 hipError_t launch_attn_generic(hipStream_t s, const AttnLaunch &a, const SeqMeta *seqs, int nseq);
 hipError_t launch_attn_verify(hipStream_t s, const AttnLaunch &a, const SeqMeta *seqs, int nseq,
-                              void *rope_scratch, const DecodePlanInput &in, uint64_t record_limit,
-                              bool strict);
+                              void *rope_scratch, const DecodePlanInput &in, uint64_t record_limit);
 
 struct GdnLaunch {
     const safetyraise_kernel_gdn_pool *pool;

@@ -103,6 +103,22 @@ def test_many_long_sequences_of_draft_rows_fit(pkg, backend, torch_mod):
     pool.destroy()
 
 
+def test_prefill_rows_whose_records_exceed_the_region(pkg, backend, torch_mod):
+    # partitions end at 32704 keys here (the page ids of 16-token pages), so the
+    # long sequence's 400 rows take five records each, 68 MB: its rows run in
+    # two launches, in both entry points.  64-token pages let one launch do.
+    outs = []
+    for page in (16, 64):
+        pool = pkg.KvCache(backend, 8, 128, page, 2 * 134000 // page, 131584, 4)
+        a, b = one_call(pkg, backend, torch_mod, pool, [131072, 2000], [400, 40], 4, heads=64)
+        assert np.isfinite(a).all()
+        assert np.array_equal(a, b)
+        outs.append(a)
+        pool.destroy()
+    err = np.abs(outs[0] - outs[1])
+    assert (err <= 2e-3 + 1e-2 * np.abs(outs[1])).all(), err.max()
+
+
 def test_noalloc_rejects_host_pointers_and_oversized_calls(pkg, backend, torch_mod):
     torch = torch_mod
     P = pkg.plugin

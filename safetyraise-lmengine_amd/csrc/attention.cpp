@@ -15,6 +15,7 @@
 #include <cstring>
 #include <vector>
 
+#include "attn_plan.hpp"
 #include "sr_internal.hpp"
 
 namespace sr {
@@ -36,8 +37,16 @@ struct Region {
 // The default scratch: context-owned buffers grown on demand.
 float *grow_partials(void *user, size_t bytes) {
     Ctx *ctx = (Ctx *)user;
-    if (ensure_buffer(ctx, ctx->partials, bytes, false) != kOk) {
-        return nullptr;
+    if (bytes > ctx->partials.bytes) {
+        // growing waits for the stream and frees the old buffer
+        const size_t want = grown_bytes(ctx->partials.bytes, bytes);
+        int32_t st = ensure_buffer(ctx, ctx->partials, want, false);
+        if (st == kNoMemory && want > bytes) {
+            (void)hipGetLastError();
+            st = ensure_buffer(ctx, ctx->partials, bytes, false);
+            if (st == kOk) ctx->error.clear();
+        }
+        if (st != kOk) return nullptr;
     }
     return (float *)ctx->partials.ptr;
 }

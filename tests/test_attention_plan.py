@@ -15,8 +15,13 @@ REGION = 64 << 20  # the no-allocation entry point's scratch
 
 PROGRAM = r"""
 #include <cstdio>
+#include <cstdlib>
 #include "attn_plan.hpp"
-int main() {
+int main(int argc, char **argv) {
+    if (argc == 3) {
+        printf("%zu\n", sr::grown_bytes(strtoull(argv[1], nullptr, 10), strtoull(argv[2], nullptr, 10)));
+        return 0;
+    }
     unsigned heads, kv, dim, page, n;
     unsigned long long limit;
     while (scanf("%u %u %u %u %llu %u", &heads, &kv, &dim, &page, &limit, &n) == 6) {
@@ -52,6 +57,9 @@ def plans(tmp_path_factory):
         return [dict(zip(("part", "bytes", "rows_per_slice", "per_part", "direct"),
                          map(int, line.split()))) for line in out.splitlines()]
 
+    ask.grown = lambda have, need: int(subprocess.run(
+        [str(where / "plan"), str(have), str(need)], capture_output=True, text=True,
+        check=True).stdout)
     return ask
 
 
@@ -115,3 +123,20 @@ def test_plans_are_whole_and_a_limit_only_enlarges_partitions(plans):
             assert plan["bytes"] == (0 if plan["direct"] else records * heads * (dim + 4) * 4)
         if q["bytes"] <= p["bytes"] // 2:
             assert q["part"] >= p["part"]
+
+
+@pytest.mark.parametrize("heads,kv,dim", [(32, 8, 128), (16, 2, 256)])
+def test_a_prompt_in_small_chunks_replaces_its_records_a_few_times(plans, heads, kv, dim):
+    # 32-row chunks up to 32 K keys: each replacement waits for the stream
+    chunks = [(heads, kv, dim, 64, REGION, [(c, 32)]) for c in range(0, 32768, 32)]
+    needs = sorted({p["bytes"] for p in plans(chunks)})
+    assert len(needs) >= 16
+    have, grown = 0, 0
+    for need in needs:
+        if need > have:
+            have = up(plans.grown(have, need), 1 << 20) << 20
+            grown += 1
+            assert need <= have <= max(need + (1 << 20), REGION)
+    assert grown <= 3
+    # a single need above the usual limit is met and no more
+    assert plans.grown(REGION, REGION + 5) == REGION + 5

@@ -368,6 +368,52 @@ def test_routes_of_many_rows(backend, rng, torch_mod, rows, cols, out):
             prepared.destroy()
 
 
+def check_call(backend, rng, torch, rows, cols, out):
+    """One device call of random and one of integer inputs; the kernels that ran."""
+    ran = set()
+    for integers in (False, True):
+        if integers:
+            x = rng.integers(-8, 9, size=(rows, cols)).astype(np.float32)
+            w = rng.integers(-8, 9, size=(out, cols)).astype(np.float32)
+        else:
+            x = (2 * rng.standard_normal((rows, cols))).astype(np.float32)
+            w = rng.standard_normal((out, cols)).astype(np.float32)
+        bits = weight_bits(w, BF16)
+        wide = torch.from_numpy(widened(bits, BF16)).cuda()
+        x64 = torch.from_numpy(x).cuda().double()
+        ref = x64 @ wide.T
+        bound = 1e-5 * (x64.abs() @ wide.abs().T) + 1e-4 * ref.abs()
+        prepared = backend.create_weight(bits, BF16)
+        try:
+            dx = torch.from_numpy(x).cuda()
+            dy = torch.full((rows, out), float("nan"), device="cuda")
+            torch.cuda.synchronize()
+            backend.timing(True)
+            try:
+                device_call(backend, prepared, dx, dy, rows, cols, out)
+                backend.synchronize()
+                ran |= set(backend.kernel_times())
+            finally:
+                backend.timing(False)
+            if integers:
+                assert torch.equal(dy.double(), ref), (rows, cols, out)
+            else:
+                assert bool(((dy.double() - ref).abs() <= bound).all()), (rows, cols, out)
+        finally:
+            prepared.destroy()
+    return ran
+
+
+# short columns, rows and outputs on and off the tiles: 128 and more output tiles
+# of 128 x 128, and one per CU at 64 columns
+@pytest.mark.parametrize("rows,cols,out,kernel", [(3840, 64, 1024, "linear_rows_kernel"),
+                                                  (64, 128, 16400, "linear_rows_kernel"),
+                                                  (237, 128, 9073, "linear_rows_kernel"),
+                                                  (1528, 64, 2752, "linear_gemm_wide_kernel")])
+def test_many_rows_of_few_columns(backend, rng, torch_mod, rows, cols, out, kernel):
+    assert kernel in check_call(backend, rng, torch_mod, rows, cols, out)
+
+
 def test_captured_call_keeps_no_scratch(backend, rng, torch_mod):
     # a call whose K split is optional is captured without it: its replays
     # stay right after a larger call has replaced the context's scratch

@@ -1,0 +1,75 @@
+"""Which kernels a linear call takes (csrc/linear_plan.hpp), without a GPU.
+
+linear_choice is host code: a small program compiled from the header answers
+for shapes written to its standard input.
+"""
+import random
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+CUS = 256
+F32, F16, BF16 = 1, 2, 3
+TILE, PAIR, ROWS, WIDE = range(4)
+ANY = 2 ** 64 - 1  # as much scratch as a call likes
+
+PROGRAM = r"""
+#include <cstdio>
+#include "linear_plan.hpp"
+int main() {
+    unsigned m, n, k, dtype, aligned;
+    unsigned long long scratch;
+    while (scanf("%u %u %u %u %u %llu", &m, &n, &k, &dtype, &aligned, &scratch) == 6) {
+        const sr::LinChoice c =
+            sr::linear_choice(m, n, k, dtype, 256, aligned != 0, (size_t)scratch);
+        printf("%d %u %zu\n", (int)c.route, c.splits, c.scratch);
+    }
+}
+"""
+
+
+@pytest.fixture(scope="session")
+def choose(tmp_path_factory):
+    where = tmp_path_factory.mktemp("plan")
+    (where / "plan.cpp").write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", f"-I{ROOT / 'include'}",
+                    f"-I{ROOT / 'safetyraise-lmengine_amd' / 'csrc'}", str(where / "plan.cpp"),
+                    "-o", str(where / "plan")], check=True)
+
+    def ask(shapes, scratch=ANY, dtype=BF16, aligned=True):
+        """(route, K splits, scratch bytes) of each (rows, outputs, columns)."""
+        text = "".join(f"{m} {n} {k} {dtype} {int(aligned)} {scratch}\n" for m, n, k in shapes)
+        out = subprocess.run([str(where / "plan")], input=text, capture_output=True, text=True,
+                             check=True).stdout
+        return [tuple(map(int, line.split())) for line in out.splitlines()]
+
+    return ask
+
+
+def up(x, unit):
+    return -(-x // unit)
+
+
+def shapes(seed, count, cols=64):
+    """(rows, outputs, columns), columns a multiple of `cols`."""
+    rng = random.Random(seed)
+
+    def spread(lo, hi):
+        return int(2 ** rng.uniform(lo, hi))
+
+    return [(spread(0, 17), spread(4, 14), up(spread(4, 14), cols) * cols) for _ in range(count)]
+
+
+def tiles(m, n):
+    return up(m, 128) * up(n, 128)
+
+
+def test_short_columns_do_not_send_many_rows_to_the_row_tiles(choose):
+    # a 128 x 128 output tile for every other CU, however little there is to add up
+    many = [s for s in shapes(1, 6000) if s[0] >= 64 and 2 * tiles(s[0], s[1]) >= CUS]
+    many += [(3840, 1024, 64), (237, 9088, 128), (64, 16384, 64), (17384, 64, 576)]
+    assert len(many) > 1000
+    for shape, (route, _, _) in zip(many, choose(many)):
+        assert route in (ROWS, WIDE), shape

@@ -22,6 +22,7 @@ constexpr int kRowsBN = kLinTile * kRowsWaves;  // 128 outputs per workgroup
 
 // linear_gemm_wide_kernel
 constexpr uint32_t kGemmK = 64;  // K granularity: stages in pairs
+constexpr uint32_t kWideMinOutputs = 2048;
 constexpr int kWideWM = 2, kWideWN = 2;           // waves over rows, over outputs
 constexpr int kWideRT = 4, kWideCT = 4;           // 16 x 16 tiles per wave
 constexpr int kWideBM = 16 * kWideRT * kWideWM;   // 128 rows per workgroup
@@ -123,10 +124,13 @@ inline LinChoice linear_choice(uint32_t M, uint32_t N, uint32_t K, uint32_t dtyp
     // 4096 (1536 tiles) 476 against 540 with kRows, of 4096 x 4096 (512) 185 / 210;
     // with fewer kRows, which can split K: 1500 rows of it (384) 173 / 160, 1024
     // (256) 160 / 106; but one tile per CU where a K block or two is all there is
-    // (1528 rows of 2752 x 64, 264 tiles: 11.7 / 13.4)
+    // (1528 rows of 2752 x 64, 264 tiles: 11.7 / 13.4).  Not with fewer outputs than
+    // 2048 (k/v projections): there kRows is the faster one (7168 rows of 1024 x
+    // 4096 246 / 210, of 1024 x 12288 727 / 628), and kWide's one chain of all three
+    // parts of x rounds more (relative error at K = 4096 7.0e-7 / 1.4e-7).
     const uint64_t tiles = (uint64_t)((M + kWideBM - 1) / kWideBM) * ((N + kWideBN - 1) / kWideBN);
-    if (M > 64 && K % kGemmK == 0 && K > 0 && 4 * tiles >= (K <= kGemmK ? 4 : 7) * cus &&
-        split_x_bytes(M, K) <= scratch) {
+    if (M > 64 && N >= kWideMinOutputs && K % kGemmK == 0 && K > 0 &&
+        4 * tiles >= (K <= kGemmK ? 4 : 7) * cus && split_x_bytes(M, K) <= scratch) {
         return {LinRoute::kWide, 1, split_x_bytes(M, K)};
     }
     const bool pair = M <= 2 * kLinTile;

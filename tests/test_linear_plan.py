@@ -73,3 +73,12 @@ def test_short_columns_do_not_send_many_rows_to_the_row_tiles(choose):
     assert len(many) > 1000
     for shape, (route, _, _) in zip(many, choose(many)):
         assert route in (ROWS, WIDE), shape
+
+
+def test_calls_of_few_outputs_sum_the_parts_of_x_in_two_chains(choose):
+    # the tiled product adds the three parts of x in one chain: not below 2048 outputs
+    few = [s for s in shapes(2, 6000) if s[1] < 2048 and 4 * tiles(s[0], s[1]) >= 7 * CUS]
+    few += [(7168, 1024, 4096), (3840, 1920, 12288), (60000, 1024, 64)]
+    assert len(few) > 200
+    for shape, (route, _, _) in zip(few, choose(few)):
+        assert route == ROWS, shape

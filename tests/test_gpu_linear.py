@@ -414,6 +414,43 @@ def test_many_rows_of_few_columns(backend, rng, torch_mod, rows, cols, out, kern
     assert kernel in check_call(backend, rng, torch_mod, rows, cols, out)
 
 
+# rows, columns and outputs where 16-row calls sum K in eight ranges
+@pytest.mark.parametrize("rows,cols,out", [(1024, 1024, 1024), (512, 2048, 2048)])
+def test_many_rows_sum_as_precisely_as_few(backend, torch_mod, rows, cols, out):
+    # the same inputs in one call (linear_rows_kernel) and 16 rows at a time
+    # (linear_kernel): the one call's error against 64 bits is no larger but for
+    # the order in which the eight ranges' totals meet.  With partial sums of
+    # variance proportional to their length, and a rounding of each proportional
+    # to its size, chains of 4 products and their join give 3.25 eighths' worth
+    # of rounding in both; eight totals one after another give 35/8 more, four
+    # and four 3.25: sqrt(7.6 / 6.5) = 1.085
+    torch = torch_mod
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows + cols)
+    x = torch.randn((rows, cols), generator=gen, device="cuda")
+    w = torch.randn((out, cols), generator=gen, device="cuda").bfloat16()
+    prepared = backend.create_weight(w.view(torch.uint16).cpu().numpy(), BF16)
+    ref = x.double() @ w.double().T
+    errors, kernels = [], []
+    try:
+        for step in (rows, 16):
+            dy = torch.full((rows, out), float("nan"), device="cuda")
+            torch.cuda.synchronize()
+            backend.timing(True)
+            try:
+                for r in range(0, rows, step):
+                    device_call(backend, prepared, x[r:], dy[r:], step, cols, out)
+                backend.synchronize()
+                kernels.append(" ".join(backend.kernel_times()))
+            finally:
+                backend.timing(False)
+            errors.append(float((dy.double() - ref).norm() / ref.norm()))
+    finally:
+        prepared.destroy()
+    assert "linear_rows_kernel" in kernels[0] and "linear_kernel" in kernels[1]
+    assert errors[0] <= 1.1 * errors[1], errors
+
+
 def test_captured_call_keeps_no_scratch(backend, rng, torch_mod):
     # a call whose K split is optional is captured without it: its replays
     # stay right after a larger call has replaced the context's scratch

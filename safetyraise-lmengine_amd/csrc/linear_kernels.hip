@@ -779,13 +779,9 @@ hipError_t linear_pack_bf16(hipStream_t stream, const void *src, void *dst, uint
     return hipGetLastError();
 }
 
-size_t linear_scratch_bytes(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus) {
-    return linear_choice(M, N, K, dtype, num_cus, true, SIZE_MAX).scratch;
-}
-
-bool linear_scratch_required(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus) {
-    const LinChoice c = linear_choice(M, N, K, dtype, num_cus, true, SIZE_MAX);
-    return c.scratch > 0 && c.route != LinRoute::kRows;
+size_t linear_scratch_bytes(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus,
+                            bool x_aligned, bool split_rows) {
+    return linear_choice(M, N, K, dtype, num_cus, x_aligned, SIZE_MAX, split_rows).scratch;
 }
 
 // y = 0 for calls with no inputs per output (K = 0): the sum over an empty
@@ -811,8 +807,8 @@ hipError_t launch_linear_input(hipStream_t stream, const float *src, float *dst,
 }
 
 hipError_t launch_linear(hipStream_t stream, const float *x, const void *w, uint32_t dtype,
-                         float *y, uint32_t M, uint32_t N, uint32_t K, float *scratch,
-                         size_t scratch_bytes, int num_cus) {
+                         float *y, uint32_t M, uint32_t N, uint32_t K, const LinScratch &scratch,
+                         int num_cus) {
     if (M == 0 || N == 0) return hipSuccess;
     if (K == 0) {
         const uint64_t count = (uint64_t)M * N;
@@ -829,20 +825,18 @@ hipError_t launch_linear(hipStream_t stream, const float *x, const void *w, uint
         for (uint32_t r0 = 0; r0 < M; r0 += per) {
             const uint32_t m = std::min(per, M - r0);
             const hipError_t e = launch_linear(stream, x + (size_t)r0 * K, w, dtype,
-                                               y + (size_t)r0 * N, m, N, K, nullptr, 0, num_cus);
+                                               y + (size_t)r0 * N, m, N, K, LinScratch{}, num_cus);
             if (e != hipSuccess) return e;
         }
         return hipSuccess;
     }
     const bool x_aligned = ((uintptr_t)x & 15u) == 0;
     const LinChoice choice = linear_choice(M, N, K, dtype, num_cus, x_aligned,
-                                           scratch != nullptr ? scratch_bytes : 0);
-    if (choice.scratch > 0 && (scratch == nullptr || choice.scratch > scratch_bytes)) {
-        return hipErrorInvalidValue;
-    }
+                                           scratch.ptr != nullptr ? scratch.bytes : 0,
+                                           scratch.split_rows);
     if (choice.route == LinRoute::kWide) {
         // x split once into scratch, then the tiled product
-        uint16_t *xs = (uint16_t *)scratch;
+        uint16_t *xs = (uint16_t *)scratch.ptr;
         const uint64_t chunks = (uint64_t)((M + kLinTile - 1) / kLinTile) * (K / kLinBlock) * 64;
         const dim3 sgrid((uint32_t)((chunks + 255) / 256));
         if (x_aligned) {
@@ -858,7 +852,7 @@ hipError_t launch_linear(hipStream_t stream, const float *x, const void *w, uint
         return hipGetLastError();
     }
     const uint32_t splits = choice.splits;
-    float *dst = splits > 1 ? scratch : y;
+    float *dst = splits > 1 ? scratch.ptr : y;
     if (choice.route == LinRoute::kRows) {
         const bool pair = M <= 2 * kLinTile;
         const uint32_t rows = pair ? 2 * kLinTile : 4 * kLinTile;
@@ -888,7 +882,7 @@ hipError_t launch_linear(hipStream_t stream, const float *x, const void *w, uint
                       0, stream, x, w, y, M, N, K);
         }
     } else {
-        const LinPlan plan = linear_plan(M, N, K, dtype, num_cus);
+        const LinPlan &plan = choice.plan;
         switch (dtype) {
             case SAFETYRAISE_KERNEL_DTYPE_F32:
                 launch_dt_plan<SAFETYRAISE_KERNEL_DTYPE_F32>(stream, x, w, dst, M, N, K, plan, num_cus);
@@ -908,7 +902,7 @@ hipError_t launch_linear(hipStream_t stream, const float *x, const void *w, uint
         // the CUs, kRows checks it)
         const uint32_t count = M * N;
         SR_LAUNCH("linear_split_sum_kernel", linear_split_sum_kernel, dim3((count + 255) / 256),
-                  dim3(256), 0, stream, scratch, y, count, splits);
+                  dim3(256), 0, stream, scratch.ptr, y, count, splits);
     }
     return hipGetLastError();
 }

@@ -37,19 +37,21 @@ constexpr int kWideBN = 16 * kWideCT * kWideWN;   // 128 outputs per workgroup
 // workgroups cover 7/8 of the CUs without a split, or with one when the
 // weight is large enough (kLinSplitTElems) that the second kernel's few
 // microseconds are small against the stream; otherwise one tile per wave
-// and 4 waves, K split until the CUs are covered.
+// and 4 waves, K split until the CUs are covered.  max_splits: what the
+// scratch for partial sums holds.
 constexpr uint64_t kLinSplitTElems = (uint64_t)32 << 20;
 struct LinPlan {
     uint32_t T, W, splits;
 };
-inline LinPlan linear_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus) {
+inline LinPlan linear_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus,
+                           uint64_t max_splits = kLinMaxSplits) {
     const uint64_t cus = (uint64_t)(num_cus > 0 ? num_cus : 1);
     const uint64_t mt = (M + kLinTile - 1) / kLinTile;
     auto splits_for = [&](uint64_t tiles) -> uint32_t {
         if (tiles == 0 || tiles >= cus) return 1;
         uint64_t s = cus / tiles;
         s = std::min<uint64_t>(s, K / kLinMinSplitK);
-        s = std::min<uint64_t>(s, kLinMaxSplits);
+        s = std::min<uint64_t>(s, std::min<uint64_t>(max_splits, kLinMaxSplits));
         return s < 1 ? 1u : (uint32_t)s;
     };
     const uint32_t t_max = dtype == SAFETYRAISE_KERNEL_DTYPE_BF16 ? 4 : 3;
@@ -76,7 +78,8 @@ enum class LinRoute {
 };
 struct LinChoice {
     LinRoute route;
-    uint32_t splits;  // of K over grid z (kRows)
+    LinPlan plan;     // kTile's
+    uint32_t splits;  // of K over grid z (kTile, kRows)
     size_t scratch;   // bytes the route uses
 };
 
@@ -91,7 +94,7 @@ inline size_t split_x_bytes(uint32_t M, uint32_t K) {
 // measured split or one within 5 % of it, e.g. 512 rows of 3072 x 1024: 1
 // (17.6; 2: 25.7), 1024 of 1024 x 4096: 4 (35.1; 1: 55.4, 3: 40.3).
 inline uint32_t rows_splits(uint32_t M, uint32_t N, uint32_t units, uint32_t base, bool two_tiles,
-                     uint64_t cus, size_t scratch) {
+                            uint64_t cus, size_t scratch) {
     const double one = two_tiles ? 1.1 : 0.86, two = two_tiles ? 1.9 : 1.5;  // us per stage
     const uint64_t outputs = (uint64_t)M * N;
     uint32_t best = 1;
@@ -111,13 +114,16 @@ inline uint32_t rows_splits(uint32_t M, uint32_t N, uint32_t units, uint32_t bas
     return best;
 }
 
-// scratch: the bytes that are there (SIZE_MAX: as many as the call likes).
+// scratch: the bytes that are there (SIZE_MAX: as many as the call likes).  No
+// route needs any: without it K is not split, and kWide's calls take kRows.
+// split_rows: kRows may use it.
 inline LinChoice linear_choice(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus,
-                        bool x_aligned, size_t scratch) {
+                               bool x_aligned, size_t scratch, bool split_rows) {
     const uint64_t cus = (uint64_t)(num_cus > 0 ? num_cus : 1);
-    const LinPlan plan = linear_plan(M, N, K, dtype, num_cus);
-    const LinChoice tile = {LinRoute::kTile, plan.splits,
-                            plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0};
+    const size_t split_bytes = (size_t)M * N * sizeof(float);  // partial sums of one split
+    const LinPlan plan = linear_plan(M, N, K, dtype, num_cus, split_bytes ? scratch / split_bytes : 1);
+    const LinChoice tile = {LinRoute::kTile, plan, plan.splits,
+                            plan.splits > 1 ? plan.splits * split_bytes : 0};
     if (dtype != SAFETYRAISE_KERNEL_DTYPE_BF16 || M <= (uint32_t)kLinTile || M > kMaxRows) return tile;
     const uint64_t weight = (uint64_t)N * K, work = weight * M;
     // nearly two 128 x 128 output tiles per CU or more: 2048 rows of 12288 x
@@ -131,13 +137,13 @@ inline LinChoice linear_choice(uint32_t M, uint32_t N, uint32_t K, uint32_t dtyp
     const uint64_t tiles = (uint64_t)((M + kWideBM - 1) / kWideBM) * ((N + kWideBN - 1) / kWideBN);
     if (M > 64 && N >= kWideMinOutputs && K % kGemmK == 0 && K > 0 &&
         4 * tiles >= (K <= kGemmK ? 4 : 7) * cus && split_x_bytes(M, K) <= scratch) {
-        return {LinRoute::kWide, 1, split_x_bytes(M, K)};
+        return {LinRoute::kWide, {}, 1, split_x_bytes(M, K)};
     }
     const bool pair = M <= 2 * kLinTile;
     // 32 rows, one workgroup of three output tiles on nearly every CU: 12288 x
     // 4096 25.1 against 34.8 (kTile) and 28.2 (kRows, its best split)
     if (pair && x_aligned && K % 8 == 0 && 8 * ((uint64_t)(N + 3 * kLinTile - 1) / (3 * kLinTile)) >= 7 * cus) {
-        return {LinRoute::kPair, 1, 0};
+        return {LinRoute::kPair, {}, 1, 0};
     }
     const uint32_t stage = pair ? 4 * kLinBlock : 2 * kLinBlock;
     if (K == 0 || K % stage != 0) return tile;
@@ -167,8 +173,8 @@ inline LinChoice linear_choice(uint32_t M, uint32_t N, uint32_t K, uint32_t dtyp
     if (!pays) return tile;
     const uint32_t rows = pair ? 2 * kLinTile : 4 * kLinTile;
     const uint32_t base = ((N + kRowsBN - 1) / kRowsBN) * ((M + rows - 1) / rows);
-    const uint32_t s = rows_splits(M, N, K / stage, base, pair, cus, scratch);
-    return {LinRoute::kRows, s, s > 1 ? (size_t)s * M * N * sizeof(float) : 0};
+    const uint32_t s = rows_splits(M, N, K / stage, base, pair, cus, split_rows ? scratch : 0);
+    return {LinRoute::kRows, {}, s, s > 1 ? s * split_bytes : 0};
 }
 
 }  // namespace sr

@@ -370,32 +370,38 @@ static int32_t check_linear(Ctx *ctx, const safetyraise_kernel_weight *w, const 
     return kOk;
 }
 
-// The context's linear scratch for a call (none: nullptr and 0 bytes).  A call
-// that can do without (linear_scratch_required) goes without when the buffer
-// cannot grow, and while the stream is captured: a graph would keep the
-// buffer's address, and a later, larger call replaces the buffer.
+// The context's linear scratch for a call.  Every call can do without: it goes
+// without when the buffer cannot grow, and with what is there while the stream
+// is captured, when nothing may be allocated or waited for.  The K splits of
+// linear_rows_kernel are not captured: a graph would keep the buffer's address,
+// and a later, larger call replaces the buffer.
 static int32_t linear_scratch(Ctx *ctx, const safetyraise_kernel_weight *w, uint64_t rows,
-                              float **part, size_t *have) {
-    const uint32_t m = (uint32_t)rows, n = (uint32_t)w->rows, k = (uint32_t)w->cols;
-    const size_t bytes = linear_scratch_bytes(m, n, k, w->dtype, ctx->num_cus);
-    *part = nullptr;
-    *have = 0;
+                              const float *x, LinScratch *scratch) {
+    *scratch = LinScratch{};
+    auto bytes_for = [&](bool split_rows) {
+        return linear_scratch_bytes((uint32_t)rows, (uint32_t)w->rows, (uint32_t)w->cols, w->dtype,
+                                    ctx->num_cus, ((uintptr_t)x & 15u) == 0, split_rows);
+    };
+    size_t bytes = bytes_for(true);
     if (bytes == 0) return kOk;
-    const bool required = linear_scratch_required(m, n, k, w->dtype, ctx->num_cus);
-    if (!required) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess) (void)hipGetLastError();
-        if (capture != hipStreamCaptureStatusNone) return kOk;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess) (void)hipGetLastError();
+    if (capture != hipStreamCaptureStatusNone) {
+        scratch->split_rows = false;
+        bytes = bytes_for(false);
+        if (bytes == 0) return kOk;
     }
-    const int32_t e = ensure_buffer(ctx, ctx->linear_part, bytes, false);
-    if (e == kNoMemory && !required) {
-        (void)hipGetLastError();
-        ctx->error.clear();
-        return kOk;
+    if (bytes > ctx->linear_part.bytes && capture == hipStreamCaptureStatusNone) {
+        const int32_t e = ensure_buffer(ctx, ctx->linear_part, bytes, false);
+        if (e == kNoMemory) {
+            (void)hipGetLastError();
+            ctx->error.clear();
+            return kOk;
+        }
+        if (e != kOk) return e;
     }
-    if (e != kOk) return e;
-    *part = (float *)ctx->linear_part.ptr;
-    *have = bytes;
+    scratch->ptr = (float *)ctx->linear_part.ptr;
+    scratch->bytes = ctx->linear_part.bytes;
     return kOk;
 }
 
@@ -454,11 +460,10 @@ SAFETYRAISE_KERNEL_EXPORT int32_t safetyraise_kernel_linear(
         e = ensure_buffer(context, context->linear_out, (size_t)out_count * 4, false);
         if (e != kOk) return e;
     }
-    float *part = nullptr;
-    size_t part_bytes = 0;
-    e = linear_scratch(context, weight, input_rows, &part, &part_bytes);
-    if (e != kOk) return e;
     float *d_in = (float *)context->linear_in.ptr;
+    LinScratch scratch;
+    e = linear_scratch(context, weight, input_rows, d_in, &scratch);
+    if (e != kOk) return e;
     float *d_out = host_out != nullptr ? context->linear_host_dev + kLinearHostBytes / 4
                                        : (float *)context->linear_out.ptr;
     if (in_count != 0 && host_in != nullptr) {
@@ -470,8 +475,7 @@ SAFETYRAISE_KERNEL_EXPORT int32_t safetyraise_kernel_linear(
     }
     SR_HIP(context, launch_linear(context->stream, d_in, weight->d_data, weight->dtype, d_out,
                                   (uint32_t)input_rows, (uint32_t)weight->rows,
-                                  (uint32_t)weight->cols, part, part_bytes,
-                                  context->num_cus));
+                                  (uint32_t)weight->cols, scratch, context->num_cus));
     if (host_out == nullptr) {
         SR_HIP(context, hipMemcpyAsync(output, d_out, out_count * 4, hipMemcpyDeviceToHost,
                                        context->stream));
@@ -494,14 +498,12 @@ SAFETYRAISE_KERNEL_EXPORT int32_t safetyraise_kernel_linear_device(
                                     output_rows, output_cols, &in_count, &out_count);
     if (st != kOk) return st;
     if (out_count == 0) return kOk;
-    float *part = nullptr;
-    size_t part_bytes = 0;
-    const int32_t e = linear_scratch(context, weight, input_rows, &part, &part_bytes);
+    LinScratch scratch;
+    const int32_t e = linear_scratch(context, weight, input_rows, input, &scratch);
     if (e != kOk) return e;
     SR_HIP(context, launch_linear(context->stream, input, weight->d_data, weight->dtype, output,
                                   (uint32_t)input_rows, (uint32_t)weight->rows,
-                                  (uint32_t)weight->cols, part, part_bytes,
-                                  context->num_cus));
+                                  (uint32_t)weight->cols, scratch, context->num_cus));
     return kOk;
 }
 

@@ -390,11 +390,16 @@ struct GdnRollback {
 hipError_t launch_gdn_rollback(hipStream_t stream, const GdnRollback &r);
 
 // y[M][N] = x[M][K] . W[N][K]^T with f32 products, W of dtype F32/F16/BF16
-// (linear_kernels.hip).  linear_scratch_bytes: the scratch a call likes (split
-// x, or partial sums of calls that split K); unless linear_scratch_required(),
-// a call without it takes a route that needs none.
-size_t linear_scratch_bytes(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus);
-bool linear_scratch_required(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus);
+// (linear_kernels.hip).  A call takes a route that needs no more scratch than
+// there is; linear_scratch_bytes: what it would like (split x, or partial sums of
+// calls that split K; with split_rows also those of linear_rows_kernel).
+struct LinScratch {
+    float *ptr = nullptr;
+    size_t bytes = 0;
+    bool split_rows = true;
+};
+size_t linear_scratch_bytes(uint32_t M, uint32_t N, uint32_t K, uint32_t dtype, int num_cus,
+                            bool x_aligned, bool split_rows);
 // Device bytes of a [rows][cols] weight as the kernels read it: row-major for
 // F32 and F16, whole 1 KB tiles for BF16 (SIZE_MAX when that overflows).
 size_t linear_weight_bytes(uint64_t rows, uint64_t cols, uint32_t dtype);
@@ -405,8 +410,8 @@ hipError_t linear_pack_bf16(hipStream_t stream, const void *src, void *dst, uint
 // with room up to a multiple of four floats)
 hipError_t launch_linear_input(hipStream_t stream, const float *src, float *dst, uint64_t count);
 hipError_t launch_linear(hipStream_t stream, const float *x, const void *w, uint32_t dtype,
-                         float *y, uint32_t M, uint32_t N, uint32_t K, float *scratch,
-                         size_t scratch_bytes, int num_cus);
+                         float *y, uint32_t M, uint32_t N, uint32_t K, const LinScratch &scratch,
+                         int num_cus);
 
 // Conv + delta rule over every row of every sequence, then RMSNorm * silu(z).
 // Calls that take the chunked form need g.chunk_rec with

@@ -485,6 +485,45 @@ def test_captured_call_keeps_no_scratch(backend, rng, torch_mod):
         prepared.destroy()
 
 
+# a K split of the row tiles, the tiled product, a K split of linear_rows_kernel
+@pytest.mark.parametrize("rows,cols,out", [(1, 4096, 1024), (2048, 512, 4096), (64, 4096, 4096)])
+def test_captured_first_call_of_a_context(pkg, backend, rng, torch_mod, rows, cols, out):
+    # nothing can be allocated under capture: the call runs without scratch.  (The
+    # session's context has launched the kernels before: their code is loaded.)
+    torch = torch_mod
+    bits = weight_bits(rng.integers(-8, 9, size=(out, cols)).astype(np.float32), BF16)
+    wide = torch.from_numpy(widened(bits, BF16)).cuda()
+    x = torch.from_numpy(rng.integers(-8, 9, size=(rows, cols)).astype(np.float32)).cuda()
+    dy = torch.zeros((rows, out), device="cuda")
+    warm = backend.create_weight(bits, BF16)
+    device_call(backend, warm, x, dy, rows, cols, out)
+    backend.synchronize()
+    warm.destroy()
+    fresh = pkg.NativeBackend.load()
+    prepared = fresh.create_weight(bits, BF16)
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    fresh.set_stream(stream.cuda_stream)
+    try:
+        with torch.cuda.graph(graph, stream=stream):
+            device_call(fresh, prepared, x, dy, rows, cols, out)
+        for _ in range(3):
+            x.copy_(torch.from_numpy(rng.integers(-8, 9, size=(rows, cols)).astype(np.float32)))
+            dy.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(dy.double(), x.double() @ wide.T)
+            device_call(fresh, prepared, x, dy, rows, cols, out)  # with scratch
+            torch.cuda.synchronize()
+            assert torch.equal(dy.double(), x.double() @ wide.T)
+    finally:
+        fresh.set_stream(None)
+        prepared.destroy()
+        fresh.close()
+
+
 # host calls whose input or output is just within and just past the 2 MB that
 # stage through pinned memory, and counts that are no multiple of four floats
 @pytest.mark.parametrize("rows,cols,out", [(512, 1024, 33), (512, 1025, 33), (1024, 40, 512),

@@ -19,11 +19,11 @@ PROGRAM = r"""
 #include <cstdio>
 #include "linear_plan.hpp"
 int main() {
-    unsigned m, n, k, dtype, aligned;
+    unsigned m, n, k, dtype, aligned, split;
     unsigned long long scratch;
-    while (scanf("%u %u %u %u %u %llu", &m, &n, &k, &dtype, &aligned, &scratch) == 6) {
-        const sr::LinChoice c =
-            sr::linear_choice(m, n, k, dtype, 256, aligned != 0, (size_t)scratch);
+    while (scanf("%u %u %u %u %u %u %llu", &m, &n, &k, &dtype, &aligned, &split, &scratch) == 7) {
+        const sr::LinChoice c = sr::linear_choice(m, n, k, dtype, 256, aligned != 0,
+                                                  (size_t)scratch, split != 0);
         printf("%d %u %zu\n", (int)c.route, c.splits, c.scratch);
     }
 }
@@ -38,9 +38,10 @@ def choose(tmp_path_factory):
                     f"-I{ROOT / 'safetyraise-lmengine_amd' / 'csrc'}", str(where / "plan.cpp"),
                     "-o", str(where / "plan")], check=True)
 
-    def ask(shapes, scratch=ANY, dtype=BF16, aligned=True):
+    def ask(shapes, scratch=ANY, dtype=BF16, aligned=True, split_rows=True):
         """(route, K splits, scratch bytes) of each (rows, outputs, columns)."""
-        text = "".join(f"{m} {n} {k} {dtype} {int(aligned)} {scratch}\n" for m, n, k in shapes)
+        text = "".join(f"{m} {n} {k} {dtype} {int(aligned)} {int(split_rows)} {scratch}\n"
+                       for m, n, k in shapes)
         out = subprocess.run([str(where / "plan")], input=text, capture_output=True, text=True,
                              check=True).stdout
         return [tuple(map(int, line.split())) for line in out.splitlines()]
@@ -82,3 +83,20 @@ def test_calls_of_few_outputs_sum_the_parts_of_x_in_two_chains(choose):
     assert len(few) > 200
     for shape, (route, _, _) in zip(few, choose(few)):
         assert route == ROWS, shape
+
+
+@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+@pytest.mark.parametrize("aligned", [True, False])
+@pytest.mark.parametrize("scratch", [0, 1 << 20, 40 << 20])
+def test_no_call_needs_more_scratch_than_there_is(choose, dtype, aligned, scratch):
+    calls = shapes(3, 3000, cols=8) + [(1, 1024, 4096), (9, 4096, 12288), (2048, 4096, 4096)]
+    liked = choose(calls, dtype=dtype, aligned=aligned)
+    got = choose(calls, scratch=scratch, dtype=dtype, aligned=aligned)
+    short = 0
+    for call, like, have in zip(calls, liked, got):
+        short += like[2] > scratch
+        assert have[2] <= scratch, call
+        assert have[1] <= like[1] or like[0] != have[0], call
+        if like[2] <= scratch:
+            assert have == like, call
+    assert short > 0 or dtype != BF16

@@ -93,12 +93,15 @@ inline size_t split_x_bytes(uint32_t M, uint32_t K) {
 // split, the second launch and the partial sums' traffic.  Reproduces the best
 // measured split or one within 5 % of it, e.g. 512 rows of 3072 x 1024: 1
 // (17.6; 2: 25.7), 1024 of 1024 x 4096: 4 (35.1; 1: 55.4, 3: 40.3).
-inline uint32_t rows_splits(uint32_t M, uint32_t N, uint32_t units, uint32_t base, bool two_tiles,
-                            uint64_t cus, size_t scratch) {
+struct RowsSplit {
+    uint32_t splits;
+    double us;
+};
+inline RowsSplit rows_splits(uint32_t M, uint32_t N, uint32_t units, uint32_t base, bool two_tiles,
+                             uint64_t cus, size_t scratch) {
     const double one = two_tiles ? 1.1 : 0.86, two = two_tiles ? 1.9 : 1.5;  // us per stage
     const uint64_t outputs = (uint64_t)M * N;
-    uint32_t best = 1;
-    double best_us = 0.0;
+    RowsSplit best{1, 0.0};
     for (uint32_t s = 1; s <= kLinMaxSplits && s <= units; ++s) {
         if (s > 1 && (outputs > UINT32_MAX || outputs * s > scratch / sizeof(float))) break;
         const uint64_t wgs = (uint64_t)base * s;
@@ -106,12 +109,18 @@ inline uint32_t rows_splits(uint32_t M, uint32_t N, uint32_t units, uint32_t bas
         double us = (double)((units + s - 1) / s) *
                     ((double)rounds * two + (rest == 0 ? 0.0 : rest <= cus ? one : two));
         if (s > 1) us += 3.0 + (double)(outputs * (2 * s + 1) * sizeof(float)) / 5e6;
-        if (s == 1 || us < best_us) {
-            best = s;
-            best_us = us;
-        }
+        if (s == 1 || us < best.us) best = {s, us};
     }
     return best;
+}
+
+// linear_kernel on a bf16 weight, unsplit, in us: 5 and 0.034 per 16 x 16 x 32
+// block of the product and CU.  Of 180 timings from 6 to 1300 us half lie within
+// 15 %; calls of 17 to 64 rows, which wait for the weight, take up to 2.6 times
+// that.
+inline double tile_us(uint32_t M, uint32_t N, uint32_t K, uint64_t cus) {
+    return 5.0 + 0.034 / (double)cus * ((double)((M + kLinTile - 1) / kLinTile) * N / kLinTile) *
+                     ((double)K / kLinBlock);
 }
 
 // scratch: the bytes that are there (SIZE_MAX: as many as the call likes).  No
@@ -173,8 +182,13 @@ inline LinChoice linear_choice(uint32_t M, uint32_t N, uint32_t K, uint32_t dtyp
     if (!pays) return tile;
     const uint32_t rows = pair ? 2 * kLinTile : 4 * kLinTile;
     const uint32_t base = ((N + kRowsBN - 1) / kRowsBN) * ((M + rows - 1) / rows);
-    const uint32_t s = rows_splits(M, N, K / stage, base, pair, cus, split_rows ? scratch : 0);
-    return {LinRoute::kRows, {}, s, s > 1 ? s * split_bytes : 0};
+    const RowsSplit liked = rows_splits(M, N, K / stage, base, pair, cus, SIZE_MAX);
+    const RowsSplit split = rows_splits(M, N, K / stage, base, pair, cus, split_rows ? scratch : 0);
+    // Without the split it likes, a few workgroups walk all of K: 32 rows of 4096
+    // x 4096 35.5 (13.1 split) against 20.9 with kTile, 64 of it 57 / 29, 512 of
+    // 1024 x 12288 163 / 104, but 200 of 4096 x 4096 57 / 71
+    if (split.splits < liked.splits && split.us + 2.0 > tile_us(M, N, K, cus)) return tile;
+    return {LinRoute::kRows, {}, split.splits, split.splits > 1 ? split.splits * split_bytes : 0};
 }
 
 }  // namespace sr

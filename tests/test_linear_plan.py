@@ -100,3 +100,20 @@ def test_no_call_needs_more_scratch_than_there_is(choose, dtype, aligned, scratc
         if like[2] <= scratch:
             assert have == like, call
     assert short > 0 or dtype != BF16
+
+
+# without a K split; us of the row tiles and of linear_rows_kernel
+@pytest.mark.parametrize("shape,route", [
+    ((32, 4096, 4096), TILE),     # 21 / 36
+    ((64, 4096, 4096), TILE),     # 29 / 57
+    ((256, 1024, 4096), TILE),    # 25 / 56
+    ((512, 1024, 12288), TILE),   # 104 / 163
+    ((200, 4096, 4096), ROWS),    # 71 / 57
+    ((400, 2048, 6144), ROWS),    # 106 / 83
+    ((1024, 1024, 12288), ROWS),  # 186 / 162
+])
+def test_a_call_that_cannot_split_takes_the_faster_kernel(choose, shape, route):
+    liked, splits, _ = choose([shape])[0]
+    assert liked == ROWS and splits > 1
+    for got in (choose([shape], split_rows=False), choose([shape], scratch=0)):
+        assert got[0][0] == route and got[0][1] == 1

@@ -353,7 +353,13 @@ SAFETYRAISE_KERNEL_EXPORT int32_t safetyraise_kernel_gdn_forward(
  * same shape checks as linear (status 1); the input is not scanned for
  * non-finite values (linear does that on the host, native/cpu/
  * safetyraise_cpu.c:221-226): non-finite inputs give non-finite outputs.
- * The weight is any handle from create_weight (dtype F32, F16 or BF16). */
+ * The weight is any handle from create_weight (dtype F32, F16 or BF16).
+ *
+ * Calls may be captured into a HIP graph, which stays valid as long as the
+ * context and the weight.  Nothing is allocated then: a call takes the scratch
+ * that earlier calls of the context have left, or a route without.  Calls that
+ * split K share that scratch, so a replay is ordered with the context's other
+ * linear calls, like these among themselves. */
 SAFETYRAISE_KERNEL_EXPORT int32_t safetyraise_kernel_linear_device(
     safetyraise_kernel_context *context, safetyraise_kernel_weight *weight, const float *input,
     uint64_t input_rows, uint64_t input_cols, float *output, uint64_t output_rows,

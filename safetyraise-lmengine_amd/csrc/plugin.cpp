@@ -250,6 +250,7 @@ SAFETYRAISE_KERNEL_EXPORT int32_t safetyraise_kernel_destroy_context(
                             &context->linear_part}) {
         if (b->ptr != nullptr) (void)hipFree(b->ptr);
     }
+    for (const DeviceBuffer &b : context->linear_kept) (void)hipFree(b.ptr);
     if (context->linear_host != nullptr) (void)hipHostFree(context->linear_host);
     destroy_timer_events(context->timer);
     if (context->d_error_word != nullptr) (void)hipFree(context->d_error_word);
@@ -372,9 +373,11 @@ static int32_t check_linear(Ctx *ctx, const safetyraise_kernel_weight *w, const 
 
 // The context's linear scratch for a call.  Every call can do without: it goes
 // without when the buffer cannot grow, and with what is there while the stream
-// is captured, when nothing may be allocated or waited for.  The K splits of
-// linear_rows_kernel are not captured: a graph would keep the buffer's address,
-// and a later, larger call replaces the buffer.
+// is captured, when nothing may be allocated or waited for.  A buffer that a
+// graph knows is not freed but kept when a larger one replaces it, and the larger
+// one is at least twice its size, so what is kept stays below what is in use.
+// The K splits of linear_rows_kernel are not captured: graphs of many rows have no
+// scratch to share with each other, or with calls that run beside them.
 static int32_t linear_scratch(Ctx *ctx, const safetyraise_kernel_weight *w, uint64_t rows,
                               const float *x, LinScratch *scratch) {
     *scratch = LinScratch{};
@@ -391,8 +394,22 @@ static int32_t linear_scratch(Ctx *ctx, const safetyraise_kernel_weight *w, uint
         bytes = bytes_for(false);
         if (bytes == 0) return kOk;
     }
-    if (bytes > ctx->linear_part.bytes && capture == hipStreamCaptureStatusNone) {
-        const int32_t e = ensure_buffer(ctx, ctx->linear_part, bytes, false);
+    if (capture != hipStreamCaptureStatusNone) {
+        ctx->linear_captured = ctx->linear_captured || ctx->linear_part.ptr != nullptr;
+    } else if (bytes > ctx->linear_part.bytes) {
+        size_t want = bytes;
+        if (ctx->linear_captured) {
+            want = std::max(bytes, 2 * ctx->linear_part.bytes);
+            ctx->linear_kept.push_back(ctx->linear_part);
+            ctx->linear_part = DeviceBuffer{};
+            ctx->linear_captured = false;
+        }
+        int32_t e = ensure_buffer(ctx, ctx->linear_part, want, false);
+        if (e == kNoMemory && want > bytes) {
+            (void)hipGetLastError();
+            e = ensure_buffer(ctx, ctx->linear_part, bytes, false);
+            if (e == kOk) ctx->error.clear();
+        }
         if (e == kNoMemory) {
             (void)hipGetLastError();
             ctx->error.clear();

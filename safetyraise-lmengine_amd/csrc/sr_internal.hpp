@@ -113,7 +113,11 @@ struct safetyraise_kernel_context {
     sr::DeviceBuffer rope_scratch;     // prefill: per-row RoPE cos/sin
     sr::DeviceBuffer linear_in;        // linear: the host input's device copy
     sr::DeviceBuffer linear_out;       // linear: the output before it goes back
-    sr::DeviceBuffer linear_part;      // linear: partial sums of calls that split K
+    sr::DeviceBuffer linear_part;      // linear: split x, partial sums of calls that split K
+    // whether a captured call uses linear_part, and earlier ones that one did: graphs
+    // keep their addresses, so they live as long as the context
+    bool linear_captured = false;
+    std::vector<sr::DeviceBuffer> linear_kept;
     // linear: pinned host staging, kLinearHostBytes of input, then of output,
     // and its device address
     void *linear_host = nullptr;

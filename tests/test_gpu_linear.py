@@ -524,6 +524,49 @@ def test_captured_first_call_of_a_context(pkg, backend, rng, torch_mod, rows, co
         fresh.close()
 
 
+# a K split of the row tiles, and the tiled product
+@pytest.mark.parametrize("rows,cols,out", [(1, 4096, 1024), (2048, 512, 4096)])
+def test_captured_calls_keep_their_scratch(pkg, backend, rng, torch_mod, rows, cols, out):
+    # a call captured with scratch, whose buffer two larger calls then replace;
+    # what would be freed is taken by tensors that the replays must not write to
+    torch = torch_mod
+    fresh = pkg.NativeBackend.load()
+    bits = weight_bits(rng.integers(-8, 9, size=(out, cols)).astype(np.float32), BF16)
+    wide = torch.from_numpy(widened(bits, BF16)).cuda()
+    prepared = fresh.create_weight(bits, BF16)
+    large = fresh.create_weight(weight_bits(rng.standard_normal((4096, 2048)), BF16), BF16)
+    x = torch.zeros((rows, cols), device="cuda")
+    dy = torch.zeros((rows, out), device="cuda")
+    big = torch.zeros((16384, 2048), device="cuda")
+    by = torch.zeros((16384, 4096), device="cuda")
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    fresh.set_stream(stream.cuda_stream)
+    try:
+        device_call(fresh, prepared, x, dy, rows, cols, out)
+        fresh.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            device_call(fresh, prepared, x, dy, rows, cols, out)
+        guard = []
+        for n in (4096, 16384, 16384):
+            device_call(fresh, large, big, by, n, 2048, 4096)
+            fresh.synchronize()
+            guard += [torch.ones(1 << 18, device="cuda") for _ in range(16)]
+            x.copy_(torch.from_numpy(rng.integers(-8, 9, size=(rows, cols)).astype(np.float32)))
+            dy.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(dy.double(), x.double() @ wide.T)
+            assert all(bool((g == 1).all()) for g in guard)
+    finally:
+        fresh.set_stream(None)
+        prepared.destroy()
+        large.destroy()
+        fresh.close()
+
+
 # host calls whose input or output is just within and just past the 2 MB that
 # stage through pinned memory, and counts that are no multiple of four floats
 @pytest.mark.parametrize("rows,cols,out", [(512, 1024, 33), (512, 1025, 33), (1024, 40, 512),

@@ -1334,10 +1334,6 @@ __global__ void __launch_bounds__(kScanThreads) gdn_chunk_scan_kernel(const GdnP
     };
     f32x4 xs[kSeg];
     fetch(rec_of(0), xs);
-    // e^{g_C} of this chunk and the next: requested with their records.  Read
-    // where it is used, its latency followed each chunk's barrier: two prompts
-    // of 2048 rows by 64, 774 to 768 us.
-    float ec = rec_of(0)[kRecEc], ec_next = 0.0f;
     float *state = p.state + (((size_t)m.state_in * p.value_heads + h) * kHeadDv + vq * kVs) * kDk;
     {
         const int v = tid >> 4, d0 = (tid & 15) * 4;
@@ -1347,10 +1343,7 @@ __global__ void __launch_bounds__(kScanThreads) gdn_chunk_scan_kernel(const GdnP
         }
     }
     put(L.r[0], xs);
-    if (nchunks > 1) {
-        fetch(rec_of(1), xs);
-        ec_next = rec_of(1)[kRecEc];
-    }
+    if (nchunks > 1) fetch(rec_of(1), xs);
     __syncthreads();
     for (uint32_t c = 0; c < nchunks; ++c) {
         const uint32_t r0 = c * kCk;
@@ -1395,6 +1388,7 @@ __global__ void __launch_bounds__(kScanThreads) gdn_chunk_scan_kernel(const GdnP
             }
         } else {
             // S_C = e^{g_C} S0 + Delta^T Ks^T over state rows 16 tr.., dims 64 tc..
+            const float eC = p.chunk_rec[((size_t)(m.chunk0 + c) * p.value_heads + h) * kRecFloats + kRecEc];
             Ops<2> da;
             load_ops(da, &L.dt[16 * tr][0], kPc, lane);
             Ops<2> kb4[4];
@@ -1418,18 +1412,14 @@ __global__ void __launch_bounds__(kScanThreads) gdn_chunk_scan_kernel(const GdnP
             for (int n = 0; n < 4; ++n)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    L.s0[16 * tr + 4 * sl + i][64 * tc + 16 * n + r16] = s4[n][i] + ec * s0v[n][i];
+                    L.s0[16 * tr + 4 * sl + i][64 * tc + 16 * n + r16] = s4[n][i] + eC * s0v[n][i];
                 }
         }
         // the next chunk's record into the other buffer (last read in the
         // previous chunk), and the loads for the one after
         if (c + 1 < nchunks) {
             put(L.r[(c + 1) & 1], xs);
-            ec = ec_next;
-            if (c + 2 < nchunks) {
-                fetch(rec_of(c + 2), xs);
-                ec_next = rec_of(c + 2)[kRecEc];
-            }
+            if (c + 2 < nchunks) fetch(rec_of(c + 2), xs);
         }
         __syncthreads();  // the next chunk reads S0, its record, and rewrites dt
     }

@@ -875,10 +875,10 @@ hipError_t launch_linear(hipStream_t stream, const float *x, const void *w, uint
         const dim3 grid((N + 3 * kLinTile - 1) / (3 * kLinTile), 1);
         constexpr int DT = SAFETYRAISE_KERNEL_DTYPE_BF16;
         if (K % (kLinBlock * 16) == 0) {  // eight waves' ranges in whole pairs of blocks
-            SR_LAUNCH("linear_kernel_t3", (linear_kernel<DT, true, 3, 8, 1, true, 2>), grid, dim3(512), 0,
-                      stream, x, w, y, M, N, K);
+            SR_LAUNCH("linear_kernel_pair", (linear_kernel<DT, true, 3, 8, 1, true, 2>), grid, dim3(512),
+                      0, stream, x, w, y, M, N, K);
         } else {
-            SR_LAUNCH("linear_kernel_t3", (linear_kernel<DT, true, 3, 8, 1, false, 2>), grid, dim3(512),
+            SR_LAUNCH("linear_kernel_pair", (linear_kernel<DT, true, 3, 8, 1, false, 2>), grid, dim3(512),
                       0, stream, x, w, y, M, N, K);
         }
     } else {

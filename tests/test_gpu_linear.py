@@ -156,10 +156,11 @@ def test_multi_tile_plans_with_partial_blocks(backend, rng, rows, cols, out):
                                            (2048, 128, 1024)])
 def test_prefill_sized_calls_take_the_tiled_product(backend, rng, rows, cols, out):
     # 64+ rows with K a multiple of 64 on a bf16 weight, with at least 128
-    # output tiles of 128 x 128, take the tiled product (x split once per
-    # workgroup through LDS): calls with 2048+ outputs the 4-wave form, the
-    # 1024-output call the 8-wave one; one, three and eight stage pairs, rows
-    # and outputs past the last whole tile; random and integer inputs
+    # output tiles of 128 x 128: linear_rows_kernel (x split in LDS by every
+    # workgroup), or, from seven output tiles for every four CUs and at 64
+    # columns, the tiled product (x split once, before it); one, three and eight
+    # stage pairs, rows and outputs past the last whole tile; random and integer
+    # inputs
     x = (2 * rng.standard_normal((rows, cols))).astype(np.float32)
     bits = weight_bits(rng.standard_normal((out, cols)), BF16)
     got = backend.linear(bits, x, BF16)
@@ -320,12 +321,18 @@ def test_inputs_above_the_bf16_range(backend, rng, torch_mod, rows, cols, out):
 
 
 # bf16 calls of more than 16 rows: (rows, cols, out) at the edges of each route
-# (linear_choice in linear_kernels.hip): 32 rows per workgroup with whole and
+# (linear_choice in linear_plan.hpp): 32 rows per workgroup with whole and
 # ragged k ranges; 32- and 64-row workgroups with and without a K split, row
-# and output counts on and off the tiles; the tiled product
-ROUTES = [(17, 512, 10800), (32, 520, 10753), (17, 12288, 1027), (32, 4096, 4099), (33, 4096, 4099),
-          (64, 12352, 1030), (65, 4160, 1111), (100, 2112, 1500), (129, 2048, 1140),
-          (300, 960, 3000), (1000, 64, 7100), (130, 128, 28700)]
+# and output counts on and off the tiles; the tiled product.  The kernel that a
+# 16-byte aligned x takes, and another where an unaligned one does.
+PAIR, TILES, BY_ROWS, WIDE = ("linear_kernel_pair", "linear_kernel_t3", "linear_rows_kernel",
+                              "linear_gemm_wide_kernel")
+ROUTES = [(17, 512, 10800, PAIR, TILES), (32, 520, 10753, PAIR, TILES),
+          (17, 12288, 1027, BY_ROWS, BY_ROWS), (32, 4096, 4099, BY_ROWS, BY_ROWS),
+          (33, 4096, 4099, BY_ROWS, BY_ROWS), (64, 12352, 1030, BY_ROWS, BY_ROWS),
+          (65, 4160, 1111, BY_ROWS, BY_ROWS), (100, 2112, 1500, BY_ROWS, BY_ROWS),
+          (129, 2048, 1140, BY_ROWS, BY_ROWS), (300, 960, 3000, BY_ROWS, BY_ROWS),
+          (1000, 64, 7100, WIDE, WIDE), (130, 128, 28700, WIDE, WIDE)]
 
 
 def device_call(backend, prepared, x, dy, rows, cols, out):
@@ -334,10 +341,10 @@ def device_call(backend, prepared, x, dy, rows, cols, out):
         C.c_void_p(dy.data_ptr()), rows, out), "linear_device")
 
 
-@pytest.mark.parametrize("rows,cols,out", ROUTES)
-def test_routes_of_many_rows(backend, rng, torch_mod, rows, cols, out):
+@pytest.mark.parametrize("rows,cols,out,aligned,unaligned", ROUTES)
+def test_routes_of_many_rows(backend, rng, torch_mod, rows, cols, out, aligned, unaligned):
     # random inputs at the reordered-sum bound, from a 16-byte aligned and an
-    # unaligned x, and integer inputs bit for bit
+    # unaligned x, and integer inputs bit for bit; the kernel that ran
     torch = torch_mod
     for integers in (False, True):
         if integers:
@@ -358,8 +365,14 @@ def test_routes_of_many_rows(backend, rng, torch_mod, rows, cols, out):
                 buf[shift:shift + rows * cols] = torch.from_numpy(x).cuda().flatten()
                 dy = torch.full((rows, out), float("nan"), device="cuda")
                 torch.cuda.synchronize()
-                device_call(backend, prepared, buf[shift:], dy, rows, cols, out)
-                backend.synchronize()
+                backend.timing(True)
+                try:
+                    device_call(backend, prepared, buf[shift:], dy, rows, cols, out)
+                    backend.synchronize()
+                    ran = set(backend.kernel_times())
+                finally:
+                    backend.timing(False)
+                assert (unaligned if shift else aligned) in ran, ran
                 if integers:
                     assert torch.equal(dy.double(), ref), (rows, cols, out, shift)
                 else:

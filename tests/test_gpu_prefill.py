@@ -316,3 +316,39 @@ def test_prefill_rows_split_over_the_keys(pkg, backend, rng, heads, kv_heads, di
         backend.timing(False)
     assert set(kernels) <= ran and (MERGE in kernels) == (MERGE in ran), ran
     pool.destroy()
+
+
+# rows that are their own records, and rows cut into partitions
+@pytest.mark.parametrize("heads,seqs,merged", [(16, [(250, 700), (40, 500)], False),
+                                               (8, [(0, 600)], True)])
+def test_split_rows_beyond_fp16_range_are_recomputed(pkg, backend, rng, torch_mod, heads, seqs,
+                                                     merged):
+    # the same on the split-K kernel: one value in the last sequence's new rows
+    torch = torch_mod
+    pool = new_pool(pkg, backend, 2, 256, page_tokens=64, max_tokens=1024, seqs=4)
+    gq, gk = gammas(rng, 256)
+    cases = [Case(rng, pool, heads, 2, 256, ctx=c, rows=r) for c, r in seqs]
+    cases[-1].v[7, 300] = 2.0e5
+    backend.timing(True)
+    try:
+        run_case(pkg, backend, pool, cases, rotary=256, gq=gq, gk=gk)
+        ran = set(backend.kernel_times())
+    finally:
+        backend.timing(False)
+    assert SPLIT in ran and "attn_decode_kernel" in ran and (MERGE in ran) == merged, ran
+    for c in cases:
+        pool.close(c.seq)
+    c = Case(rng, pool, heads, 2, 256, ctx=seqs[-1][0], rows=seqs[-1][1])
+    d = Case(rng, pool, heads, 2, 256, ctx=seqs[0][0], rows=seqs[0][1])
+    c.v[3, 9] = -3.0e5
+    q, k, v, pos = (torch.from_numpy(np.concatenate([getattr(x, n) for x in (c, d)])).cuda()
+                    for n in ("q", "k", "v", "pos"))
+    out = torch.zeros((c.rows + d.rows, heads * 256), device="cuda")
+    pkg.attention_forward(backend, pool, [c.seq, d.seq], [c.rows, d.rows], q, k, v, pos, out,
+                          heads=heads, kv_heads=2, head_dim=256, rotary_dim=256, rope_theta=1e6,
+                          q_norm=torch.from_numpy(gq).cuda(), k_norm=torch.from_numpy(gk).cuda(),
+                          asynchronous=True)
+    with pytest.raises(pkg.PluginError) as err:
+        backend.synchronize()
+    assert "fp16 range" in str(err.value)
+    pool.destroy()

@@ -115,8 +115,8 @@ int32_t run_prefill_pack(Ctx *ctx, AttnLaunch &a, const std::vector<SeqMeta> &pa
 // to the limit (rows by the hundred at contexts of several partitions, which a
 // small page holds short) is cut: into two packs, or one sequence's rows into
 // two launches, the second of which attends to the first's rows.  Where there
-// is no memory for the records, and for a few rows that do not fit on their
-// own, the prefill kernels run instead.
+// is no memory for the records, or none to cut to (a RoPE table that leaves the
+// records of a few rows no room), the prefill kernels run instead.
 int32_t run_split_pack(Ctx *ctx, AttnLaunch &a, const std::vector<SeqMeta> &pack,
                        const AttnScratch &scratch, void *rope, uint64_t record_limit) {
     if (!split_fits(a, pack.data(), (int)pack.size(), ctx->num_cus, record_limit)) {
@@ -126,15 +126,19 @@ int32_t run_split_pack(Ctx *ctx, AttnLaunch &a, const std::vector<SeqMeta> &pack
             const auto middle = pack.begin() + (ptrdiff_t)(pack.size() / 2);
             first.assign(pack.begin(), middle);
             second.assign(middle, pack.end());
-        } else if (m.rows >= 2 * kPrefillMinRows) {
+        } else {
+            SeqMeta least = m;
+            least.rows = kPrefillMinRows;
+            if (m.rows < 2 * kPrefillMinRows ||
+                !split_fits(a, &least, 1, ctx->num_cus, record_limit)) {
+                return run_prefill_pack(ctx, a, pack, rope);
+            }
             const uint32_t half = m.rows / 2;
             first = second = pack;
             first[0].rows = half;
             second[0].ctx += half;
             second[0].row0 += half;
             second[0].rows -= half;
-        } else {
-            return run_prefill_pack(ctx, a, pack, rope);
         }
         const int32_t st = run_split_pack(ctx, a, first, scratch, rope, record_limit);
         return st != kOk ? st : run_split_pack(ctx, a, second, scratch, rope, record_limit);

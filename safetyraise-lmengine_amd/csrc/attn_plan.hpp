@@ -65,38 +65,41 @@ inline SplitPlan split_plan(const SplitShape &a, const SeqMeta *seqs, int nseq,
     constexpr uint64_t kEnds = 5 * kKeyTile;
     constexpr uint64_t kMerge = 3 * kKeyTile;
     auto up = [](uint64_t x, uint64_t unit) { return (x + unit - 1) / unit; };
-    auto total = [&](int i) { return (uint64_t)seqs[i].ctx + seqs[i].rows; };
     SplitPlan plan{};
     uint64_t max_rows = 0;
-    for (int i = 0; i < nseq; ++i) max_rows = std::max<uint64_t>(max_rows, seqs[i].rows);
+    uint64_t total[kMetaPerLaunch], slices[kMetaPerLaunch];  // keys, row slices
+    for (int i = 0; i < nseq; ++i) {
+        max_rows = std::max<uint64_t>(max_rows, seqs[i].rows);
+        total[i] = (uint64_t)seqs[i].ctx + seqs[i].rows;
+    }
     // query vectors per workgroup: 64 in the pair mode; at D <= 128 a call
     // with more takes the all-tiles form (128 vectors over its four consumer
     // waves), rows beyond run as further slices of the rows
     plan.all_tiles = a.head_dim <= 128 && max_rows * group > 64;
     plan.rows_per_slice = (uint32_t)((plan.all_tiles ? 128 : 64) / group);
     plan.records_per_part = (a.head_dim <= 128 && !plan.all_tiles) ? 2 : 1;
-    auto slices = [&](int i) { return up(seqs[i].rows, plan.rows_per_slice); };
-    auto direct = [&](uint64_t part) { return plan.records_per_part == 1 && total(0) <= part; };
+    for (int i = 0; i < nseq; ++i) slices[i] = up(seqs[i].rows, plan.rows_per_slice);
+    auto direct = [&](uint64_t part) { return plan.records_per_part == 1 && total[0] <= part; };
     auto bytes = [&](uint64_t part) -> uint64_t {
         if (direct(part)) return 0;
         uint64_t n = 0;
-        for (int i = 0; i < nseq; ++i) n += up(total(i), part) * seqs[i].rows;
+        for (int i = 0; i < nseq; ++i) n += up(total[i], part) * seqs[i].rows;
         return n * plan.records_per_part * a.heads * record_stride(a.head_dim) * sizeof(float);
     };
     // a partition starting mid-page touches at most part/page_tokens + 2 pages
     const uint64_t max_part = std::min<uint64_t>(
         ((uint64_t)(kVerifyPageSlots - 2) * a.page_tokens) / kKeyTile * kKeyTile, 1u << 30);
-    const uint64_t longest = up(total(0), kKeyTile) * kKeyTile;
+    const uint64_t longest = up(total[0], kKeyTile) * kKeyTile;
     const uint64_t most = std::min(longest, max_part);
     uint64_t keys = 0, unsplit = 0, before = 0;
     for (int i = 0; i < nseq; ++i) {
-        const uint64_t n = slices(i) * kvv;
+        const uint64_t n = slices[i] * kvv;
         // (a slice sees the context and the rows up to its own last)
         keys += n * seqs[i].ctx +
-                kvv * (seqs[i].rows + plan.rows_per_slice * (slices(i) - 1)) * slices(i) / 2;
-        unsplit = std::max(unsplit, i == 0 ? up(n, cus) * (total(i) + kEnds)
-                                           : (before + n * (total(i) + kEnds)) / cus + total(i));
-        before += n * (total(i) + kEnds);
+                kvv * (seqs[i].rows + plan.rows_per_slice * (slices[i] - 1)) * slices[i] / 2;
+        unsplit = std::max(unsplit, i == 0 ? up(n, cus) * (total[i] + kEnds)
+                                           : (before + n * (total[i] + kEnds)) / cus + total[i]);
+        before += n * (total[i] + kEnds);
     }
     uint64_t best = 0, best_time = ~0ull, first = 0;
     if (longest <= max_part && bytes(longest) <= record_limit) {
@@ -108,8 +111,8 @@ inline SplitPlan split_plan(const SplitShape &a, const SeqMeta *seqs, int nseq,
         // (each sequence's last partition is short: a few steps up until they fit)
         for (int step = 0; step < 32 && part < longest; ++step) {
             uint64_t n = 0;
-            for (int i = 0; i < nseq; ++i) n += up(total(i), part) * kvv * slices(i);
-            if (n <= per * cus) break;
+            for (int i = 0; i < nseq; ++i) n += up(total[i], part) * slices[i];
+            if (n * kvv <= per * cus) break;
             part += up(part, 32 * kKeyTile) * kKeyTile;
         }
         part = std::min(part, most);

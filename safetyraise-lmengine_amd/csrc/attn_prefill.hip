@@ -1380,11 +1380,11 @@ __device__ __forceinline__ void store_dims(const PrefillParams &p, uint32_t call
     if (!finite) atomicOr(p.err_word, kErrPrefillRange);
 }
 
-// store_rows for a wave's 32 rows through a 4 KB slice of LDS, 32 dims at a
+// store_dims for a wave's 32 rows through a 4 KB slice of LDS, 32 dims at a
 // time: the lanes write their accumulator values (row col, dims 8a + 4h ..)
 // to the slice and read them back row-major, so each store instruction
 // writes whole 128-byte lines (8 rows x 32 dims) instead of 32 bytes of each
-// of 32 rows.  Same values, gate and finite check as store_rows; rows from
+// of 32 rows.  Same values, gate and finite check as store_dims; rows from
 // `valid` on are not stored.  Both write the output with nontemporal stores:
 // the kernel never reads it back, and streaming it out took 2.2 us off a
 // 512-row call at head_dim 128.
@@ -2326,9 +2326,10 @@ hipError_t launch_d(hipStream_t stream, PrefillParams &p, uint32_t g, const SeqM
 
 
 // ---------------------------------------------------------------------------
-// Multi-row verify (MTP drafts): split-K flash decoding with MFMA inner
-// products.  A call appends R (2..15) rows per sequence; row r sees the
-// context plus rows 0..r.  The R x G query vectors of a KV head (row r, head
+// Multi-row verify (MTP drafts), and prefill rows that would leave most CUs idle
+// (split_preferred): split-K flash decoding with MFMA inner products.  A call
+// appends R rows per sequence (drafts 2..15); row r sees the context plus rows
+// 0..r.  The R x G query vectors of a KV head (row r, head
 // g: vector r*G + g) fill the N dimension of the MFMA tiles, 32 per wave, so
 // each K/V tile of the cache is read once for all rows and heads.  The keys
 // of a sequence are cut into partitions of part_keys (a multiple of 64); one
@@ -2348,7 +2349,8 @@ hipError_t launch_d(hipStream_t stream, PrefillParams &p, uint32_t g, const SeqM
 // (unit, slice) grid that leave at once still take their turn, and every other
 // one being empty (the second slice of sequences that have one) left half of
 // the engines idle while the next block waited for a full one.  4 sequences of
-// 40 K to 131 K keys with 2 to 9 rows (16 / 2 x 256): 214 to 134 us.
+// 40 K to 131 K keys with 2 to 9 rows (16 / 2 x 256): 214 to 149 us (with the
+// slices' own ranges and the partition rule of attn_plan.hpp 138 to 147, by box).
 // ---------------------------------------------------------------------------
 struct VerifyParams {
     PrefillParams p;       // meta[s].nblk = records per (row, head) of sequence s

@@ -21,14 +21,15 @@
 //
 // Work split of linear_kernel.  A workgroup owns 16 R rows (R = 1, or 2 in one
 // plan) x 16 T outputs (T tiles per wave) and a contiguous range of K; its W
-// waves take equal parts of that range and meet in LDS.  Decode-sized calls (M <= 16) stream every weight row
-// once, the HBM-bound regime the ABI's projections live in; each k block
-// loads 32 bytes of x per lane, used by T tiles, and 8 weight elements per
-// tile.  x is the larger share of the bytes a lane loads, so T > 1 keeps the
+// waves take equal parts of that range and meet in LDS.  Decode-sized calls
+// (M <= 16) stream every weight row once, the HBM-bound regime the ABI's
+// projections live in; each k block loads 32 bytes of x per lane, used by T
+// tiles, and 8 weight elements per tile.  x is the larger share of the bytes a lane loads, so T > 1 keeps the
 // load pipeline (texture address unit) from being the limit.  A call whose
 // tiles do not cover the CUs splits K over up to kLinMaxSplits workgroups per
 // tile (grid z): those write partial sums and a second kernel adds them in
-// split order, so results do not depend on timing (linear_plan chooses).
+// split order, so results do not depend on timing (linear_plan.hpp: how a call
+// is cut, and which calls of more than 16 rows take the kernels further down).
 //
 // Operand order.  For a 32-wide k block, lane (r = lane % 16, g = lane / 16)
 // holds x[row r][k0 + 8g .. + 8] and W[output r][same k] (any order of k
@@ -131,13 +132,14 @@ __device__ __forceinline__ void split3(const f32x8 &x, bf16x8 &hi, bf16x8 &mid, 
 }
 
 // y: the output, or (grid z > 1) partial sums [grid z][M][N].  T: output tiles
-// per wave (the workgroup owns 16 T outputs; each x fragment a lane loads feeds T MFMAs, so x is read once
-// per 16 T outputs).  R: row tiles per workgroup (each weight fragment feeds
-// R rows' MFMAs; with R = 2 the weight is read once per 32 rows).  W: waves per
-// workgroup, splitting its k range.  kGroup: k blocks per register set (4; 2 for calls with many workgroups per CU, which
-// then hold more waves per SIMD).  kExact: every wave's k range is a whole
-// number of pairs of groups of whole blocks (the host checks), so no load
-// reaches past it, nothing is masked and the last pair prefetches nothing.
+// per wave (the workgroup owns 16 T outputs; each x fragment a lane loads feeds
+// T MFMAs, so x is read once per 16 T outputs).  R: row tiles per workgroup (each
+// weight fragment feeds R rows' MFMAs; with R = 2 the weight is read once per 32
+// rows).  W: waves per workgroup, splitting its k range.  kGroup: k blocks per
+// register set (4; 2 for calls with many workgroups per CU, which then hold more
+// waves per SIMD).  kExact: every wave's k range is a whole number of pairs of
+// groups of whole blocks (the host checks), so no load reaches past it, nothing
+// is masked and the last pair prefetches nothing.
 template <int DT, bool kVec, int T, int W, int kGroup, bool kExact, int R>
 __global__ __launch_bounds__(64 * W) void linear_kernel(const float *x, const void *w, float *y,
                                                         uint32_t M, uint32_t N, uint32_t K) {
@@ -507,8 +509,8 @@ __global__ __launch_bounds__(64 * kRowsWaves, 4) void linear_rows_kernel(const f
 }
 
 // ---------------------------------------------------------------------------
-// Calls whose 128 x 128 output tiles exceed two per CU (large prefill chunks):
-// a tiled product.  linear_split_x_kernel first writes x once as its three
+// Calls of 2048 outputs or more with nearly two 128 x 128 output tiles per CU
+// (large prefill chunks): a tiled product.  linear_split_x_kernel first writes x once as its three
 // bf16 parts (split3) in MFMA lane order: for row tile t (16 rows), k block b
 // (32 columns) and part c, the 1 KB at ((t * nblk + b) * 3 + c) KB holds, at
 // lane 16 g + r, x[16 t + r][32 b + 8 g .. + 8].  linear_gemm_wide_kernel then

@@ -1387,7 +1387,9 @@ __device__ __forceinline__ void store_dims(const PrefillParams &p, uint32_t call
 // of 32 rows.  Same values, gate and finite check as store_dims; rows from
 // `valid` on are not stored.  Both write the output with nontemporal stores:
 // the kernel never reads it back, and streaming it out took 2.2 us off a
-// 512-row call at head_dim 128.
+// 512-row call at head_dim 128.  Gated and plain calls each have a loop: with the
+// test inside it the gates' loads cost plain calls 0.3 to 0.5 us each (two
+// sequences of 44 rows at 32 / 8 x 128 19.5 against 19.0).
 template <int D>
 __device__ __forceinline__ void store_rows_lds(const PrefillParams &p, uint32_t call_row0,
                                                int valid, uint32_t head, int h, int col,
@@ -1396,47 +1398,50 @@ __device__ __forceinline__ void store_rows_lds(const PrefillParams &p, uint32_t 
                                                __attribute__((address_space(3))) f32x4 *slice) {
     constexpr int NT = D / 32;
     const bool bf16_in = (p.flags & SAFETYRAISE_MI355X_INPUT_BF16) != 0;
-    const bool gated = (p.flags & SAFETYRAISE_MI355X_GATED) != 0;
-    const uint32_t hs = gated ? 2 * D : D;
     const float inv_l = 1.0f / l_run;
     bool finite = true;
+    auto store = [&](auto gated) __attribute__((always_inline)) {
 #pragma unroll
-    for (int tt = 0; tt < NT; ++tt) {
+        for (int tt = 0; tt < NT; ++tt) {
 #pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            f32x4 o;
+            for (int a = 0; a < 4; ++a) {
+                f32x4 o;
 #pragma unroll
-            for (int bb = 0; bb < 4; ++bb) {
-                o[bb] = oacc[tt][4 * a + bb] * inv_l;
-                finite = finite && (col >= valid || isfinite(o[bb]));
-            }
-            slice[col * 8 + ((2 * a + h) ^ (col & 7))] = o;
-        }
-        // LDS operations of one wave are performed in order; the fences keep
-        // the compiler from moving the reads above the writes
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = 8 * i + (lane >> 3), k = lane & 7;
-            f32x4 o = slice[r * 8 + (k ^ (r & 7))];
-            const uint32_t d0 = 32 * tt + 4 * k;
-            if (r < valid) {
-                const size_t row = (size_t)(call_row0 + r);
-                if (gated) {
-                    const f32x4 gate =
-                        load_act4(p.q, row * p.heads * hs + (size_t)head * hs + D + d0, bf16_in);
-#pragma unroll
-                    for (int bb = 0; bb < 4; ++bb) o[bb] *= ref_sigmoid(gate[bb]);
+                for (int bb = 0; bb < 4; ++bb) {
+                    o[bb] = oacc[tt][4 * a + bb] * inv_l;
+                    finite = finite && (col >= valid || isfinite(o[bb]));
                 }
-                __builtin_nontemporal_store(o, (f32x4 *)(p.out + row * p.heads * D + (size_t)head * D + d0));
+                slice[col * 8 + ((2 * a + h) ^ (col & 7))] = o;
             }
+            // LDS operations of one wave are performed in order; the fences keep
+            // the compiler from moving the reads above the writes
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int r = 8 * i + (lane >> 3), k = lane & 7;
+                f32x4 o = slice[r * 8 + (k ^ (r & 7))];
+                const uint32_t d0 = 32 * tt + 4 * k;
+                if (r < valid) {
+                    const size_t row = (size_t)(call_row0 + r);
+                    if constexpr (decltype(gated)::value) {
+                        const f32x4 gate =
+                            load_act4(p.q, (row * p.heads + head) * 2 * D + D + d0, bf16_in);
+#pragma unroll
+                        for (int bb = 0; bb < 4; ++bb) o[bb] *= ref_sigmoid(gate[bb]);
+                    }
+                    __builtin_nontemporal_store(
+                        o, (f32x4 *)(p.out + row * p.heads * D + (size_t)head * D + d0));
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
+    };
+    if (p.flags & SAFETYRAISE_MI355X_GATED) store(std::true_type{});
+    else store(std::false_type{});
     if (!finite) atomicOr(p.err_word, kErrPrefillRange);
 }
 

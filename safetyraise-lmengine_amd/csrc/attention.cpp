@@ -424,25 +424,25 @@ int32_t attention_forward_impl(Ctx *ctx, const safetyraise_kernel_attention_args
         });
     if (pst != kOk) return pst;
     // Prefill rows whose row blocks would leave most of the CUs idle take it too.
-    std::vector<SeqMeta> candidates;
-    std::vector<uint8_t> split(A.num_seqs, 0);
+    std::vector<SeqMeta> chunks;
+    std::vector<uint32_t> chunk_of;
     for (uint32_t i = 0; prefill_ok && i < A.num_seqs; ++i) {
-        if (A.seq_rows[i] < kPrefillMinRows || !split_candidate(L, (uint32_t)old_len[i], A.seq_rows[i])) {
-            continue;
-        }
-        split[i] = 1;
-        candidates.push_back(meta(i));
+        if (A.seq_rows[i] < kPrefillMinRows) continue;
+        chunks.push_back(meta(i));
+        chunk_of.push_back(i);
     }
-    const bool preferred =
-        split_preferred(L, candidates.data(), (int)candidates.size(), ctx->num_cus);
-    pst = run_packs([&](uint32_t i) { return preferred && split[i]; },
+    std::vector<uint8_t> chosen(chunks.size()), split(A.num_seqs, 0);
+    choose_split({L.heads, L.kv_heads * L.kv_rep, L.head_dim, pool->page_tokens, ctx->num_cus},
+                 chunks.data(), (int)chunks.size(), chosen.data());
+    for (size_t c = 0; c < chunks.size(); ++c) split[chunk_of[c]] = chosen[c];
+    pst = run_packs([&](uint32_t i) { return split[i] != 0; },
                     [&](const std::vector<SeqMeta> &pack) {
                         return run_split_pack(ctx, L, pack, scratch, rope, record_limit);
                     });
     if (pst != kOk) return pst;
     pst = run_packs(
         [&](uint32_t i) {
-            return prefill_ok && A.seq_rows[i] >= kPrefillMinRows && !(preferred && split[i]);
+            return prefill_ok && A.seq_rows[i] >= kPrefillMinRows && split[i] == 0;
         },
         [&](const std::vector<SeqMeta> &pack) { return run_prefill_pack(ctx, L, pack, rope); });
     if (pst != kOk) return pst;

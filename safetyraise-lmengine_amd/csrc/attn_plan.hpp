@@ -3,6 +3,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 
 #include "sr_internal.hpp"
@@ -34,6 +35,77 @@ struct SplitShape {
     uint32_t head_dim, page_tokens;
     int num_cus;
 };
+
+// Sequences of 16 or more rows that may take the split-K kernel.  The prefill
+// kernels run one workgroup per row block and KV head down the whole context,
+// so a chunk of few rows leaves most CUs idle: 32 rows of 32 / 8 x 128 at 4096
+// keys 90 us, split 25; at 16 K keys 323 / 38.  Below these lengths the second
+// launch and the records cost what the split gives (32 rows at 320 keys 18 / 17
+// us, 256 rows at 640 keys 31 / 24 but four such sequences 32 / 58).  Head_dim
+// 256 has no kernel but the lock-step one, 10 us per 64 keys (32 rows of 16 / 2
+// at 1 K keys 206 us, split 28; 1024 rows 364 / 88, four such 668 / 292).
+inline bool split_candidate(const SplitShape &a, const SeqMeta &m) {
+    const uint32_t g = a.heads / a.kv_heads;
+    const uint64_t keys = (uint64_t)m.ctx + m.rows;
+    if (a.head_dim > 128) return keys > 256;
+    return keys > (m.rows * g <= 128 && m.rows <= 64 ? 320u : 1024u);
+}
+
+// Which of a call's sequences of 16 or more rows take the split-K kernel: the
+// candidates, where that makes the call faster by a margin of a tenth, or none.
+// Times in us, fitted to calls of one and four sequences of 16 to 1024 rows at
+// 128 to 16 K keys: the prefill kernels take a start and a time per 64-key tile
+// of the longest workgroup (more with every CU busy), the split form a start, a
+// time per tile of an equal share per CU, and the merge of the records.  32 / 8 x
+// 128, estimated (measured): 512 rows at 4096 keys 125 (105) / 78 (65), 1024 rows
+// at 16 K 534 (373) / 400 (346), four sequences of 512 rows at 4096 keys 150 (144)
+// / 233 (243).  The sequences that are no candidates run the prefill kernels
+// beside or after them: 808 rows and 165 after 1351 keys (16 / 4 x 128) 49 us in
+// one launch, 60 with the second sequence split; 23 sequences of 23 to 1212 rows
+// (8 / 8 x 64) 48 / 77; 118 rows after 142 keys and 135 after 100 (16 / 2 x 256) 105 /
+// 127.  At head_dim 256 any candidate on its own gains.
+inline void choose_split(const SplitShape &a, const SeqMeta *seqs, int nseq, uint8_t *split) {
+    int candidates = 0;
+    for (int i = 0; i < nseq; ++i) {
+        split[i] = split_candidate(a, seqs[i]);
+        candidates += split[i];
+    }
+    if (candidates == 0) return;
+    struct Times {
+        double block, start, tile, tile_busy;          // prefill kernels; query vectors a block
+        double slice, split_start, split_tile, record;  // split form; query vectors a slice
+    };
+    const Times t = a.head_dim == 64    ? Times{256, 6, 1.43, 0.05, 128, 11, 0.95, 0.0004}
+                    : a.head_dim == 128 ? Times{256, 12, 1.22, 0.7, 128, 17, 1.4, 0.0004}
+                                        : Times{128, 60, 9, 0, 64, 22, 2.8, 0};
+    const uint32_t g = a.heads / a.kv_heads;
+    const double cus = std::max(a.num_cus, 1);
+    auto tiles = [&](int i) { return ((double)seqs[i].ctx + seqs[i].rows) / kKeyTile; };
+    // the prefill kernels over all the sequences, or those that are no candidates
+    auto whole = [&](bool all) {
+        double wgs = 0, total = 0, longest = 0;
+        for (int i = 0; i < nseq; ++i) {
+            if (split[i] && !all) continue;
+            const double blocks = std::ceil((double)seqs[i].rows * g / t.block) * a.kv_heads;
+            wgs += blocks;
+            total += blocks * tiles(i);
+            longest = std::max(longest, tiles(i));
+        }
+        return wgs == 0 ? 0.0
+                        : t.start + (t.tile + t.tile_busy * std::min(1.0, wgs / cus)) *
+                                        std::max(longest, total / cus);
+    };
+    double share = 0, records = 0;
+    for (int i = 0; i < nseq; ++i) {
+        if (!split[i]) continue;
+        const double vectors = (double)seqs[i].rows * g;
+        share += std::ceil(vectors / t.slice) * a.kv_heads * (tiles(i) - 0.5 * seqs[i].rows / kKeyTile);
+        records += vectors * a.kv_heads;
+    }
+    const double parts =
+        t.split_start + t.split_tile * std::max(share / cus, 2.0) + t.record * records + whole(false);
+    if (parts * 1.1 >= whole(true)) std::fill(split, split + nseq, (uint8_t)0);
+}
 
 struct SplitPlan {
     bool all_tiles;             // each consumer wave takes both tiles of a step

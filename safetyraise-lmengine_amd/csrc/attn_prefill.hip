@@ -38,7 +38,6 @@
 // non-finite; the row is then flagged (kErrPrefillRange) for the host, which
 // recomputes the call on the f32 split-K path.
 #include <algorithm>
-#include <cmath>
 #include <type_traits>
 
 #include "attn_plan.hpp"
@@ -2332,7 +2331,7 @@ hipError_t launch_d(hipStream_t stream, PrefillParams &p, uint32_t g, const SeqM
 
 // ---------------------------------------------------------------------------
 // Multi-row verify (MTP drafts), and prefill rows that would leave most CUs idle
-// (split_preferred): split-K flash decoding with MFMA inner products.  A call
+// (choose_split): split-K flash decoding with MFMA inner products.  A call
 // appends R rows per sequence (drafts 2..15); row r sees the context plus rows
 // 0..r.  The R x G query vectors of a KV head (row r, head
 // g: vector r*G + g) fill the N dimension of the MFMA tiles, 32 per wave, so
@@ -2940,56 +2939,6 @@ hipError_t launch_attn_prefill(hipStream_t stream, const AttnLaunch &a, const Se
         case 256: return launch_d<256>(stream, p, g, seqs, nseq);
         default: return hipErrorInvalidValue;
     }
-}
-
-// Sequences of 16 or more rows that may take the split-K kernel.  The prefill
-// kernels run one workgroup per row block and KV head down the whole context,
-// so a chunk of few rows leaves most CUs idle: 32 rows of 32 / 8 x 128 at 4096
-// keys 90 us, split 25; at 16 K keys 323 / 38.  Below these lengths the second
-// launch and the records cost what the split gives (32 rows at 320 keys 18 / 17
-// us, 256 rows at 640 keys 31 / 24 but four such sequences 32 / 58).  Head_dim
-// 256 has no kernel but the lock-step one, 10 us per 64 keys (32 rows of 16 / 2
-// at 1 K keys 206 us, split 28; 1024 rows 364 / 88, four such 668 / 292).
-bool split_candidate(const AttnLaunch &a, uint32_t ctx, uint32_t rows) {
-    if (!prefill_supported(a)) return false;
-    const uint32_t g = a.heads / (a.kv_heads * a.kv_rep);
-    const uint64_t keys = (uint64_t)ctx + rows;
-    if (a.head_dim > 128) return keys > 256;
-    return keys > (rows * g <= 128 && rows <= 64 ? 320u : 1024u);
-}
-
-// Whether the candidates of a call (all its sequences in seqs) run faster
-// split, by a margin of a tenth.  Times in us, fitted to calls of one and four
-// sequences of 16 to 1024 rows at 128 to 16 K keys: the prefill kernels take
-// a start and a time per 64-key tile of the longest workgroup (more with every
-// CU busy), the split form a start, a time per tile of an equal share per CU,
-// and the merge of the records.  32 / 8 x 128, estimated (measured): 512 rows
-// at 4096 keys 125 (105) / 78 (65), 1024 rows at 16 K 534 (373) / 400 (346),
-// four sequences of 512 rows at 4096 keys 150 (144) / 233 (243).
-bool split_preferred(const AttnLaunch &a, const SeqMeta *seqs, int nseq, int num_cus) {
-    if (nseq <= 0) return false;
-    if (a.head_dim > 128) return true;
-    struct Times {
-        double start, tile, tile_busy, split_start, split_tile;
-    };
-    const Times t = a.head_dim == 64 ? Times{6, 1.43, 0.05, 11, 0.95} : Times{12, 1.22, 0.7, 17, 1.4};
-    const uint32_t kvv = a.kv_heads * a.kv_rep, g = a.heads / kvv;
-    const double cus = num_cus > 0 ? num_cus : 1;
-    double wgs = 0, total = 0, longest = 0, split = 0, records = 0;
-    for (int i = 0; i < nseq; ++i) {
-        const double vectors = (double)seqs[i].rows * g;
-        const double tiles = ((double)seqs[i].ctx + seqs[i].rows) / kKeyTile;
-        const double blocks = ceil(vectors / 256) * kvv;
-        wgs += blocks;
-        total += blocks * tiles;
-        longest = std::max(longest, tiles);
-        split += ceil(vectors / 128) * kvv * (tiles - 0.5 * seqs[i].rows / kKeyTile);
-        records += vectors * kvv;
-    }
-    const double whole = t.start + (t.tile + t.tile_busy * std::min(1.0, wgs / cus)) *
-                                       std::max(longest, total / cus);
-    const double parts = t.split_start + t.split_tile * std::max(split / cus, 2.0) + 0.0004 * records;
-    return parts * 1.1 < whole;
 }
 
 bool verify_supported(const AttnLaunch &a, uint32_t rows) {

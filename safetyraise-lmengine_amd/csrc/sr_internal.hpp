@@ -342,10 +342,6 @@ hipError_t launch_attn_prefill(hipStream_t s, const AttnLaunch &a, const SeqMeta
 // where it can (split_fits, attn_plan.hpp); a call whose records
 // in.reserve_partials does not provide launches nothing (hipErrorOutOfMemory).
 bool verify_supported(const AttnLaunch &a, uint32_t rows);
-// Whether a sequence of prefill rows may take it, and whether a call's such
-// sequences should.
-bool split_candidate(const AttnLaunch &a, uint32_t ctx, uint32_t rows);
-bool split_preferred(const AttnLaunch &a, const SeqMeta *seqs, int nseq, int num_cus);
 bool split_fits(const AttnLaunch &a, const SeqMeta *seqs, int nseq, int num_cus,
                 uint64_t record_limit);
 // Head widths other than 64, 128 and 256 (up to kGenericMaxHeadDim): every

@@ -24,10 +24,18 @@ int main(int argc, char **argv) {
     }
     unsigned heads, kv, dim, page, n;
     unsigned long long limit;
+    const bool choose = argc == 2;
     while (scanf("%u %u %u %u %llu %u", &heads, &kv, &dim, &page, &limit, &n) == 6) {
         sr::SeqMeta m[64] = {};
         for (unsigned i = 0; i < n; ++i) {
             if (scanf("%u %u", &m[i].ctx, &m[i].rows) != 2) return 1;
+        }
+        if (choose) {
+            uint8_t split[64];
+            sr::choose_split({heads, kv, dim, page, 256}, m, (int)n, split);
+            for (unsigned i = 0; i < n; ++i) printf("%d ", (int)split[i]);
+            printf("\n");
+            continue;
         }
         const sr::SplitPlan p = sr::split_plan({heads, kv, dim, page, 256}, m, (int)n, limit);
         printf("%u %llu %u %u %d\n", p.part_keys, (unsigned long long)p.record_bytes,
@@ -46,17 +54,21 @@ def plans(tmp_path_factory):
                     f"-I{ROOT / 'safetyraise-lmengine_amd' / 'csrc'}", str(where / "plan.cpp"),
                     "-o", str(where / "plan")], check=True)
 
-    def ask(calls):
-        """calls: (heads, kv_heads, head_dim, page_tokens, limit, [(ctx, rows), ...]), the
-        sequences in descending order of their keys."""
+    def run(calls, *args):
         text = "".join(f"{h} {kv} {d} {p} {lim} {len(seqs)} "
                        + " ".join(f"{c} {r}" for c, r in seqs) + "\n"
                        for h, kv, d, p, lim, seqs in calls)
-        out = subprocess.run([str(where / "plan")], input=text, capture_output=True, text=True,
-                             check=True).stdout
-        return [dict(zip(("part", "bytes", "rows_per_slice", "per_part", "direct"),
-                         map(int, line.split()))) for line in out.splitlines()]
+        return subprocess.run([str(where / "plan"), *args], input=text, capture_output=True,
+                              text=True, check=True).stdout.splitlines()
 
+    def ask(calls):
+        """calls: (heads, kv_heads, head_dim, page_tokens, limit, [(ctx, rows), ...]), the
+        sequences in descending order of their keys."""
+        return [dict(zip(("part", "bytes", "rows_per_slice", "per_part", "direct"),
+                         map(int, line.split()))) for line in run(calls)]
+
+    ask.chosen = lambda heads, kv, dim, seqs: list(
+        map(int, run([(heads, kv, dim, 64, 0, seqs)], "choose")[0].split()))
     ask.grown = lambda have, need: int(subprocess.run(
         [str(where / "plan"), str(have), str(need)], capture_output=True, text=True,
         check=True).stdout)
@@ -140,3 +152,23 @@ def test_a_prompt_in_small_chunks_replaces_its_records_a_few_times(plans, heads,
     assert grown <= 3
     # a single need above the usual limit is met and no more
     assert plans.grown(REGION, REGION + 5) == REGION + 5
+
+
+# (context, rows) of each sequence; us of a call in one launch of the prefill
+# kernels, and with the sequences that are long enough split beside it
+@pytest.mark.parametrize("heads,kv,dim,seqs,expected", [
+    (32, 8, 128, [(4064, 32)], [1]),                               # 90 / 25
+    (32, 8, 128, [(3584, 512)], [1]),                              # 105 / 65
+    (32, 8, 128, [(3584, 512)] * 4, [0] * 4),                      # 144 / 243
+    (16, 4, 128, [(0, 808), (1351, 165)], [0, 0]),                 # 49 / 60
+    (14, 2, 64, [(790, 566), (714, 197), (0, 184), (1712, 52)], [0] * 4),  # 53 / 60
+    (8, 8, 64, [(0, 1212)] + [(3, 600)] * 22, [0] * 23),           # 48 / 77 (such a call)
+    (32, 8, 128, [(16352, 32), (0, 64)], [1, 0]),                  # 323 / 50
+    (16, 2, 256, [(142, 118), (100, 135)], [0, 0]),                # 105 / 127
+    (16, 2, 256, [(1000, 32)], [1]),                               # 206 / 28
+    (16, 2, 256, [(1000, 1024)] * 4, [1] * 4),                     # 668 / 292
+    (8, 2, 256, [(640, 96), (300, 40), (200, 48)], [1, 1, 0]),
+    (16, 2, 256, [(100, 40), (0, 200)], [0, 0]),                   # no candidate
+])
+def test_sequences_are_split_where_the_whole_call_gains(plans, heads, kv, dim, seqs, expected):
+    assert plans.chosen(heads, kv, dim, seqs) == expected

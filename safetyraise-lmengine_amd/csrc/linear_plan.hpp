@@ -138,14 +138,16 @@ inline LinChoice linear_choice(uint32_t M, uint32_t N, uint32_t K, uint32_t dtyp
     // nearly two 128 x 128 output tiles per CU or more: 2048 rows of 12288 x
     // 4096 (1536 tiles) 476 against 540 with kRows, of 4096 x 4096 (512) 185 / 210;
     // with fewer kRows, which can split K: 1500 rows of it (384) 173 / 160, 1024
-    // (256) 160 / 106; but one tile per CU where a K block or two is all there is
-    // (1528 rows of 2752 x 64, 264 tiles: 11.7 / 13.4).  Not with fewer outputs than
-    // 2048 (k/v projections): there kRows is the faster one (7168 rows of 1024 x
-    // 4096 246 / 210, of 1024 x 12288 727 / 628), and kWide's one chain of all three
-    // parts of x rounds more (relative error at K = 4096 7.0e-7 / 1.4e-7).
+    // (256) 160 / 106.  From 1.5 tiles per CU to there kWide would be up to a fifth
+    // faster (1664 rows of 4096 x 1024, 416 tiles, 51 / 61; of 4096 x 192 18.4 / 22.8),
+    // and with one stage of K from one tile on (1528 rows of 2752 x 64 11.7 / 13.4),
+    // but its one chain of all three parts of x rounds more (relative error at K =
+    // 4096 7.0e-7 / 1.4e-7), so it stays with the calls that it had.  Not with fewer
+    // outputs than 2048 (k/v projections): there kRows is the faster one too (7168
+    // rows of 1024 x 4096 246 / 210, of 1024 x 12288 727 / 628).
     const uint64_t tiles = (uint64_t)((M + kWideBM - 1) / kWideBM) * ((N + kWideBN - 1) / kWideBN);
     if (M > 64 && N >= kWideMinOutputs && K % kGemmK == 0 && K > 0 &&
-        4 * tiles >= (K <= kGemmK ? 4 : 7) * cus && split_x_bytes(M, K) <= scratch) {
+        4 * tiles >= 7 * cus && split_x_bytes(M, K) <= scratch) {
         return {LinRoute::kWide, {}, 1, split_x_bytes(M, K)};
     }
     const bool pair = M <= 2 * kLinTile;

@@ -666,7 +666,7 @@ def bench_gdn_decode(args, torch, pkg, steps, warmup, layers=64):
             "bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": traffic_from_profiles("gdn_decode_qwen35"),
-            "kernel": "gdn_head_kernel<512, ConvK<4>>",
+            "kernel": "gdn_head_kernel<ConvK<4>, 1>",
             "launch_us_mean": round(float(call_us), 2),
             "bytes_per_launch": int(per_layer),
         },
@@ -944,7 +944,7 @@ def bench_linear(args, torch, pkg, steps, warmup, rows=16):
             "bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": traffic_from_profiles("linear_qwen3_8b"),
-            "kernel": "linear_kernel<3, true, 3, 8, 2, true> (the 12288 x 4096 gate/up calls: bf16 "
+            "kernel": "linear_kernel<3, true, 3, 8, 2, true, 1> (the 12288 x 4096 gate/up calls: bf16 "
                       "weight, 3 output tiles per wave, 8 waves)",
             "launch_us_mean": round(float(big_us), 2),
             "bytes_per_launch": int(per_call[4]),
@@ -1227,7 +1227,7 @@ def bench_verify(args, torch, pkg, steps, warmup, rows=5, shape="qwen3-32b"):
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": (traffic_from_profiles("attn_verify_qwen3_32b")
                         if shape == "qwen3-32b" else None),
-            "kernel": f"attn_verify_kernel<{dim}>",
+            "kernel": f"attn_verify_kernel<{dim}, false>",
             "launch_us_mean": round(float(call_us), 2),
             "bytes_per_launch": int(nbytes),
         },

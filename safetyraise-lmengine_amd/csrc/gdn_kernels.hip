@@ -78,6 +78,9 @@ __device__ __forceinline__ float softplus_ref(float x) {
 // is in flight at once) and the per-row conv and history shift are register
 // operations.
 struct ConvChan {
+    // least waves per SIMD of the head kernel where two workgroups might share a CU
+    // (a workgroup's eight are two; held to four, these taps spill)
+    static constexpr int kSharedWaves = 2;
     float hist[kMaxK - 1];
     float w[kMaxK];
     // Every load is unconditional, at an index clamped into the row (the
@@ -314,9 +317,16 @@ struct HeadArgs {
 constexpr int kHeadCh = 2 * kDk + kHeadDv;  // q, k and v channels of one head
 constexpr int kHeadThreads = 512;
 constexpr int kHeadRows = 8;  // rows per batch of a multi-row call (one per wave)
+// rows per batch where a launch has more workgroups than CUs.  Eight take 141
+// registers, which leaves room for one workgroup per CU; four are held to 128, and
+// two share it.  12 sequences of 2, 5 and 9 rows at 16 / 32 heads: 15.9, 23.7 and 37.3
+// us with eight, 12.7, 19.8 and 28.6 with four.
+constexpr int kHeadRowsShared = 4;
 static_assert(kHeadThreads >= kHeadCh && kHeadThreads / 64 >= kHeadRows, "thread layout");
 
-// NR: rows per batch, 1 for calls with one row per sequence, else kHeadRows.
+// NR: rows per batch, 1 for calls with one row per sequence, else kHeadRows; 2
+// where no sequence has more (8 sequences at 16 / 32 heads 10.2 to 9.9 us, 12 at 16 /
+// 16 11.7 to 10.7), and kHeadRowsShared.
 // Only the delta rule is serial over the rows: the conv (registers of a
 // channel's thread), the q/k norms and the output norms of a batch's rows run
 // first and last, a row per wave, so a batch takes four barriers where each
@@ -325,10 +335,10 @@ static_assert(kHeadThreads >= kHeadCh && kHeadThreads / 64 >= kHeadRows, "thread
 // that both forms (and gdn_rollback_kernel) round alike.  4 sequences x 5 rows at 32 heads:
 // 16.8 to 12.3 us a call.
 template <class Conv, int NR>
-__global__ void __launch_bounds__(kHeadThreads) gdn_head_kernel(const GdnParams p,
-                                                                const float *norm, const void *z,
-                                                                float *out, uint32_t *err_word,
-                                                                float eps) {
+__global__ void
+__launch_bounds__(kHeadThreads, NR == kHeadRowsShared ? Conv::kSharedWaves : 2)
+gdn_head_kernel(const GdnParams p, const float *norm, const void *z, float *out,
+                uint32_t *err_word, float eps) {
     constexpr int NTH = kHeadThreads;
     __shared__ __align__(16) float conv_s[NR][kHeadCh];
     __shared__ float out_s[NR][kHeadDv];
@@ -775,6 +785,7 @@ __device__ __forceinline__ void mma(f32x4 &acc, const Ops<NK> &a, const Ops<NK> 
 // arithmetic and history layout as ConvChan.
 template <int K>
 struct ConvK {
+    static constexpr int kSharedWaves = 4;
     static constexpr int kK = K;
     static constexpr int H = K > 1 ? K - 1 : 1;
     float hist[H];
@@ -1471,19 +1482,22 @@ hipError_t launch_chunk(hipStream_t stream, const GdnParams &p, uint32_t max_chu
     return hipGetLastError();
 }
 
+template <class Conv, int NR>
+void launch_head_rows(hipStream_t stream, const GdnParams &p, const GdnLaunch &g) {
+    SR_LAUNCH("gdn_head_kernel", (gdn_head_kernel<Conv, NR>), dim3(p.value_heads, p.nseq),
+              dim3(kHeadThreads), 0, stream, p, g.norm, g.z, g.out, g.err_word, g.eps);
+}
+
 // One workgroup per (value head, sequence); a launch with a sequence of more
-// than one row takes the batched form.
+// than one row takes a batched form.
 template <class Conv>
 hipError_t launch_head(hipStream_t stream, const GdnParams &p, const GdnLaunch &g,
                        uint32_t max_rows) {
-    const dim3 grid(p.value_heads, p.nseq);
-    if (max_rows == 1) {
-        SR_LAUNCH("gdn_head_kernel", (gdn_head_kernel<Conv, 1>), grid, dim3(kHeadThreads), 0, stream,
-                  p, g.norm, g.z, g.out, g.err_word, g.eps);
-    } else {
-        SR_LAUNCH("gdn_head_kernel", (gdn_head_kernel<Conv, kHeadRows>), grid, dim3(kHeadThreads), 0,
-                  stream, p, g.norm, g.z, g.out, g.err_word, g.eps);
-    }
+    const uint64_t workgroups = (uint64_t)p.value_heads * p.nseq;
+    if (max_rows == 1) launch_head_rows<Conv, 1>(stream, p, g);
+    else if (workgroups > (uint64_t)g.num_cus) launch_head_rows<Conv, kHeadRowsShared>(stream, p, g);
+    else if (max_rows == 2) launch_head_rows<Conv, 2>(stream, p, g);
+    else launch_head_rows<Conv, kHeadRows>(stream, p, g);
     return hipGetLastError();
 }
 

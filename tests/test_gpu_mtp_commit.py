@@ -84,6 +84,31 @@ def test_gdn_rollback_to_every_row_of_a_verify_call(pkg, backend, rng):
     pool.destroy()
 
 
+# rows per batch of the head kernel: 8, 4 (more workgroups than CUs), 2 (no
+# sequence has more); conv widths with known and run-time taps
+@pytest.mark.parametrize("conv", [4, 3])
+@pytest.mark.parametrize("rows", [[5, 1, 8, 3], [5, 1, 8, 2, 3, 4, 7, 6, 1], [2, 1, 2, 2],
+                                  [2, 2, 1, 2, 2, 2, 2, 1, 2]])
+def test_verify_rows_equal_single_rows_bit_for_bit(pkg, backend, rng, conv, rows):
+    # 32 value heads: nine sequences are 288 workgroups
+    L = Layer(rng, 8, 32, 128, 128, conv)
+    n = len(rows)
+    pool = pkg.GdnState(backend, 8, 32, 128, 128, conv, 2 * n, keep_rows=8)
+    seqs = [pool.open() for _ in rows]
+    plugin_rows(pkg, backend, pool, L, seqs, [1] * n, L.inputs(rng, n))
+    forks = [pool.fork(s) for s in seqs]
+    x = L.inputs(rng, sum(rows))
+    out = gdn_rows_keep(pkg, backend, pool, L, seqs, rows, x)
+    ends = np.cumsum(rows)
+    for s, f, r, end in zip(seqs, forks, rows, ends):
+        single = np.concatenate([plugin_rows(pkg, backend, pool, L, [f], [1], rows_of(x, i, i + 1))
+                                 for i in range(end - r, end)])
+        assert np.array_equal(out[end - r:end], single)
+        for got, exp in zip(pool.read(s), pool.read(f)):
+            assert np.array_equal(got, exp)
+    pool.destroy()
+
+
 def test_gdn_rollback_batch_and_errors(pkg, backend, rng):
     L = Layer(rng, 2, 4, 128, 128, 4)
     pool = pkg.GdnState(backend, 2, 4, 128, 128, 4, 6, keep_rows=6)

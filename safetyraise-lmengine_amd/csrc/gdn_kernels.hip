@@ -1345,6 +1345,11 @@ __global__ void __launch_bounds__(kScanThreads) gdn_chunk_scan_kernel(const GdnP
     };
     f32x4 xs[kSeg];
     fetch(rec_of(0), xs);
+    // e^{g_C} of the first two chunks, all that a call of 64 rows has: read where it
+    // is used, its latency follows a barrier (two prompts of 2048 rows by 64 at 16 / 32
+    // heads 775 to 769 us, by 512 rows at 16 / 16 267 to 260).  Requesting every chunk's
+    // with its record cost calls of many chunks 5 to 13 %.
+    const float ec0 = rec_of(0)[kRecEc], ec1 = rec_of(nchunks > 1 ? 1 : 0)[kRecEc];
     float *state = p.state + (((size_t)m.state_in * p.value_heads + h) * kHeadDv + vq * kVs) * kDk;
     {
         const int v = tid >> 4, d0 = (tid & 15) * 4;
@@ -1399,7 +1404,7 @@ __global__ void __launch_bounds__(kScanThreads) gdn_chunk_scan_kernel(const GdnP
             }
         } else {
             // S_C = e^{g_C} S0 + Delta^T Ks^T over state rows 16 tr.., dims 64 tc..
-            const float eC = p.chunk_rec[((size_t)(m.chunk0 + c) * p.value_heads + h) * kRecFloats + kRecEc];
+            const float eC = c == 0 ? ec0 : c == 1 ? ec1 : rec_of(c)[kRecEc];
             Ops<2> da;
             load_ops(da, &L.dt[16 * tr][0], kPc, lane);
             Ops<2> kb4[4];
